@@ -350,7 +350,8 @@ def passes_terms(shape):
 
 def passes_name(shape):
     return {1: ", one term per pass", 3: ", three terms per pass", 4: ", four terms per pass",
-            5: ", five terms per pass"}.get(passes_terms(shape), ", several terms per pass")
+            5: ", five terms per pass",
+            32: " merged into blocks, resident passes (half or all of a step each)"}.get(passes_terms(shape), ", several terms per pass")
 
 
 def shape_json(shape):
@@ -377,7 +378,14 @@ def term_kernel_bytes(n, nnz, K, s, real=False):
 
 def kernel_label(kind, prec, K, real, threads):
     """Template name of a timed launch kind (k_block_pass<R, V, RV, mode,
-    threads, terms>)."""
+    threads, terms>; for resident passes k_ring<R, V, RV>, which pass of the
+    step it is and its terms)."""
+    if kind.startswith("ring"):
+        mode, terms = kind[4:].split("x")
+        R = "float" if prec == "fp32" else "double"
+        V = 2 if prec == "fp32" and K not in (1, 3) else 1
+        which = ("middle", "first", "last", "whole step")[int(mode)]
+        return f"k_ring<{R}, {V}, {str(bool(real)).lower()}> {which}, {terms} terms"
     if kind.startswith("pass"):
         mode, terms = kind[4:].split("x")
         slots = 1
@@ -469,6 +477,16 @@ def pass_bytes_fn(sched, n, nnz, K, s, real):
             return term_kernel_bytes(n, nnz, K, s, real)
         if kind.startswith("pass0x"):
             return full
+        if kind.startswith("ring") and sched is not None:
+            # rows of v_{m-1} of the blocks and their rings, of v_{m-2} on the
+            # rows computed (not in a first pass), and of the owned rows:
+            # output read (not in a first pass) and written, psi0 (last), two
+            # terms written (not in a last)
+            first, last = int(kind[4]) % 2, int(kind[4]) // 2
+            own = (0 if first else 1) + 1 + (1 if last else 0) + (0 if last else 2)
+            return sched["tables"] + sched["row_bytes"] * (
+                sched["gathered_rows"] + (0 if first else sched["streamed_rows"]) +
+                own * sched["owned_rows"])
         return None
     return f
 

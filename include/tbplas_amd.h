@@ -64,6 +64,14 @@ int tbg_set_real_layout(tbg_handle *h, int enable);
  * Default (3, 0).  No reference counterpart. */
 int tbg_set_blocking(tbg_handle *h, int enable, int max_rows);
 
+/* Resident passes (default off; tbg_set_blocking turns them off): runs on
+ * Hamiltonians with spatial tiles form up to a whole time step of Chebyshev
+ * terms per launch on row blocks merged from the tiles, whose states stay in
+ * LDS and registers meanwhile (same states).  Where no block fits the LDS
+ * the run takes the passes tbg_set_blocking chose.  No reference
+ * counterpart. */
+int tbg_set_resident(tbg_handle *h, int enable);
+
 /* ---- CSR assembly --------------------------------------------------------
  * Replaces the Cython build_ham_dxy_fast (tbplas/cython/sample.pyx:148-257,
  * called from tbplas/builder/sample.py:452-458).  Insertion order: within a

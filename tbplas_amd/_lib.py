@@ -40,6 +40,7 @@ _SIGS = {
     "tbg_ham_create_ordered": [_P, _I64, _P, _P, _P, _P, _P, _D, _I, _P, _P, _I64,
                                ctypes.POINTER(_P)],
     "tbg_set_blocking": [_P, _I, _I],
+    "tbg_set_resident": [_P, _I],
     "tbg_ham_blocking_info": [_P, _P, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_D)],
     "tbg_ham_blocking_launch": [_P, _P, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)],
     "tbg_ham_blocking_bytes": [_P, _P, _I, _I, _P],
@@ -185,6 +186,12 @@ class Handle:
             raise ValueError("terms per pass must be 3, 4 or 5")
         check(lib().tbg_set_blocking(self._h, int(terms) if enable else 0, int(max_rows)))
 
+    def set_resident(self, enable=True):
+        """Up to a whole time step of Chebyshev terms per launch on row
+        blocks that stay in LDS and registers, for Hamiltonians with spatial
+        tiles (same states); set_blocking turns it off again."""
+        check(lib().tbg_set_resident(self._h, 1 if enable else 0))
+
     def set_kernel_timing(self, enable=True):
         """Bracket every propagation and correlation launch by HIP events
         (graph replay is skipped while on); read with kernel_times()."""
@@ -196,7 +203,9 @@ class Handle:
         kernel), "ac_corr", "dc_qe", "dc_dot", "gram" (the Hall moments'
         Gram block), and "pass<mode>x<terms>" for
         the tile pass (mode 0 continue, 1 first terms from v_0, 2 last
-        terms, 3 with the norm, 4 with dot and norm)."""
+        terms, 3 with the norm, 4 with dot and norm), "ring<mode>x<terms>" for
+        the resident pass (mode 0 continue, 1 first of a step, 2 last, 3 the
+        whole step)."""
         cap = 64
         kinds = np.zeros(cap, dtype=np.int32)
         ms = np.zeros(cap, dtype=np.float64)
@@ -208,7 +217,8 @@ class Handle:
         out = {}
         for i in range(min(nk.value, cap)):
             k = int(kinds[i])
-            name = names.get(k) or f"pass{(k - 100) // 10}x{(k - 100) % 10}"
+            name = names.get(k) or (f"ring{(k - 300) // 100}x{k % 100}" if k >= 300 else
+                                    f"pass{(k - 100) // 10}x{(k - 100) % 10}")
             out[name] = (float(ms[i]), int(cnt[i]))
         return out
 

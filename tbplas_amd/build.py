@@ -18,7 +18,9 @@ LIB = os.path.join(OUT_DIR, "libtbplas_amd.so")
 SOURCES = ["tbg_pass_f32_t5_real.hip", "tbg_pass_f32_t5_cplx.hip", "tbg_pass_f64_t5_real.hip",
            "tbg_pass_f64_t5_cplx.hip", "tbg_prop.hip", "tbg_pass_f32_t4_real.hip",
            "tbg_pass_f32_t4_cplx.hip", "tbg_pass_f64_t4_real.hip", "tbg_pass_f64_t4_cplx.hip",
-           "tbg_pass_t2.hip",
+           "tbg_pass_t2.hip", "tbg_ring_f32_v2_real.hip", "tbg_ring_f32_v2_cplx.hip",
+           "tbg_ring_f32_v1_real.hip", "tbg_ring_f32_v1_cplx.hip", "tbg_ring_f64_v1_real.hip",
+           "tbg_ring_f64_v1_cplx.hip", "tbg_ring.hip",
            "tbg_pass_f32_t3_real.hip", "tbg_pass_f32_t3_cplx.hip", "tbg_pass_f64_t3_real.hip",
            "tbg_pass_f64_t3_cplx.hip", "tbg_super.hip", "tbg_api.hip", "tbg_cond.hip",
            "tbg_block.hip", "tbg_mlp.hip", "tbg_csr.hip", "tbg_hall.hip", "tbg_static.hip"]

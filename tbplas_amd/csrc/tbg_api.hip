@@ -65,6 +65,31 @@ struct tbg_run {
 
 namespace tbg {
 
+// A batch's concatenation and the tiles of its instances in it.
+template <typename R>
+static BlockSrc batch_src(int ni, const tbg_ham* const* hams, const Concat& cat,
+                          const std::vector<int64_t>& inst_slices,
+                          std::vector<std::vector<int64_t>>& segs) {
+    segs.assign((size_t)ni, {});
+    int64_t padded = 0;
+    for (int i = 0; i < ni; ++i) {
+        const int64_t off = inst_slices[i] * 64;
+        for (int64_t t : hams[i]->tiles) segs[i].push_back(off + t);
+        padded += hams[i]->padded;
+    }
+    BlockSrc src;
+    const MatView mv = cat.view();
+    src.cols = mv.cols;
+    src.vals = mv.vals;
+    src.sw = mv.sw;
+    src.soff = mv.soff;
+    src.nslices = cat.nslices;
+    src.padded = padded;
+    src.nrows = cat.nslices * 64;
+    src.vsz = cat.real_vals ? sizeof(R) : sizeof(typename CplxT<R>::T);
+    return src;
+}
+
 // Three-term tables over a batch's block-diagonal concatenation when every
 // instance has spatial tiles: instance i's tiles shifted to its first row,
 // blocks never spanning two instances (so the per-tile correlation sums
@@ -83,26 +108,35 @@ static std::shared_ptr<Blocking> batch_blocking(tbg_handle* h, int ni, const tbg
     for (int i = 0; i < ni; ++i) key += "|" + std::to_string(hams[i]->uid);
     for (const auto& kv : h->batch_blk)
         if (kv.first == key) return kv.second;
-    std::vector<std::vector<int64_t>> segs((size_t)ni);
-    int64_t padded = 0;
-    for (int i = 0; i < ni; ++i) {
-        const int64_t off = inst_slices[i] * 64;
-        for (int64_t t : hams[i]->tiles) segs[i].push_back(off + t);
-        padded += hams[i]->padded;
-    }
-    BlockSrc src;
-    const MatView mv = cat.view();
-    src.cols = mv.cols;
-    src.vals = mv.vals;
-    src.sw = mv.sw;
-    src.soff = mv.soff;
-    src.nslices = cat.nslices;
-    src.padded = padded;
-    src.nrows = cat.nslices * 64;
-    src.vsz = cat.real_vals ? sizeof(R) : sizeof(typename CplxT<R>::T);
+    std::vector<std::vector<int64_t>> segs;
+    const BlockSrc src = batch_src<R>(ni, hams, cat, inst_slices, segs);
     auto B = build_blocking(h, src, segs, row_bytes, h->blocking - 1);
     h->batch_blk.emplace_back(key, B);
     if (h->batch_blk.size() > 2) h->batch_blk.erase(h->batch_blk.begin());
+    return B;
+}
+
+// The same for resident passes.
+template <typename R>
+static std::shared_ptr<Ring> batch_ring(tbg_handle* h, int ni, const tbg_ham* const* hams,
+                                        const Concat& cat,
+                                        const std::vector<int64_t>& inst_slices, int K,
+                                        int terms) {
+    if (!h->resident || ni < 2) return nullptr;
+    for (int i = 0; i < ni; ++i)
+        if (hams[i]->tiles.size() < 2) return nullptr;
+    if (terms > kRingMax) terms = 20;
+    const int Kp = slots_for(K), V = ring_vectors<R>(Kp);
+    std::string key = std::to_string(V) + "|" + std::to_string(Kp / V) + "|" +
+                      std::to_string(terms);
+    for (int i = 0; i < ni; ++i) key += "|" + std::to_string(hams[i]->uid);
+    for (const auto& kv : h->batch_ring)
+        if (kv.first == key) return kv.second;
+    std::vector<std::vector<int64_t>> segs;
+    const BlockSrc src = batch_src<R>(ni, hams, cat, inst_slices, segs);
+    auto B = build_ring(h, src, segs, (int)sizeof(R), V, Kp / V, terms, cat.real_vals != 0);
+    h->batch_ring.emplace_back(key, B);
+    if (h->batch_ring.size() > 4) h->batch_ring.erase(h->batch_ring.begin());
     return B;
 }
 
@@ -132,17 +166,19 @@ struct DosRun : tbg_run {
             mv = cat.view();
         }
         std::shared_ptr<Blocking> pre;
-        if (ni > 1) pre = batch_blocking<R>(h, ni, hams, cat, inst_slices, K);
+        std::shared_ptr<Ring> ring;
+        if (ni > 1) ring = batch_ring<R>(h, ni, hams, cat, inst_slices, K, nb - 1);
+        if (ni > 1 && !ring) pre = batch_blocking<R>(h, ni, hams, cat, inst_slices, K);
         e.init(h, mv, inst_slices, K, chunk_target(h, mv.nslices), ni == 1 ? hams[0] : nullptr,
-               pre);
+               pre, nb - 1, 0, ring);
         const int Kp = e.Kp;
         nv = 3 * Kp;
         psi.alloc(e.vbytes);
         launch_fill_zero(psi.p, e.vbytes, h->stream);
         for (int i = 0; i < ni; ++i) {
             char* base = reinterpret_cast<char*>(psi.p) +
-                         (size_t)inst_slices[i] * 64 * Kp * sizeof(typename CplxT<R>::T);
-            launch_pack<R>(psi0[i], K, hams[i]->n, base, Kp, 0, hams[i]->perm_ptr(), h->stream);
+                         (size_t)inst_slices[i] * 64 * e.lay.unit() * sizeof(typename CplxT<R>::T);
+            launch_pack<R>(psi0[i], K, hams[i]->n, base, e.lay, 0, hams[i]->perm_ptr(), h->stream);
         }
         TBG_HIP(hipMemcpyAsync(e.X.p, psi.p, e.vbytes, hipMemcpyDeviceToDevice, h->stream));
         stride = (int64_t)(T + 1) * nv;
@@ -151,7 +187,7 @@ struct DosRun : tbg_run {
         counter.alloc(sizeof(int));
         TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), h->stream));
         // t = 0: <psi0|psi0> (tbpm.f90:58-62)
-        launch_dotnorm<R>(e.plan, psi.p, psi.p, Kp, Kp, e.part.template as<double>(), h->stream);
+        launch_dotnorm<R>(e.plan, psi.p, psi.p, e.lay, Kp, e.part.template as<double>(), h->stream);
         reduce(e.plan.inst_chunk_dev.template as<int>());
         sp = time_poly(bes, nb);
         TBG_HIP(hipStreamSynchronize(h->stream));
@@ -171,8 +207,11 @@ struct DosRun : tbg_run {
     }
 
     void sched(int64_t* parts, int* row_bytes) const override {
-        for (int i = 0; i < 4; ++i) parts[i] = e.blk ? e.blk->sched[i] : 0;
-        *row_bytes = e.blk ? e.blk->row_bytes : 0;
+        for (int i = 0; i < 4; ++i)
+            parts[i] = e.ring ? e.ring->sched[i] * (i == 0 ? e.Kp / e.ring_v : 1)
+                              : e.blk ? e.blk->sched[i] : 0;
+        *row_bytes = e.ring ? e.Kp * (int)sizeof(typename CplxT<R>::T)
+                            : e.blk ? e.blk->row_bytes : 0;
     }
 
     void end(int chk_step, double chk_thr, double* const* corr, int* fail_inst,
@@ -241,10 +280,11 @@ template <typename R>
 static void step_impl(tbg_handle* h, const tbg_ham* H, const StepPoly& sp, double* psi, int K,
                       uint64_t bwd) {
     Engine<R> e;
-    e.init(h, view_of(H), {0, H->nslices}, K, chunk_target(h, H->nslices), H);
-    launch_pack<R>(psi, K, H->n, e.X.p, e.Kp, 0, H->perm_ptr(), h->stream);
+    e.init(h, view_of(H), {0, H->nslices}, K, chunk_target(h, H->nslices), H, nullptr, sp.N - 1,
+           sp.N - 1);
+    launch_pack<R>(psi, K, H->n, e.X.p, e.lay, 0, H->perm_ptr(), h->stream);
     e.step(sp, bwd, 0, 0, nullptr, nullptr);
-    launch_unpack<R>(e.X.p, e.Kp, 0, H->n, psi, K, H->perm_ptr(), h->stream);
+    launch_unpack<R>(e.X.p, e.lay, 0, H->n, psi, K, H->perm_ptr(), h->stream);
     TBG_HIP(hipStreamSynchronize(h->stream));
 }
 
@@ -259,13 +299,13 @@ static void psi_t_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int n
                        double chk_thr, double* psi_t, int* fail_step) {
     const hipStream_t st = h->stream;
     Engine<R> e;
-    e.init(h, view_of(H), {0, H->nslices}, 1, chunk_target(h, H->nslices), H);
+    e.init(h, view_of(H), {0, H->nslices}, 1, chunk_target(h, H->nslices), H, nullptr, nb - 1);
     const int Kp = e.Kp, nv = 3 * Kp;
     const int64_t n = H->n;
-    launch_pack<R>(psi0, 1, n, e.X.p, Kp, 0, H->perm_ptr(), st);
+    launch_pack<R>(psi0, 1, n, e.X.p, e.lay, 0, H->perm_ptr(), st);
     DevBuf nbuf((size_t)nv * sizeof(double));
     auto norm_of_state = [&]() {
-        launch_dotnorm<R>(e.plan, e.X.p, e.X.p, Kp, Kp, e.part.template as<double>(), st);
+        launch_dotnorm<R>(e.plan, e.X.p, e.X.p, e.lay, Kp, e.part.template as<double>(), st);
         launch_reduce(e.part.template as<double>(), nv, e.plan.inst_chunk_dev.template as<int>(),
                       1, nbuf.as<double>(), 0, nullptr, 0, st);
         double v[3];
@@ -276,7 +316,7 @@ static void psi_t_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int n
     const double norm_ref = norm_of_state();
     const StepPoly sp = time_poly(bes, nb);
     auto log_frame = [&](int i) {
-        launch_unpack<R>(e.X.p, Kp, 0, n, psi_t + (size_t)i * n * 2, 1, H->perm_ptr(), st);
+        launch_unpack<R>(e.X.p, e.lay, 0, n, psi_t + (size_t)i * n * 2, 1, H->perm_ptr(), st);
     };
     int ptr = 0;
     int t = 1;   // loop index of the reference: the state holds t-1 steps
@@ -313,6 +353,17 @@ static void check_psi_args(const tbg_ham* H, const double* psi0, int K, int T) {
     TBG_REQUIRE(T >= 1, "number of time steps must be >= 1");
 }
 
+// The resident-pass tables for Kp slots of real_bytes-byte reals: those of
+// the last run, else those of a 20-term step; null when they are off.
+static std::shared_ptr<Ring> ring_of(tbg_handle* h, const tbg_ham* H, int Kp, int real_bytes) {
+    if (!h->resident) return nullptr;
+    const int V = real_bytes == 4 ? ring_vectors<float>(Kp) : ring_vectors<double>(Kp);
+    const std::string want = std::to_string(V) + "|" + std::to_string(Kp / V) + "|";
+    for (auto it = H->rings.rbegin(); it != H->rings.rend(); ++it)
+        if (it->first.compare(0, want.size(), want) == 0) return it->second;
+    return get_ring(h, H, real_bytes, V, Kp / V, 20);
+}
+
 }  // namespace tbg
 
 using namespace tbg;
@@ -337,6 +388,7 @@ int tbg_create(tbg_handle** out, int device) {
         h->num_cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
         h->max_lds = prop.sharedMemPerBlock > 0 ? (int)prop.sharedMemPerBlock : 65536;
         prepare_term3(h->max_lds);
+        prepare_ring(h->max_lds);
         static_scratch_init(device);   // the allocation-free entry point's array
         TBG_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
         *out = h.release();
@@ -383,7 +435,15 @@ int tbg_set_blocking(tbg_handle* h, int enable, int max_rows) {
         TBG_REQUIRE(enable == 0 || enable == 1 || enable == 3 || enable == 4 || enable == 5,
                     "enable must be 0 (off), 1 or 3 (three terms per pass), 4 or 5");
         h->blocking = enable == 0 ? 0 : enable == 1 ? 3 : enable;
+        h->resident = 0;
         h->block_rows = max_rows;
+    });
+}
+
+int tbg_set_resident(tbg_handle* h, int enable) {
+    return guard([&] {
+        check_handle(h);
+        h->resident = enable ? 1 : 0;
     });
 }
 
@@ -688,6 +748,11 @@ int tbg_ham_blocking_info(tbg_handle* h, const tbg_ham* H, int states, int preci
         TBG_REQUIRE(precision == TBG_FP64 || precision == TBG_FP32, "unknown precision");
         const int Kp = slots_for(states);
         const int cb = precision == TBG_FP32 ? (int)sizeof(float2) : (int)sizeof(double2);
+        if (auto r = ring_of(h, H, Kp, cb / 2)) {
+            *nblocks = r->nblocks;
+            *halo = r->halo;
+            return;
+        }
         auto b = get_blocking(h, H, Kp * cb);
         *nblocks = b ? b->nblocks : 0;
         *halo = b ? b->halo : 0.0;
@@ -704,6 +769,11 @@ int tbg_ham_blocking_launch(tbg_handle* h, const tbg_ham* H, int states, int pre
         TBG_REQUIRE(precision == TBG_FP64 || precision == TBG_FP32, "unknown precision");
         const int Kp = slots_for(states);
         const int eb = precision == TBG_FP32 ? 4 : 8;
+        if (auto r = ring_of(h, H, Kp, eb)) {
+            *max_rows = r->rows_max;
+            *threads = kRingLanes;
+            return;
+        }
         auto b = get_blocking(h, H, Kp * 2 * eb);
         *max_rows = b ? b->nA_max : 0;
         *threads = b ? term3_launch_threads(eb, H->real_vals != 0, Kp, b->nA_max) : 0;
@@ -719,6 +789,11 @@ int tbg_ham_blocking_bytes(tbg_handle* h, const tbg_ham* H, int states, int prec
         TBG_REQUIRE(precision == TBG_FP64 || precision == TBG_FP32, "unknown precision");
         const int Kp = slots_for(states);
         const int cb = precision == TBG_FP32 ? (int)sizeof(float2) : (int)sizeof(double2);
+        if (auto r = ring_of(h, H, Kp, cb / 2)) {
+            const int groups = Kp / (cb == 8 ? ring_vectors<float>(Kp) : ring_vectors<double>(Kp));
+            for (int i = 0; i < 4; ++i) parts[i] = r->sched[i] * (i == 0 ? groups : 1);
+            return;
+        }
         auto b = get_blocking(h, H, Kp * cb);
         for (int i = 0; i < 4; ++i) parts[i] = b ? b->sched[i] : 0;
     });

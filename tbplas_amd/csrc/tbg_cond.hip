@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(256)
 k_accorr(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ jx,
          const typename CplxT<R>::T* __restrict__ jy, const int64_t* __restrict__ soff,
          const int* __restrict__ sw, const int64_t* __restrict__ chunk,
-         const typename CplxT<R>::T* __restrict__ X, int Kp, int K, double* __restrict__ part) {
+         const typename CplxT<R>::T* __restrict__ X, Lay lay, int K, double* __restrict__ part) {
     __shared__ double sh[256 * 8];
     const int c = remap_chunk(blockIdx.x, gridDim.x);
     const int64_t r0 = chunk[c] * 64, r1 = chunk[c + 1] * 64;
@@ -133,14 +133,14 @@ k_accorr(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ 
                 const int col = cols[e];
                 const auto a = jx[e];
                 const auto b = jy[e];
-                const auto u = X[(int64_t)col * Kp + s];
-                const auto v = X[(int64_t)col * Kp + K + s];
+                const auto u = X[lay.at(col, s)];
+                const auto v = X[lay.at(col, K + s)];
                 w0r = fma(a.x, u.x, fma(-a.y, u.y, w0r)); w0i = fma(a.x, u.y, fma(a.y, u.x, w0i));
                 w1r = fma(b.x, u.x, fma(-b.y, u.y, w1r)); w1i = fma(b.x, u.y, fma(b.y, u.x, w1i));
                 w2r = fma(a.x, v.x, fma(-a.y, v.y, w2r)); w2i = fma(a.x, v.y, fma(a.y, v.x, w2i));
                 w3r = fma(b.x, v.x, fma(-b.y, v.y, w3r)); w3i = fma(b.x, v.y, fma(b.y, v.x, w3i));
             }
-            const auto p = X[r * Kp + 2 * K + s];
+            const auto p = X[lay.at(r, 2 * K + s)];
             const double pr = p.x, pi = p.y;
             const double wr[4] = {w0r, w1r, w2r, w3r}, wi[4] = {w0i, w1i, w2i, w3i};
             for (int q = 0; q < 4; ++q) {
@@ -177,7 +177,7 @@ __global__ void k_qe_init(const double2* __restrict__ psi0, int64_t n, int K, in
 // quasi-eigenstate update (tbpm.f90:616-638).
 template <typename R>
 __global__ void __launch_bounds__(256)
-k_qe(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, int Kp,
+k_qe(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, Lay lay,
      int K, const typename CplxT<R>::T* __restrict__ psi, double2* __restrict__ qe, int n_en,
      const double2* __restrict__ ptab, const double* __restrict__ wtab,
      const int* __restrict__ counter, double* __restrict__ part) {
@@ -193,9 +193,9 @@ k_qe(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__
     double dr = 0.0, di = 0.0;
     if (grp < ng) {
         for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const auto p = X[r * Kp + s];
-            const auto q = X[r * Kp + K + s];
-            const auto z = psi[r * Kp + s];
+            const auto p = X[lay.at(r, s)];
+            const auto q = X[lay.at(r, K + s)];
+            const auto z = psi[lay.at(r, s)];
             const double pr = p.x, pi = p.y, qr = q.x, qi = q.y;
             dr = fma((double)z.x, pr, fma((double)z.y, pi, dr));
             di = fma((double)z.x, pi, fma(-(double)z.y, pr, di));
@@ -335,7 +335,7 @@ __global__ void k_dc_y(const int* __restrict__ cols, const typename CplxT<R>::T*
 // dc[a][q] = <X2[a*K + s] | Y[a*nq + q]>, q = e*K + s.  Grid (chunks, tiles).
 template <typename R>
 __global__ void __launch_bounds__(256)
-k_dcdot(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, int Kp,
+k_dcdot(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, Lay lay,
         int K, const double2* __restrict__ Y, int64_t nq2, int64_t nq,
         double* __restrict__ part) {
     __shared__ double sh[256 * 2];
@@ -352,7 +352,7 @@ k_dcdot(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restric
     double dr = 0, di = 0;
     if (grp < ng) {
         for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const auto x = X[r * Kp + slot];
+            const auto x = X[lay.at(r, slot)];
             const double2 y = Y[r * nq2 + q2];
             const double xr = x.x, xi = x.y;
             dr = fma(xr, y.x, fma(xi, y.y, dr));
@@ -376,7 +376,7 @@ k_dcdot(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restric
 // (inner_prod(psi2, density_q .pMul. psi1), tbpm.f90:455-478).
 template <typename R>
 __global__ void __launch_bounds__(256)
-k_rhocorr(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, int Kp,
+k_rhocorr(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, Lay lay,
           int K, const double2* __restrict__ rho, double* __restrict__ part) {
     __shared__ double sh[256];
     const int c = remap_chunk(blockIdx.x, gridDim.x);
@@ -386,8 +386,8 @@ k_rhocorr(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restr
     double d = 0.0;
     if (grp < ng) {
         for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const auto a = X[r * Kp + s];
-            const auto b = X[r * Kp + K + s];
+            const auto a = X[lay.at(r, s)];
+            const auto b = X[lay.at(r, K + s)];
             const double2 q = rho[r];
             const double ar = a.x, ai = a.y;
             const double wr = q.x * ar - q.y * ai, wi = q.x * ai + q.y * ar;
@@ -405,18 +405,18 @@ k_rhocorr(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restr
 
 // Slots [0, K) of X times conj(rho) per layout row (density(-q) .pMul. wf0).
 template <typename R>
-__global__ void k_rho_conj_mul(typename CplxT<R>::T* __restrict__ X, int Kp, int K,
+__global__ void k_rho_conj_mul(typename CplxT<R>::T* __restrict__ X, Lay lay, int K,
                                const double2* __restrict__ rho, int64_t n_pad) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_pad * K) return;
     const int64_t r = i / K;
     const int s = (int)(i - r * K);
-    auto v = X[r * Kp + s];
+    auto v = X[lay.at(r, s)];
     const double2 q = rho[r];
     const double vr = v.x, vi = v.y;
     v.x = (R)(q.x * vr + q.y * vi);
     v.y = (R)(q.x * vi - q.y * vr);
-    X[r * Kp + s] = v;
+    X[lay.at(r, s)] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -435,16 +435,17 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
                   int chk_step, double chk_thr, double* corr, int* fail_step) {
     using C = typename CplxT<R>::T;
     Engine<R> e;
-    e.init(h, view_of(H), {0, H->nslices}, 3 * K, chunks_for(h, H->nslices), H);
+    e.init(h, view_of(H), {0, H->nslices}, 3 * K, chunks_for(h, H->nslices), H, nullptr, nb - 1,
+           std::max(nF, nO) - 1);
     const int Kp = e.Kp;
     const hipStream_t st = h->stream;
     DevBuf psi(e.vbytes);
     launch_fill_zero(psi.p, e.vbytes, st);
-    launch_pack<R>(psi0, K, H->n, psi.p, Kp, 0, H->perm_ptr(), st);
+    launch_pack<R>(psi0, K, H->n, psi.p, e.lay, 0, H->perm_ptr(), st);
     // psi1_x = J_x psi0, psi1_y = J_y psi0, psi2 = psi0 (tbpm.f90:279-281)
-    launch_spmv<R>(H, H->jx.p, psi.p, Kp, 0, e.X.p, Kp, 0, K, st);
-    launch_spmv<R>(H, H->jy.p, psi.p, Kp, 0, e.X.p, Kp, K, K, st);
-    launch_pack<R>(psi0, K, H->n, e.X.p, Kp, 2 * K, H->perm_ptr(), st);
+    launch_spmv<R>(H, H->jx.p, psi.p, e.lay, 0, e.X.p, e.lay, 0, K, st);
+    launch_spmv<R>(H, H->jy.p, psi.p, e.lay, 0, e.X.p, e.lay, K, K, st);
+    launch_pack<R>(psi0, K, H->n, e.X.p, e.lay, 2 * K, H->perm_ptr(), st);
     // Fermi operators: class 0 = 1 - F on psi1, class 1 = F on psi2.
     uint64_t cls = 0;
     for (int k = 2 * K; k < 3 * K; ++k) cls |= 1ull << k;
@@ -460,7 +461,7 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     TBG_HIP(hipMemsetAsync(abuf.p, 0, (size_t)T * 8 * K * sizeof(double), st));
     DevBuf counter(sizeof(int));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-    launch_dotnorm<R>(e.plan, e.X.p, e.X.p, Kp, Kp, e.part.template as<double>(), st);
+    launch_dotnorm<R>(e.plan, e.X.p, e.X.p, e.lay, Kp, e.part.template as<double>(), st);
     launch_reduce(e.part.template as<double>(), nvn, e.plan.inst_chunk_dev.template as<int>(), 1,
                   nbuf.as<double>(), 0, counter.as<int>(), 0, st);
     const StepPoly sp = time_poly(bes, nb);
@@ -471,7 +472,7 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
             hipLaunchKernelGGL(k_accorr<R>, dim3(e.plan.nchunks), dim3(256), 0, st,
                                H->cols.as<int>(), H->jx.as<C>(), H->jy.as<C>(),
                                H->slice_off.as<int64_t>(), H->slice_w.as<int>(),
-                               e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), Kp, K,
+                               e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay, K,
                                e.part.template as<double>());
         });
         launch_reduce(e.part.template as<double>(), 8 * K, e.plan.inst_chunk_dev.template as<int>(),
@@ -521,7 +522,8 @@ void dyn_pol_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     using C = typename CplxT<R>::T;
     const hipStream_t st = h->stream;
     Engine<R> e;
-    e.init(h, view_of(H), {0, H->nslices}, 2 * K, chunks_for(h, H->nslices), H);
+    e.init(h, view_of(H), {0, H->nslices}, 2 * K, chunks_for(h, H->nslices), H, nullptr, nb - 1,
+           std::max(nF, nO) - 1);
     const int Kp = e.Kp;
     const int64_t n = H->n, n_pad = e.n_pad;
     uint64_t cls = 0;
@@ -537,7 +539,7 @@ void dyn_pol_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     std::vector<double> out((size_t)K * n_q * T);
     auto corr_now = [&]() {
         hipLaunchKernelGGL(k_rhocorr<R>, dim3(e.plan.nchunks), dim3(256), 0, st,
-                           e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), Kp, K,
+                           e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay, K,
                            rho.as<double2>(), e.part.template as<double>());
         launch_reduce(e.part.template as<double>(), K, e.plan.inst_chunk_dev.template as<int>(),
                       1, cbuf.as<double>(), 0, counter.as<int>(), 0, st);
@@ -561,17 +563,17 @@ void dyn_pol_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
         launch_pack<double>(rho_in.as<double>(), 1, n, rho.p, 1, 0, H->perm_ptr(), st);
         // psi1 = (1 - F) density(-q) psi0 in slots [0, K), psi2 = F psi0 in [K, 2K)
         launch_fill_zero(e.X.p, e.vbytes, st);
-        launch_pack<R>(psi0, K, n, e.X.p, Kp, 0, H->perm_ptr(), st);
-        launch_pack<R>(psi0, K, n, e.X.p, Kp, K, H->perm_ptr(), st);
+        launch_pack<R>(psi0, K, n, e.X.p, e.lay, 0, H->perm_ptr(), st);
+        launch_pack<R>(psi0, K, n, e.X.p, e.lay, K, H->perm_ptr(), st);
         hipLaunchKernelGGL(k_rho_conj_mul<R>, dim3(nblk(n_pad * K)), dim3(256), 0, st,
-                           e.X.template as<C>(), Kp, K, rho.as<double2>(), n_pad);
+                           e.X.template as<C>(), e.lay, K, rho.as<double2>(), n_pad);
         TBG_HIP(hipGetLastError());
         {
             TimingHold hold(h);
             e.step(fp, 0, cls, 0, nullptr, nullptr);
         }
         TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-        launch_dotnorm<R>(e.plan, e.X.p, e.X.p, Kp, Kp, e.part.template as<double>(), st);
+        launch_dotnorm<R>(e.plan, e.X.p, e.X.p, e.lay, Kp, e.part.template as<double>(), st);
         launch_reduce(e.part.template as<double>(), nvn, e.plan.inst_chunk_dev.template as<int>(),
                       1, nbuf.as<double>(), 0, counter.as<int>(), 0, st);
         corr_now();   // t = 1 (tbpm.f90:459-466)
@@ -612,15 +614,15 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     using C = typename CplxT<R>::T;
     const hipStream_t st = h->stream;
     Engine<R> e;
-    e.init(h, view_of(H), {0, H->nslices}, 2 * K, chunks_for(h, H->nslices), H);
+    e.init(h, view_of(H), {0, H->nslices}, 2 * K, chunks_for(h, H->nslices), H, nullptr, nb - 1);
     const int Kp = e.Kp;
     const int64_t n = H->n, n_pad = e.n_pad;
     const int64_t nq = (int64_t)n_en * K;
     DevBuf psi(e.vbytes);
     launch_fill_zero(psi.p, e.vbytes, st);
-    launch_pack<R>(psi0, K, n, psi.p, Kp, 0, H->perm_ptr(), st);
-    launch_pack<R>(psi0, K, n, e.X.p, Kp, 0, H->perm_ptr(), st);
-    launch_pack<R>(psi0, K, n, e.X.p, Kp, K, H->perm_ptr(), st);
+    launch_pack<R>(psi0, K, n, psi.p, e.lay, 0, H->perm_ptr(), st);
+    launch_pack<R>(psi0, K, n, e.X.p, e.lay, 0, H->perm_ptr(), st);
+    launch_pack<R>(psi0, K, n, e.X.p, e.lay, K, H->perm_ptr(), st);
     uint64_t bwd = 0;
     for (int k = K; k < 2 * K; ++k) bwd |= 1ull << k;
     DevBuf qe((size_t)std::max<int64_t>(n_pad * nq, 1) * sizeof(double2));
@@ -647,7 +649,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     DevBuf dbuf((size_t)T * 2 * K * sizeof(double));
     DevBuf counter(sizeof(int));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-    launch_dotnorm<R>(e.plan, e.X.p, e.X.p, Kp, Kp, e.part.template as<double>(), st);
+    launch_dotnorm<R>(e.plan, e.X.p, e.X.p, e.lay, Kp, e.part.template as<double>(), st);
     launch_reduce(e.part.template as<double>(), nvn, e.plan.inst_chunk_dev.template as<int>(), 1,
                   nbuf.as<double>(), 0, counter.as<int>(), 0, st);
     const StepPoly sp = time_poly(bes, nb);
@@ -676,7 +678,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
                       counter.as<int>(), 0, st);
         timed_launch(h, kTimeQe, [&] {
             hipLaunchKernelGGL(k_qe<R>, dim3(e.plan.nchunks), dim3(256), 0, st,
-                               e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), Kp, K,
+                               e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay, K,
                                psi.as<C>(), qe.as<double2>(), n_en, dptab.as<double2>(),
                                dwtab.as<double>(), counter.as<int>(),
                                e.part.template as<double>());
@@ -741,8 +743,8 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     // Phase 2: J_x psi0, J_y psi0 propagated forward (tbpm.f90:655-697).
     e.drop_graph();
     launch_fill_zero(e.X.p, e.vbytes, st);
-    launch_spmv<R>(H, H->jx.p, psi.p, Kp, 0, e.X.p, Kp, 0, K, st);
-    launch_spmv<R>(H, H->jy.p, psi.p, Kp, 0, e.X.p, Kp, K, K, st);
+    launch_spmv<R>(H, H->jx.p, psi.p, e.lay, 0, e.X.p, e.lay, 0, K, st);
+    launch_spmv<R>(H, H->jy.p, psi.p, e.lay, 0, e.X.p, e.lay, K, K, st);
     const int64_t nq2 = 2 * nq;
     DevBuf cbuf((size_t)std::max<int64_t>(T * nq2 * 2, 1) * sizeof(double));
     DevBuf cpart((size_t)std::max<int64_t>((int64_t)e.plan.nchunks * nq2 * 2, 1) * sizeof(double));
@@ -752,7 +754,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
         if (nq2 == 0) return;
         timed_launch(h, kTimeDcDot, [&] {
             hipLaunchKernelGGL(k_dcdot<R>, dim3(e.plan.nchunks, (unsigned)ntiles2), dim3(256), 0,
-                               st, e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), Kp,
+                               st, e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay,
                                K, Y.as<double2>(), nq2, nq, cpart.as<double>());
         });
         launch_reduce(cpart.as<double>(), (int)(nq2 * 2), e.plan.inst_chunk_dev.template as<int>(),

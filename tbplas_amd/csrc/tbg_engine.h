@@ -6,6 +6,7 @@
 
 #include "tbg_block.h"
 #include "tbg_prop.h"
+#include "tbg_ring.h"
 
 namespace tbg {
 
@@ -100,12 +101,20 @@ struct Engine {
     std::shared_ptr<Blocking> blk;
     DevBuf Q, S, tile_range;
     bool epi_tiles = false;
+    // Resident passes (tbg_ring.hip), when the handle asks for them and the
+    // run's matrix has spatial tiles: the states then lie in planes.
+    std::shared_ptr<Ring> ring;
+    Lay lay{1};
+    int ring_v = 1;
+
+    static int ring_passes(int terms, int depth) { return (terms + depth - 1) / depth; }
 
     // H: the run's single Hamiltonian (its spatial tiles enable three terms
     // per pass); pre: tables built elsewhere (a batch's concatenation).
     void init(tbg_handle* hh, const MatView& m, const std::vector<int64_t>& inst_slices,
               int k_needed, int chunk_target, const tbg_ham* H = nullptr,
-              std::shared_ptr<Blocking> pre = nullptr) {
+              std::shared_ptr<Blocking> pre = nullptr, int terms = 0, int max_terms = 0,
+              std::shared_ptr<Ring> ring_pre = nullptr) {
         h = hh;
         M = m;
         Kp = slots_for(k_needed);
@@ -118,35 +127,57 @@ struct Engine {
         make_plan(h, plan, inst_slices, chunk_target);
         n_pad = m.nslices * 64;
         vbytes = (size_t)n_pad * Kp * sizeof(typename CplxT<R>::T);
+        ring_v = ring_vectors<R>(Kp);
+        lay = Lay(Kp);
+        ring = ring_pre;
+        if (!ring && H != nullptr && terms > 0)
+            ring = get_ring(h, H, (int)sizeof(R), ring_v, Kp / ring_v, terms);
         X.alloc(vbytes);
-        P.alloc(vbytes);
         Y.alloc(vbytes);
         launch_fill_zero(X.p, vbytes, h->stream);
-        launch_fill_zero(P.p, vbytes, h->stream);
         launch_fill_zero(Y.p, vbytes, h->stream);
         blk.reset();
+        epi_tiles = false;
+        if (ring) {
+            lay = Lay(Kp, ring_v == 2 ? 1 : 0, n_pad * ring_v);
+            const int passes = ring_passes(std::max(terms, max_terms), ring->depth);
+            for (DevBuf* b : {&P, &Q, &S}) {   // two passes need P and Q, more also S
+                if (passes < (b == &S ? 3 : 2)) continue;
+                b->alloc(vbytes);
+                launch_fill_zero(b->p, vbytes, h->stream);
+            }
+            set_tile_range(ring->seg_block, (int)inst_slices.size());
+            part.alloc((size_t)std::max(plan.nchunks, ring->nblocks) * 3 * Kp * sizeof(double) +
+                       64);
+            return;
+        }
+        P.alloc(vbytes);
+        launch_fill_zero(P.p, vbytes, h->stream);
         if (pre) blk = pre;
         else if (H != nullptr) blk = get_blocking(h, H, Kp * (int)sizeof(typename CplxT<R>::T));
         int nparts = plan.nchunks;
         if (blk) {
-            TBG_REQUIRE(blk->row_bytes == Kp * (int)sizeof(typename CplxT<R>::T) &&
-                            (int)blk->seg_block.size() == (int)inst_slices.size(),
+            TBG_REQUIRE(blk->row_bytes == Kp * (int)sizeof(typename CplxT<R>::T),
                         "internal: blocking tables of another shape");
             Q.alloc(vbytes);
             S.alloc(vbytes);
             launch_fill_zero(Q.p, vbytes, h->stream);
             launch_fill_zero(S.p, vbytes, h->stream);
-            // partial sums of a pair pass: one row per tile; instance i owns
-            // tiles [seg_block[i], seg_block[i+1])
-            tile_range.alloc(blk->seg_block.size() * sizeof(int));
-            TBG_HIP(hipMemcpyAsync(tile_range.p, blk->seg_block.data(),
-                                   blk->seg_block.size() * sizeof(int), hipMemcpyHostToDevice,
-                                   h->stream));
-            TBG_HIP(hipStreamSynchronize(h->stream));
+            set_tile_range(blk->seg_block, (int)inst_slices.size());
             nparts = std::max(nparts, blk->nblocks);
         }
         part.alloc((size_t)nparts * 3 * Kp * sizeof(double) + 64);
-        epi_tiles = false;
+    }
+
+    // partial sums of a pass that ends the step: one row per tile; instance
+    // i owns tiles [seg_block[i], seg_block[i+1])
+    void set_tile_range(const std::vector<int>& seg_block, int bounds) {
+        TBG_REQUIRE((int)seg_block.size() == bounds,
+                    "internal: blocking tables of another shape");
+        tile_range.alloc(seg_block.size() * sizeof(int));
+        TBG_HIP(hipMemcpyAsync(tile_range.p, seg_block.data(), seg_block.size() * sizeof(int),
+                               hipMemcpyHostToDevice, h->stream));
+        TBG_HIP(hipStreamSynchronize(h->stream));
     }
 
     // The partial-row range (per instance) that the last step's F_DOT /
@@ -266,11 +297,89 @@ struct Engine {
         parity ^= 1;
     }
 
+    // The step's N - 1 terms in passes of at most depth terms, as even as
+    // they come; the output receives the terms in the order m = 0, 1, 2, ...
+    // as in the one-term schedule, so the states are bit-identical to it.
+    void step_ring(const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi, const void* psi0,
+                   int* counter) {
+        const int terms = sp.N - 1;
+        const int passes = ring_passes(terms, ring->depth);
+        RingArgs<R> a{};
+        a.acc = Y.p;
+        a.plane = lay.plane;
+        a.depth = ring->depth;
+        a.groups = Kp / ring_v;
+        a.lds_rows = ring->rows_max;
+        // the two recurrences there are: time steps (alpha = -2i, beta = 1)
+        // and Chebyshev polynomials (2, -1), which run as u_m = (-i)^m T_m
+        const bool time = sp.ar == 0.0 && sp.ar1 == 0.0 && sp.ai == -2.0 && sp.ai1 == -1.0 &&
+                          sp.beta == 1.0;
+        TBG_REQUIRE(time || (sp.ar == 2.0 && sp.ar1 == 1.0 && sp.ai == 0.0 && sp.ai1 == 0.0 &&
+                             sp.beta == -1.0),
+                    "internal: unknown recurrence");
+        a.ai[1][0] = R(-2);
+        a.ai[1][1] = R(2);
+        a.bwd_mask = bwd;
+        a.cls_mask = cls;
+        a.nv = 3 * Kp;
+        void* b0 = nullptr;   // v_{m-2}, v_{m-1} and two free buffers
+        void* b1 = X.p;
+        void* b2 = P.p;
+        void* b3 = Q.p;
+        int m = 1;
+        for (int p = 0; p < passes; ++p) {
+            a.first = p == 0;
+            a.T = terms / passes + (p < terms % passes ? 1 : 0);
+            a.ai[0][0] = a.first ? R(-1) : R(-2);
+            a.ai[0][1] = -a.ai[0][0];
+            a.poly = time ? 0 : 1;
+            a.turn = 0;
+            for (int t = 0; t < a.T; ++t) {
+                const int r = time ? 0 : (m + t) % 4;   // T_m = i^m u_m
+                if (r % 2) a.turn |= 1u << t;
+                for (int q = 0; q < 2; ++q)
+                    a.c[t][q] = (R)(r < 2 ? sp.c[q][m + t] : -sp.c[q][m + t]);
+            }
+            for (int q = 0; q < 2; ++q) a.c0[q] = (R)sp.c[q][0];
+            a.counter = a.first ? counter : nullptr;
+            a.p0 = b0;
+            a.p1 = b1;
+            const bool last = p == passes - 1;
+            a.q1 = last ? nullptr : b2;
+            a.q2 = last ? nullptr : b3;
+            if (last && (epi & (F_DOT | F_NORM))) {
+                a.part = part.template as<double>();
+                a.psi0 = (epi & F_DOT) ? psi0 : nullptr;
+            }
+            const int kind = kTimeRing + 100 * ((a.first ? 1 : 0) + (last ? 2 : 0)) + a.T;
+            timed_launch(h, kind, [&] {
+                launch_ring<R>(a, *ring, ring_v, M.real_vals != 0, h->stream);
+            });
+            m += a.T;
+            if (p == 0) {   // v_0 is not needed any more
+                b0 = P.p;
+                b1 = Q.p;
+                b2 = S.p;
+                b3 = X.p;
+            } else {
+                std::swap(b0, b2);
+                std::swap(b1, b3);
+            }
+        }
+        epi_tiles = (epi & (F_DOT | F_NORM)) != 0;
+        std::swap(X, Y);
+        parity ^= 1;
+    }
+
     // One step: X holds the input, the result is left in X (buffers swap).
     void step(const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi, const void* psi0,
               int* counter) {
         const int N = sp.N;
         TBG_REQUIRE(N >= 3, "at least 3 expansion terms are required");
+        if (ring) {
+            step_ring(sp, bwd, cls, epi, psi0, counter);
+            return;
+        }
         if (blk && N >= blk->depth + 3) {
             step_blocked(sp, bwd, cls, epi, psi0, counter);
             return;

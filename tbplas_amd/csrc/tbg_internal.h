@@ -104,6 +104,7 @@ constexpr int kSlice = 64;
 constexpr int kWave = 64;
 
 struct Blocking;
+struct Ring;
 
 }  // namespace tbg
 
@@ -119,6 +120,7 @@ struct tbg_handle {
     int stage = 1;
     int real_layout = 1;      // store real values when H has no imaginary part
     int blocking = 3;         // terms per pass where H has spatial tiles (3 to 5; 0: one)
+    int resident = 0;         // resident passes where H has spatial tiles (over blocking)
     int block_rows = 0;       // cap on rows owned per workgroup (0: from LDS)
     int max_lds = 65536;      // LDS bytes one workgroup may use
     tbg::DevBuf scratch;      // reduction partials and small tables
@@ -126,6 +128,7 @@ struct tbg_handle {
     // three-term tables of recent batches (key: state row bytes, limits and
     // the instances' ids); a null entry records tiles that do not fit
     std::vector<std::pair<std::string, std::shared_ptr<tbg::Blocking>>> batch_blk;
+    std::vector<std::pair<std::string, std::shared_ptr<tbg::Ring>>> batch_ring;   // the last four
     // Per-launch timing (tbg_set_kernel_timing): a pair of events around
     // every propagation and correlation launch, tagged with the launch kind
     // (tbg_kernel_times sums them); events are reused from ev_pool.
@@ -143,9 +146,10 @@ namespace tbg {
 
 // Kinds of timed launches: the one-term kernel, the AC / DC correlation
 // kernels, the Hall moments' Gram block, and the tile pass as kTimePass +
-// 10 * mode + terms.
+// 10 * mode + terms, the resident pass as kTimeRing
+// + 100 * (1 for the first of a step + 2 for the last) + terms.
 enum TimedKind : int { kTimeTerm = 1, kTimeAcCorr = 2, kTimeQe = 3, kTimeDcDot = 4,
-                       kTimeGram = 5, kTimePass = 100 };
+                       kTimeGram = 5, kTimePass = 100, kTimeRing = 300 };
 
 // Runs launch() on h->stream, bracketed by two events when timing is on.
 template <typename F>
@@ -216,5 +220,7 @@ struct tbg_ham {
     mutable int blk_row_bytes = 0;
     mutable int blk_rows_cap = 0;
     mutable int blk_depth = 0;
+    // tables of resident passes (tbg_ring.hip), the last two used
+    mutable std::vector<std::pair<std::string, std::shared_ptr<tbg::Ring>>> rings;
     uint64_t uid = 0;         // unique per Hamiltonian created in the process
 };

@@ -5,6 +5,22 @@
 
 namespace tbg {
 
+// Where state k of row r lies in a state buffer (in complex elements): K
+// states interleaved per row (sh < 0), or, for resident passes, planes of
+// 2^sh states of every row.
+struct Lay {
+    int K;
+    int sh = -1;
+    int64_t plane = 0;
+    Lay(int K_) : K(K_) {}
+    Lay(int K_, int sh_, int64_t plane_) : K(K_), sh(sh_), plane(plane_) {}
+    // complex elements from one row to the next
+    int unit() const { return sh < 0 ? K : 1 << sh; }
+    __host__ __device__ __forceinline__ int64_t at(int64_t r, int k) const {
+        return sh < 0 ? r * K + k : (int64_t)(k >> sh) * plane + (r << sh) + (k & ((1 << sh) - 1));
+    }
+};
+
 // Flags of the fused term kernel (compile-time).
 enum TermFlags : int {
     F_PREV = 1,      // recurrence uses beta * v_{m-2} (row-aligned read)
@@ -90,19 +106,19 @@ template <typename R> void launch_term(int flags, const TermArgs& a, int nchunks
 void launch_reduce(const double* part, int nv, const int* inst_chunk, int ninst,
                    double* out, int64_t inst_stride, const int* counter, int toff,
                    hipStream_t s);
-// pack complex128 (K, n) -> interleaved [n_pad][Kp] complex<R> at slot offset;
+// pack complex128 (K, n) -> complex<R> rows of layout lay at a slot offset;
 // with perm (layout row -> caller row) layout row r takes caller row perm[r].
 template <typename R> void launch_pack(const double* src, int K, int64_t n,
-                                       void* dst, int Kp, int slot0, const int* perm,
+                                       void* dst, Lay lay, int slot0, const int* perm,
                                        hipStream_t s);
-template <typename R> void launch_unpack(const void* src, int Kp, int slot0, int64_t n,
+template <typename R> void launch_unpack(const void* src, Lay lay, int slot0, int64_t n,
                                          double* dst, int K, const int* perm, hipStream_t s);
 // Per-vector dot/norm of packed vectors a (conj) and b -> partials (3 per vector).
 template <typename R> void launch_dotnorm(const Plan& p, const void* a, const void* b,
-                                          int Kp, int K, double* part, hipStream_t s);
+                                          Lay lay, int K, double* part, hipStream_t s);
 // y[slot] = M x[slot] for nk vectors (M = H values or a current operator).
 template <typename R> void launch_spmv(const tbg_ham* H, const void* mvals, const void* x,
-                                       int Kx, int sx, void* y, int Ky, int sy, int nk,
+                                       Lay lx, int sx, void* y, Lay ly, int sy, int nk,
                                        hipStream_t s);
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s);
 

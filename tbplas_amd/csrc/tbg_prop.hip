@@ -193,7 +193,7 @@ k_reduce(const double* part, int nv, const int* inst_chunk, double* out,
 // writes the caller's row perm[r] (r without a permutation).
 template <typename R>
 __global__ void k_pack(const double2* __restrict__ src, int K, int64_t n,
-                       typename CplxT<R>::T* __restrict__ dst, int Kp, int slot0,
+                       typename CplxT<R>::T* __restrict__ dst, Lay lay, int slot0,
                        const int* __restrict__ perm) {
     // consecutive threads take consecutive states of one row: the stores of
     // a row's slots are one contiguous run
@@ -205,17 +205,17 @@ __global__ void k_pack(const double2* __restrict__ src, int K, int64_t n,
     typename CplxT<R>::T o;
     o.x = (R)v.x;
     o.y = (R)v.y;
-    dst[r * Kp + slot0 + k] = o;
+    dst[lay.at(r, slot0 + (int)k)] = o;
 }
 
 template <typename R>
-__global__ void k_unpack(const typename CplxT<R>::T* __restrict__ src, int Kp, int slot0,
+__global__ void k_unpack(const typename CplxT<R>::T* __restrict__ src, Lay lay, int slot0,
                          int64_t n, double2* __restrict__ dst, int K, const int* __restrict__ perm) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)K * n) return;
     const int64_t r = i / K, k = i - r * K;
     const int64_t c = perm ? (int64_t)perm[r] : r;
-    const typename CplxT<R>::T v = src[r * Kp + slot0 + k];
+    const typename CplxT<R>::T v = src[lay.at(r, slot0 + (int)k)];
     dst[k * n + c] = make_double2((double)v.x, (double)v.y);
 }
 
@@ -226,17 +226,19 @@ __global__ void k_unpack(const typename CplxT<R>::T* __restrict__ src, int Kp, i
 template <typename R>
 __global__ void __launch_bounds__(256)
 k_dotnorm(const int64_t* chunk, const typename CplxT<R>::T* a, const typename CplxT<R>::T* b,
-          int Kp, int K, double* part) {
+          Lay lay, int K, double* part) {
     const int c = remap_chunk(blockIdx.x, gridDim.x);
     const int64_t r0 = chunk[c] * 64, r1 = chunk[c + 1] * 64;
     __shared__ double sh[256 * 3];
+    const int Kp = lay.K;
     const int RG = 256 / Kp;
     const int k = threadIdx.x % Kp, rg = threadIdx.x / Kp;
     double dr = 0, di = 0, nn = 0;
     if (rg < RG && k < K) {
         for (int64_t r = r0 + rg; r < r1; r += RG) {
-            const auto x = a[r * Kp + k];
-            const auto y = b[r * Kp + k];
+            const int64_t at = lay.at(r, k);
+            const auto x = a[at];
+            const auto y = b[at];
             const double xr = x.x, xi = x.y, yr = y.x, yi = y.y;
             dr = fma(xr, yr, fma(xi, yi, dr));
             di = fma(xr, yi, fma(-xi, yr, di));
@@ -259,8 +261,8 @@ k_dotnorm(const int64_t* chunk, const typename CplxT<R>::T* a, const typename Cp
 template <typename R>
 __global__ void k_spmv(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ mv,
                        const int64_t* __restrict__ soff, const int* __restrict__ sw,
-                       int64_t n_pad, const typename CplxT<R>::T* __restrict__ x, int Kx, int sx,
-                       typename CplxT<R>::T* __restrict__ y, int Ky, int sy, int nk) {
+                       int64_t n_pad, const typename CplxT<R>::T* __restrict__ x, Lay lx, int sx,
+                       typename CplxT<R>::T* __restrict__ y, Lay ly, int sy, int nk) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_pad * nk) return;
     const int64_t r = i / nk;
@@ -273,7 +275,7 @@ __global__ void k_spmv(const int* __restrict__ cols, const typename CplxT<R>::T*
     for (int j = 0; j < w; ++j) {
         const int col = cols[off + j * 64 + lr];
         const auto h = mv[off + j * 64 + lr];
-        const auto v = x[(int64_t)col * Kx + sx + k];
+        const auto v = x[lx.at(col, sx + k)];
         sr = fma(h.x, v.x, sr);
         sr = fma(-h.y, v.y, sr);
         si = fma(h.x, v.y, si);
@@ -282,7 +284,7 @@ __global__ void k_spmv(const int* __restrict__ cols, const typename CplxT<R>::T*
     typename CplxT<R>::T o;
     o.x = sr;
     o.y = si;
-    y[r * Ky + sy + k] = o;
+    y[ly.at(r, sy + k)] = o;
 }
 
 __global__ void k_fill_zero(uint4* p, int64_t n16) {
@@ -369,58 +371,58 @@ void launch_reduce(const double* part, int nv, const int* inst_chunk, int ninst,
 }
 
 template <typename R>
-void launch_pack(const double* src, int K, int64_t n, void* dst, int Kp, int slot0,
+void launch_pack(const double* src, int K, int64_t n, void* dst, Lay lay, int slot0,
                  const int* perm, hipStream_t s) {
     const int64_t tot = (int64_t)K * n;
     if (tot == 0) return;
     hipLaunchKernelGGL(k_pack<R>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
                        reinterpret_cast<const double2*>(src), K, n,
-                       reinterpret_cast<typename CplxT<R>::T*>(dst), Kp, slot0, perm);
+                       reinterpret_cast<typename CplxT<R>::T*>(dst), lay, slot0, perm);
     TBG_HIP(hipGetLastError());
 }
-template void launch_pack<float>(const double*, int, int64_t, void*, int, int, const int*, hipStream_t);
-template void launch_pack<double>(const double*, int, int64_t, void*, int, int, const int*, hipStream_t);
+template void launch_pack<float>(const double*, int, int64_t, void*, Lay, int, const int*, hipStream_t);
+template void launch_pack<double>(const double*, int, int64_t, void*, Lay, int, const int*, hipStream_t);
 
 template <typename R>
-void launch_unpack(const void* src, int Kp, int slot0, int64_t n, double* dst, int K,
+void launch_unpack(const void* src, Lay lay, int slot0, int64_t n, double* dst, int K,
                    const int* perm, hipStream_t s) {
     const int64_t tot = (int64_t)K * n;
     if (tot == 0) return;
     hipLaunchKernelGGL(k_unpack<R>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const typename CplxT<R>::T*>(src), Kp, slot0, n,
+                       reinterpret_cast<const typename CplxT<R>::T*>(src), lay, slot0, n,
                        reinterpret_cast<double2*>(dst), K, perm);
     TBG_HIP(hipGetLastError());
 }
-template void launch_unpack<float>(const void*, int, int, int64_t, double*, int, const int*, hipStream_t);
-template void launch_unpack<double>(const void*, int, int, int64_t, double*, int, const int*, hipStream_t);
+template void launch_unpack<float>(const void*, Lay, int, int64_t, double*, int, const int*, hipStream_t);
+template void launch_unpack<double>(const void*, Lay, int, int64_t, double*, int, const int*, hipStream_t);
 
 template <typename R>
-void launch_dotnorm(const Plan& p, const void* a, const void* b, int Kp, int K, double* part,
+void launch_dotnorm(const Plan& p, const void* a, const void* b, Lay lay, int K, double* part,
                     hipStream_t s) {
-    if (Kp < 1 || Kp > 256 || K > Kp) throw Error{TBG_EINVAL, "internal: bad slot count"};
+    if (lay.K < 1 || lay.K > 256 || K > lay.K) throw Error{TBG_EINVAL, "internal: bad slot count"};
     hipLaunchKernelGGL(k_dotnorm<R>, dim3(p.nchunks), dim3(256), 0, s, p.chunk.as<int64_t>(),
                        reinterpret_cast<const typename CplxT<R>::T*>(a),
-                       reinterpret_cast<const typename CplxT<R>::T*>(b), Kp, K, part);
+                       reinterpret_cast<const typename CplxT<R>::T*>(b), lay, K, part);
     TBG_HIP(hipGetLastError());
 }
-template void launch_dotnorm<float>(const Plan&, const void*, const void*, int, int, double*, hipStream_t);
-template void launch_dotnorm<double>(const Plan&, const void*, const void*, int, int, double*, hipStream_t);
+template void launch_dotnorm<float>(const Plan&, const void*, const void*, Lay, int, double*, hipStream_t);
+template void launch_dotnorm<double>(const Plan&, const void*, const void*, Lay, int, double*, hipStream_t);
 
 template <typename R>
-void launch_spmv(const tbg_ham* H, const void* mvals, const void* x, int Kx, int sx, void* y,
-                 int Ky, int sy, int nk, hipStream_t s) {
+void launch_spmv(const tbg_ham* H, const void* mvals, const void* x, Lay lx, int sx, void* y,
+                 Lay ly, int sy, int nk, hipStream_t s) {
     const int64_t n_pad = H->nslices * 64;
     const int64_t tot = n_pad * nk;
     if (tot == 0) return;
     hipLaunchKernelGGL(k_spmv<R>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
                        H->cols.as<int>(), reinterpret_cast<const typename CplxT<R>::T*>(mvals),
                        H->slice_off.as<int64_t>(), H->slice_w.as<int>(), n_pad,
-                       reinterpret_cast<const typename CplxT<R>::T*>(x), Kx, sx,
-                       reinterpret_cast<typename CplxT<R>::T*>(y), Ky, sy, nk);
+                       reinterpret_cast<const typename CplxT<R>::T*>(x), lx, sx,
+                       reinterpret_cast<typename CplxT<R>::T*>(y), ly, sy, nk);
     TBG_HIP(hipGetLastError());
 }
-template void launch_spmv<float>(const tbg_ham*, const void*, const void*, int, int, void*, int, int, int, hipStream_t);
-template void launch_spmv<double>(const tbg_ham*, const void*, const void*, int, int, void*, int, int, int, hipStream_t);
+template void launch_spmv<float>(const tbg_ham*, const void*, const void*, Lay, int, void*, Lay, int, int, hipStream_t);
+template void launch_spmv<double>(const tbg_ham*, const void*, const void*, Lay, int, void*, Lay, int, int, hipStream_t);
 
 void launch_fill_zero(void* p, size_t bytes, hipStream_t s) {
     if (bytes == 0) return;

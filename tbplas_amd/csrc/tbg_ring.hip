@@ -1,0 +1,622 @@
+// Resident passes of the Chebyshev recurrence: host tables and launch.
+//
+// A tile pass (tbg_block.hip) keeps two vectors of a tile in LDS, which
+// limits it to five terms on about 900 rows of 64 bytes, and while a tile
+// computes its workgroup's compute unit reads nothing.  A resident pass
+// takes the states of a run in groups of 16 bytes a row (two complex64
+// states or one complex128): one workgroup owns a row block for one group,
+// holds only v_{m-1} of the block and its halo rings in LDS, and v_{m-2},
+// the entries of the matrix and the step output in registers (512 KB a
+// compute unit against 160 KB of LDS).  A block with its rings has up to
+// 4096 rows, two fit a compute unit, and a pass is half or all of a time
+// step of 20 terms: nothing is read or written in between.
+//
+// The blocks are made here, on the host, from the caller's spatial tiles:
+// tiles (or runs of a tile's rows) are merged along the matrix' own
+// couplings into compact blocks sized for the LDS, then each block's rings
+// are found, sorted by layout row (coalesced loads), and its tables written
+// (positions in the block, 16 bits, and values).  Blocks are independent,
+// so the work is spread over the host's cores.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <thread>
+
+#include "tbg_ring.h"
+
+namespace tbg {
+
+namespace {
+
+// f(i, thread) for i < n on up to 16 host threads; the first exception is
+// rethrown here.
+template <typename F>
+void parallel_for(int64_t n, int64_t grain, F&& f) {
+    const int nt = (int)std::max<int64_t>(
+        1, std::min<int64_t>(std::min(16u, std::max(1u, std::thread::hardware_concurrency())),
+                             n / std::max<int64_t>(grain, 1)));
+    std::atomic<int64_t> next{0};
+    std::exception_ptr err;
+    std::mutex mu;
+    const int64_t step = std::max<int64_t>(1, std::min<int64_t>(grain, n / (4 * nt) + 1));
+    auto work = [&](int th) {
+        try {
+            for (;;) {
+                const int64_t a = next.fetch_add(step);
+                if (a >= n) break;
+                for (int64_t i = a; i < std::min(n, a + step); ++i) f(i, th);
+            }
+        } catch (...) {
+            std::lock_guard<std::mutex> g(mu);
+            if (!err) err = std::current_exception();
+            next.store(n);
+        }
+    };
+    std::vector<std::thread> ts;
+    try {
+        for (int t = 1; t < nt; ++t) ts.emplace_back(work, t);
+    } catch (...) {   // no more threads: the ones that started do the work
+    }
+    work(0);
+    for (auto& t : ts) t.join();
+    if (err) std::rethrow_exception(err);
+}
+
+constexpr int kHostThreads = 16;
+
+struct Csr {   // the sliced-ELL matrix on the host
+    std::vector<int> cols, sw;
+    std::vector<int64_t> soff;
+    std::vector<unsigned char> vals;
+    int width(int r) const { return sw[r >> 6]; }
+    int64_t elem(int r, int j) const { return soff[r >> 6] + (int64_t)j * 64 + (r & 63); }
+};
+
+// Per-thread marks over the rows (zeroed pages are only touched where used).
+struct Marks {
+    int *mark = nullptr, *loc = nullptr;
+    int stamp = 0;
+    ~Marks() {
+        std::free(mark);
+        std::free(loc);
+    }
+    void need(int64_t n) {
+        if (mark) return;
+        mark = (int*)std::calloc((size_t)n, sizeof(int));
+        loc = (int*)std::calloc((size_t)n, sizeof(int));
+        if (!mark || !loc) throw std::bad_alloc();
+    }
+};
+
+// rows = owned rows + rings 1 .. depth (each sorted); ends[k]; false when
+// more than cap rows.
+bool grow(const Csr& A, Marks& mk, std::vector<int>& rows, int depth, int64_t cap,
+          std::vector<int>& ends) {
+    const int st = ++mk.stamp;
+    for (size_t q = 0; q < rows.size(); ++q) {
+        mk.mark[rows[q]] = st;
+        mk.loc[rows[q]] = (int)q;
+    }
+    ends.assign(1, (int)rows.size());
+    size_t from = 0;
+    for (int k = 1; k <= depth; ++k) {
+        const size_t to = rows.size();
+        for (size_t q = from; q < to; ++q) {
+            const int r = rows[q], w = A.width(r);
+            for (int j = 0; j < w; ++j) {
+                const int c = A.cols[A.elem(r, j)];
+                if (mk.mark[c] != st) {
+                    mk.mark[c] = st;
+                    rows.push_back(c);
+                }
+            }
+        }
+        std::sort(rows.begin() + to, rows.end());
+        for (size_t q = to; q < rows.size(); ++q) mk.loc[rows[q]] = (int)q;
+        ends.push_back((int)rows.size());
+        if ((int64_t)rows.size() > cap) return false;
+        from = to;
+    }
+    return true;
+}
+
+// A compact piece of a caller's tile, from which blocks are made.
+struct Atom {
+    std::vector<int> rows;
+    int seg = 0;
+};
+
+// Rows r0 .. r1 of a tile in k x k pieces of about equal size: k runs of
+// rows (strips, where the rows follow a lattice), each cut across by the
+// distance from one of its ends (breadth first along the couplings).
+void split_tile(const Csr& A, Marks& mk, int64_t r0, int64_t r1, int k, int seg,
+                std::vector<Atom>& out) {
+    for (int q = 0; q < k; ++q) {
+        const int a = (int)(r0 + (r1 - r0) * q / k), b = (int)(r0 + (r1 - r0) * (q + 1) / k);
+        std::vector<int> order;
+        int from = a;
+        for (int sweep = 0; sweep < 2; ++sweep) {   // the second from the farthest row
+            const int st = ++mk.stamp;
+            order.clear();
+            auto visit = [&](int r) {
+                mk.mark[r] = st;
+                order.push_back(r);
+            };
+            visit(from);
+            for (size_t head = 0, next = a; order.size() < (size_t)(b - a); ++head) {
+                if (head == order.size()) {         // another component
+                    while (mk.mark[next] == st) ++next;
+                    visit((int)next);
+                }
+                const int r = order[head];
+                for (int j = 0, w = A.width(r); j < w; ++j) {
+                    const int c = A.cols[A.elem(r, j)];
+                    if (c >= a && c < b && mk.mark[c] != st) visit(c);
+                }
+            }
+            from = order.back();
+        }
+        for (int p = 0; p < k; ++p) {
+            const size_t n = order.size();
+            Atom at;
+            at.seg = seg;
+            at.rows.assign(order.begin() + n * p / k, order.begin() + n * (p + 1) / k);
+            if (at.rows.empty()) continue;
+            std::sort(at.rows.begin(), at.rows.end());
+            out.push_back(std::move(at));
+        }
+    }
+}
+
+struct Block {
+    std::vector<int> rows, ends;
+    int seg = 0, w = 0;
+};
+
+}  // namespace
+
+std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
+                                 const std::vector<std::vector<int64_t>>& segs, int real_bytes,
+                                 int V, int groups, int terms, bool real_vals) {
+    const int unit_bytes = V * 2 * real_bytes;
+    const int64_t n = src.nrows;
+    const size_t vsz = src.vsz;
+    Csr A;
+    A.cols.resize((size_t)src.padded);
+    A.sw.resize((size_t)src.nslices);
+    A.soff.resize((size_t)src.nslices + 1);
+    A.vals.resize((size_t)src.padded * vsz);
+    auto down = [&](void* dst, const void* from, size_t bytes) {
+        if (bytes) TBG_HIP(hipMemcpyAsync(dst, from, bytes, hipMemcpyDeviceToHost, h->stream));
+    };
+    down(A.cols.data(), src.cols, A.cols.size() * sizeof(int));
+    down(A.vals.data(), src.vals, A.vals.size());
+    down(A.sw.data(), src.sw, A.sw.size() * sizeof(int));
+    down(A.soff.data(), src.soff, A.soff.size() * sizeof(int64_t));
+    TBG_HIP(hipStreamSynchronize(h->stream));
+
+    int64_t covered = 0;
+    int wmax = 0;
+    for (const auto& t : segs) {
+        covered += t.back() - t.front();
+        for (int64_t s = t.front() >> 6; s <= (t.back() - 1) >> 6; ++s)
+            wmax = std::max(wmax, A.sw[s]);
+    }
+    if (covered < 1 || wmax < 1) return nullptr;
+    const int W = wmax <= 3 ? 3 : wmax <= 4 ? 4 : 0;
+    const int nr = ring_rows(real_bytes, V, real_vals, W);
+    const int nro = ring_owned(real_bytes, V, real_vals, W);
+    std::vector<Marks> marks(kHostThreads);
+
+    // growth of a block per ring, from a few tiles: side(k) = side(0) + k c
+    // with side = sqrt(rows)
+    double growth = 0.0;
+    {
+        int cnt = 0;
+        std::vector<int> rows, ends;
+        marks[0].need(n);
+        for (const auto& t : segs) {
+            const size_t nt = t.size() - 1;
+            const size_t step = std::max<size_t>(1, nt * segs.size() / 8);
+            for (size_t i = nt / 2 % step; i < nt; i += step) {
+                rows.clear();
+                for (int64_t r = t[i]; r < t[i + 1]; ++r) rows.push_back((int)r);
+                const int d = std::min(terms, 8);
+                grow(A, marks[0], rows, d, n + 1, ends);
+                if (ends.back() * 2 < t.back() - t.front() || cnt == 0) {
+                    growth += (std::sqrt((double)ends.back()) - std::sqrt((double)ends[0])) / d;
+                    ++cnt;
+                }
+            }
+        }
+        growth /= std::max(cnt, 1);
+    }
+
+    // Depth and owned rows: the least estimated cycles of a compute unit per
+    // owned row and step.  A row of three
+    // entries costs about 0.9 cycles a term (LDS: its entries, its own
+    // value twice); bytes
+    // from HBM pass at about 10 a cycle; of tables that several groups read,
+    // two thirds come from L2.  With two workgroups a compute unit most of
+    // the lesser of the two hides behind the other.  Measured, one pass a
+    // step against two (ms a step): 8.4M rows, four complex64 groups 2.26 /
+    // 2.21; 0.9M rows, eight complex128 groups 0.71 / 0.57; 0.5M rows, six
+    // complex64 groups (15 terms) 0.25 / 0.30; 4.2M rows, one complex128
+    // group 0.36 / 0.37.
+    const int64_t cap = std::min<int64_t>((int64_t)nr * kRingLanes,
+                                          (int64_t)h->max_lds / kRingPerCu / unit_bytes);
+    const int64_t own_cap = (int64_t)nro * kRingLanes;
+    const double row_cost = 0.18 * ((W ? W : wmax) + 2);
+    const double fill = 0.85;   // blocks are not squares: room for their rings
+    int depth = 0;
+    int64_t target = 0;
+    double best = 0.0;
+    for (int passes = 1; passes <= 8; ++passes) {
+        const int d = (terms + passes - 1) / passes;
+        if (d > kRingMax || (passes > 1 && d < 3)) continue;
+        const double side = std::sqrt(fill * cap) - growth * d;
+        if (side < 8.0) continue;
+        const double slots = (double)h->num_cus * kRingPerCu;
+        double own = std::min<double>((double)own_cap, side * side);
+        // a small sample: a block for every workgroup that runs at once
+        own = std::min(own, std::max(64.0, (double)covered * groups / (0.9 * slots)));
+        double comp = 0.0;
+        for (int k = 0; k < d; ++k) {
+            const double s = std::sqrt(own) + growth * k;
+            comp += std::max(row_cost * s * s, 300.0);
+        }
+        const double all = std::pow(std::sqrt(own) + growth * d, 2);
+        const double table = 8.0 + (W ? W : wmax) * (double)vsz;
+        const double bytes = all * (4.0 + unit_bytes * (passes > 1 ? 2 : 1)) +
+                             all * (groups > 1 ? table / 3.0 : table) +
+                             own * unit_bytes * (passes > 1 ? 4 : 3);
+        const double mem = bytes / 10.0 + 2000.0;
+        const double cost = passes * (std::max(comp, mem) + 0.4 * std::min(comp, mem)) / own;
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            depth = d;
+            target = (int64_t)own;
+        }
+    }
+    if (depth == 0) return nullptr;
+
+    // atoms: runs of a tile's rows no longer than a fraction of the target
+    std::vector<Atom> atoms;
+    {
+        std::vector<std::pair<int, int64_t>> tiles;   // (segment, first row's place)
+        for (size_t sg = 0; sg < segs.size(); ++sg)
+            for (size_t i = 0; i + 1 < segs[sg].size(); ++i) tiles.emplace_back((int)sg, (int64_t)i);
+        std::vector<std::vector<Atom>> cut(tiles.size());
+        const double piece = std::max(24.0, target / 8.0);
+        parallel_for((int64_t)tiles.size(), 16, [&](int64_t i, int th) {
+            marks[th].need(n);
+            const auto& t = segs[tiles[i].first];
+            const int64_t a = t[tiles[i].second], b = t[tiles[i].second + 1];
+            const int k = std::max(1, (int)std::lround(std::sqrt((b - a) / piece)));
+            split_tile(A, marks[th], a, b, k, tiles[i].first, cut[i]);
+        });
+        for (auto& c : cut)
+            for (auto& a : c) atoms.push_back(std::move(a));
+    }
+    const int na = (int)atoms.size();
+    std::vector<int> atom_of((size_t)n, -1);
+    parallel_for(na, 64, [&](int64_t i, int) {
+        for (int r : atoms[i].rows) atom_of[r] = (int)i;
+    });
+    std::vector<std::vector<std::pair<int, int>>> nbr((size_t)na);   // (atom, couplings)
+    parallel_for(na, 64, [&](int64_t i, int) {
+        auto& v = nbr[i];
+        for (int r : atoms[i].rows)
+            for (int j = 0, w = A.width(r); j < w; ++j) {
+                const int t = atom_of[A.cols[A.elem(r, j)]];
+                if (t == (int)i || t < 0) continue;
+                size_t q = 0;
+                while (q < v.size() && v[q].first != t) ++q;
+                if (q == v.size()) v.emplace_back(t, 0);
+                ++v[q].second;
+            }
+    });
+    // grow each block from the first free atom by the neighbour with the
+    // most couplings to it (most of its own couplings first among equals)
+    std::vector<std::vector<int>> groups_of;
+    {
+        std::vector<char> used((size_t)na, 0);
+        std::vector<int> link((size_t)na, 0), cand;
+        for (int i = 0; i < na; ++i) {
+            if (used[i]) continue;
+            std::vector<int> blk{i};
+            used[i] = 1;
+            int64_t rows = (int64_t)atoms[i].rows.size();
+            cand.clear();
+            auto join = [&](int a) {
+                for (const auto& e : nbr[a]) {
+                    if (used[e.first]) continue;
+                    if (link[e.first] == 0) cand.push_back(e.first);
+                    link[e.first] += e.second;
+                }
+            };
+            join(i);
+            for (;;) {
+                int bi = -1;
+                double bv = 0.0;
+                for (size_t q = 0; q < cand.size(); ++q) {
+                    const int c = cand[q];
+                    const int64_t sz = (int64_t)atoms[c].rows.size();
+                    if (used[c] || rows + sz > target) continue;
+                    const double v = link[c] / std::sqrt((double)sz);
+                    if (bi < 0 || v > bv * 1.02 || (v > bv * 0.98 && c < bi)) {
+                        bi = c;
+                        bv = v;
+                    }
+                }
+                if (bi < 0) break;
+                used[bi] = 1;
+                blk.push_back(bi);
+                rows += (int64_t)atoms[bi].rows.size();
+                join(bi);
+            }
+            for (int c : cand) link[c] = 0;
+            std::sort(blk.begin(), blk.end());
+            groups_of.push_back(std::move(blk));
+        }
+    }
+    // small leftovers go to their neighbours, where these have room
+    {
+        std::vector<int> owner((size_t)na, -1), rows_of(groups_of.size(), 0);
+        for (size_t b = 0; b < groups_of.size(); ++b)
+            for (int at : groups_of[b]) {
+                owner[at] = (int)b;
+                rows_of[b] += (int)atoms[at].rows.size();
+            }
+        std::vector<int> by_size(groups_of.size());
+        for (size_t b = 0; b < by_size.size(); ++b) by_size[b] = (int)b;
+        std::stable_sort(by_size.begin(), by_size.end(),
+                         [&](int x, int y) { return rows_of[x] < rows_of[y]; });
+        const int64_t most = std::min<int64_t>(own_cap, target + target / 25);
+        for (int b : by_size) {
+            if (rows_of[b] * 5 > target * 3) break;
+            std::vector<std::pair<int, int>> moves;
+            std::vector<std::pair<int, int>> added;   // (block, rows)
+            for (int at : groups_of[b]) {
+                int to = -1, link = 0;
+                for (const auto& e : nbr[at]) {
+                    const int o = owner[e.first];
+                    if (o == b || atoms[e.first].seg != atoms[at].seg || e.second <= link) continue;
+                    int64_t r = rows_of[o] + (int64_t)atoms[at].rows.size();
+                    for (const auto& x : added)
+                        if (x.first == o) r += x.second;
+                    if (r > most) continue;
+                    to = o;
+                    link = e.second;
+                }
+                if (to < 0) break;
+                moves.emplace_back(at, to);
+                added.emplace_back(to, (int)atoms[at].rows.size());
+            }
+            if (moves.size() < groups_of[b].size()) continue;
+            for (const auto& m : moves) {
+                owner[m.first] = m.second;
+                groups_of[m.second].push_back(m.first);
+                rows_of[m.second] += (int)atoms[m.first].rows.size();
+            }
+            groups_of[b].clear();
+            rows_of[b] = 0;
+        }
+        std::vector<std::vector<int>> kept;
+        for (auto& g : groups_of)
+            if (!g.empty()) {
+                std::sort(g.begin(), g.end());
+                kept.push_back(std::move(g));
+            }
+        groups_of = std::move(kept);
+    }
+    std::stable_sort(groups_of.begin(), groups_of.end(),
+                     [&](const std::vector<int>& x, const std::vector<int>& y) {
+                         return atoms[x[0]].seg < atoms[y[0]].seg;
+                     });
+
+    // rings and tables, split where a block does not fit
+    const int64_t ng = (int64_t)groups_of.size();
+    std::vector<std::vector<Block>> made((size_t)ng);
+    std::atomic<bool> fits{true};
+    parallel_for(ng, 4, [&](int64_t i, int th) {
+        Marks& mk = marks[th];
+        mk.need(n);
+        std::vector<std::vector<int>> todo(1);
+        for (int a : groups_of[i])
+            todo[0].insert(todo[0].end(), atoms[a].rows.begin(), atoms[a].rows.end());
+        std::sort(todo[0].begin(), todo[0].end());
+        while (!todo.empty() && fits) {
+            Block b;
+            b.rows = todo.back();
+            todo.pop_back();
+            b.seg = atoms[groups_of[i][0]].seg;
+            const size_t n0 = b.rows.size();
+            if ((int64_t)n0 > own_cap || !grow(A, mk, b.rows, depth, cap, b.ends)) {
+                if (n0 < 16) {
+                    fits = false;
+                    return;
+                }
+                b.rows.resize(n0);
+                todo.emplace_back(b.rows.begin() + n0 / 2, b.rows.end());
+                todo.emplace_back(b.rows.begin(), b.rows.begin() + n0 / 2);
+                continue;
+            }
+            for (int r : b.rows) b.w = std::max(b.w, A.width(r));
+            made[i].push_back(std::move(b));
+        }
+    });
+    if (!fits) return nullptr;
+    auto R = std::make_shared<Ring>();
+    std::vector<Block*> blocks;
+    for (auto& v : made)
+        for (auto& b : v) blocks.push_back(&b);
+    const int nb = (int)blocks.size();
+    std::vector<RingMeta> meta((size_t)nb);
+    std::vector<int> ends((size_t)nb * (depth + 1));
+    int64_t nrow = 0, ntab = 0, nent = 0, computed = 0;
+    R->seg_block.clear();
+    for (int b = 0; b < nb; ++b) {
+        while ((int)R->seg_block.size() <= blocks[b]->seg) R->seg_block.push_back(b);
+        const Block& k = *blocks[b];
+        RingMeta& m = meta[b];
+        const int nC = k.ends[depth - 1];
+        m.offR = nrow;
+        m.offT = ntab;
+        m.offE = nent;
+        m.w = k.w;
+        m.pad = nC;
+        nrow += k.ends[depth];
+        ntab += W ? nC : 0;
+        nent += W ? 0 : (int64_t)nC * k.w;
+        computed += nC;
+        for (int q = 0; q <= depth; ++q) ends[(size_t)b * (depth + 1) + q] = k.ends[q];
+        R->rows_max = std::max(R->rows_max, k.ends[depth]);
+        R->owned_max = std::max(R->owned_max, k.ends[0]);
+    }
+    while (R->seg_block.size() < segs.size() + 1) R->seg_block.push_back(nb);
+    std::vector<int> rows((size_t)nrow);
+    std::vector<uint16_t> idx((size_t)(W ? ntab * 4 : nent));
+    std::vector<unsigned char> vals((size_t)(W ? ntab * W : nent) * vsz);
+    const int shift = unit_bytes == 16 ? 4 : 3;
+    TBG_REQUIRE(unit_bytes == 16 || unit_bytes == 8, "internal: unit of another size");
+    std::atomic<bool> sound{true};
+    parallel_for(nb, 4, [&](int64_t b, int th) {
+        const Block& k = *blocks[b];
+        const RingMeta& m = meta[b];
+        Marks& mk = marks[th];
+        mk.need(n);
+        const int st = ++mk.stamp;
+        for (size_t q = 0; q < k.rows.size(); ++q) {
+            mk.mark[k.rows[q]] = st;
+            mk.loc[k.rows[q]] = (int)q;
+            rows[m.offR + q] = k.rows[q];
+        }
+        // every position a row of ring q reads lies in the rings up to q + 1,
+        // which the pass holds one term earlier
+        int ring = 0;
+        for (int l = 0; l < m.pad; ++l) {
+            while (l >= k.ends[ring]) ++ring;
+            const int r = k.rows[l], w = A.width(r);
+            const int ww = W ? W : m.w;
+            for (int j = 0; j < ww; ++j) {
+                const int64_t at = m.offE + (int64_t)j * m.pad + l;
+                const int64_t av = W ? (m.offT + l) * W + j : at;
+                int pos = l;                    // (zero value on the row itself)
+                if (j < w) {
+                    const int64_t e = A.elem(r, j);
+                    const int c = A.cols[e];
+                    if (mk.mark[c] != st || mk.loc[c] >= k.ends[ring + 1]) {
+                        sound = false;
+                        return;
+                    }
+                    pos = mk.loc[c];
+                    std::memcpy(vals.data() + av * vsz, A.vals.data() + e * vsz, vsz);
+                } else {
+                    std::memset(vals.data() + av * vsz, 0, vsz);
+                }
+                if (W) {
+                    uint32_t& word = reinterpret_cast<uint32_t*>(idx.data())[(m.offT + l) * 2 +
+                                                                              j % 2];
+                    word |= j < 2 ? (uint32_t)pos << shift : (uint32_t)pos << 18;
+                } else {
+                    idx[at] = (uint16_t)pos;
+                }
+            }
+        }
+    });
+    TBG_REQUIRE(sound, "internal: resident-pass table out of range");
+    R->depth = depth;
+    R->width = W;
+    R->nblocks = nb;
+    R->rows_lane = nr;
+    R->owned_lane = nro;
+    R->halo = (double)computed / (double)covered;
+    R->sched[0] = (int64_t)(rows.size() * 4 + idx.size() * 2 + vals.size()) +
+                  (int64_t)nb * (int64_t)(sizeof(RingMeta) + 4 * (depth + 1));
+    R->sched[1] = nrow;
+    R->sched[2] = computed;
+    R->sched[3] = covered;
+    auto up = [&](DevBuf& d, const void* p, size_t bytes) {
+        d.alloc(std::max<size_t>(bytes, 16));
+        if (bytes) TBG_HIP(hipMemcpyAsync(d.p, p, bytes, hipMemcpyHostToDevice, h->stream));
+    };
+    up(R->meta, meta.data(), meta.size() * sizeof(RingMeta));
+    up(R->ends, ends.data(), ends.size() * sizeof(int));
+    up(R->rows, rows.data(), rows.size() * sizeof(int));
+    // (a group of rows past the last table stays inside the allocation)
+    idx.resize(idx.size() + kRingLanes * 4);
+    vals.resize(vals.size() + kRingLanes * 4 * vsz);
+    up(R->idx, idx.data(), idx.size() * sizeof(uint16_t));
+    up(R->vals, vals.data(), vals.size());
+    TBG_HIP(hipStreamSynchronize(h->stream));
+    return R;
+}
+
+std::shared_ptr<Ring> get_ring(tbg_handle* h, const tbg_ham* H, int real_bytes, int V, int groups,
+                               int terms) {
+    if (!h->resident || H->tiles.size() < 2) return nullptr;
+    if (terms > kRingMax) terms = 20;    // a long series: any depth divides it well
+    const std::string key = std::to_string(V) + "|" + std::to_string(groups) + "|" +
+                            std::to_string(terms);
+    for (const auto& kv : H->rings)
+        if (kv.first == key) return kv.second;
+    BlockSrc src;
+    src.cols = H->cols.as<int>();
+    src.vals = H->vals.p;
+    src.sw = H->slice_w.as<int>();
+    src.soff = H->slice_off.as<int64_t>();
+    src.nslices = H->nslices;
+    src.padded = H->padded;
+    src.nrows = H->n;
+    src.vsz = H->vals.bytes / (size_t)std::max<int64_t>(H->padded, 1);
+    auto R = build_ring(h, src, {H->tiles}, real_bytes, V, groups, terms, H->real_vals);
+    H->rings.emplace_back(key, R);
+    if (H->rings.size() > 2) H->rings.erase(H->rings.begin());
+    return R;
+}
+
+template <typename R>
+void launch_ring(const RingArgs<R>& a, const Ring& r, int V, bool real_vals, hipStream_t s) {
+    if (a.T < 1 || a.T > r.depth || a.depth != r.depth || r.depth > kRingMax)
+        throw Error{TBG_EINVAL, "internal: more terms in a pass than the tables' rings allow"};
+    if (r.rows_lane != ring_rows(sizeof(R), V, real_vals, r.width) ||
+        r.owned_lane != ring_owned(sizeof(R), V, real_vals, r.width) ||
+        r.rows_max > r.rows_lane * kRingLanes || r.owned_max > r.owned_lane * kRingLanes ||
+        a.lds_rows < r.rows_max)
+        throw Error{TBG_EINVAL, "internal: resident pass beyond its workgroup"};
+    if ((a.q1 == nullptr) != (a.q2 == nullptr) || a.acc == nullptr || a.p1 == nullptr ||
+        (!a.first && a.p0 == nullptr))
+        throw Error{TBG_EINVAL, "internal: resident pass without its vectors"};
+#define TBG_RING_RV(VV)                                                        \
+    do {                                                                       \
+        if (real_vals) launch_ring_rt<R, VV, true>(a, r, s);                   \
+        else launch_ring_rt<R, VV, false>(a, r, s);                            \
+    } while (0)
+    if constexpr (sizeof(R) == 4) {
+        if (V == 2) {
+            TBG_RING_RV(2);
+            return;
+        }
+    }
+    if (V != 1) throw Error{TBG_EINVAL, "internal: unsupported vectors per lane"};
+    TBG_RING_RV(1);
+#undef TBG_RING_RV
+}
+template void launch_ring<float>(const RingArgs<float>&, const Ring&, int, bool, hipStream_t);
+template void launch_ring<double>(const RingArgs<double>&, const Ring&, int, bool, hipStream_t);
+
+void prepare_ring(int max_lds) {
+    allow_ring_lds<float, 1, true>(max_lds);
+    allow_ring_lds<float, 1, false>(max_lds);
+    allow_ring_lds<float, 2, true>(max_lds);
+    allow_ring_lds<float, 2, false>(max_lds);
+    allow_ring_lds<double, 1, true>(max_lds);
+    allow_ring_lds<double, 1, false>(max_lds);
+}
+
+}  // namespace tbg

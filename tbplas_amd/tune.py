@@ -26,6 +26,8 @@ CANDIDATES = [(bpc, stage) for bpc in (4, 8, 12, 16) for stage in (True, False)]
 # untuned: blocks per CU and staging; the terms per pass are those the
 # tiles of auto_tile_nm are sized for (sample.pass_terms)
 DEFAULT = (16, True)
+# "terms per pass" of a shape that runs resident passes (up to a whole step)
+RESIDENT = 32
 
 _lock = threading.Lock()
 _mem = {}
@@ -113,7 +115,7 @@ def autotune(H, K, bes, steps=6, warmup=2, candidates=None, use_cache=True):
             timings[cand + (1,)] = timed(cand + (1,))
         best = min(timings, key=timings.get)
         if all(getattr(Hi, "tiled", False) for Hi in hams):
-            for terms in (3, 4, 5):
+            for terms in (3, 4, 5, RESIDENT):
                 blocked = best[:2] + (terms,)
                 timings[blocked] = timed(blocked)
             best = min(timings, key=timings.get)
@@ -128,7 +130,9 @@ def autotune(H, K, bes, steps=6, warmup=2, candidates=None, use_cache=True):
 
 def _set(handle, shape):
     handle.set_tuning(shape[0], shape[1])
-    handle.set_blocking(shape[2] > 1, terms=max(int(shape[2]), 3))
+    terms = int(shape[2])
+    handle.set_blocking(terms > 1, terms=5 if terms == RESIDENT else max(terms, 3))
+    handle.set_resident(terms == RESIDENT)
 
 
 def apply(H, K, bes, enabled=True):
@@ -141,4 +145,5 @@ def apply(H, K, bes, enabled=True):
     prec = "fp32" if H0.precision == _lib.TBG_FP32 else "fp64"
     shape = DEFAULT + (pass_terms(K, prec),)
     _set(H0.handle, shape)
+    H0.handle.set_resident(True)
     return shape

@@ -1,0 +1,196 @@
+"""Resident passes (up to a whole time step per launch on blocks held in LDS
+and registers) against one term per pass on the same Hamiltonian: states bit
+for bit, correlations to the grouping of their FP64 sums (1e-13, sums of at
+most a few thousand partials of size <= 1)."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle
+import tbplas_amd as tb
+from tbplas_amd import tbpm
+from conftest import golden, tau_of
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def handle(gpu):
+    h = tb._lib.Handle(0)
+    yield h
+    h.close()
+
+
+def _sample(L1, L2, field=0.0, vac=0.02, W=0.6, seed=11):
+    v = tb.random_vacancies(2 * L1 * L2, vac, seed) if vac else None
+    s = tb.make_graphene_sample(L1, L2, vacancies=v)
+    if W:
+        tb.add_anderson_disorder(s, W, seed + 1)
+    if field:
+        s.set_magnetic_field(field, 0)
+    s.rescale_ham(9.0)
+    return s, oracle.build_ham_csr(s.orb_eng, s.hop_i, s.hop_j, s.hop_v)
+
+
+def _states(n, K, seed=21):
+    return tb.states.random_states(n, tb.states.sample_seeds(seed, K))
+
+
+def _agree(h, H, bes, psi, T=9):
+    """Resident passes on, then off: steps, a long series and C(t)."""
+    coef = np.cos(np.arange(75) * 0.7) / (1.0 + np.arange(75))
+    res = {}
+    for on in (True, False):
+        h.set_blocking(False)
+        h.set_resident(on)
+        h.set_kernel_timing(True)
+        steps = [tbpm.cheb_step(H, bes, psi, fwd) for fwd in (True, False)]
+        h.set_kernel_timing(False)
+        assert any(k.startswith("ring") for k in h.kernel_times()) == on
+        res[on] = steps + [tbpm.cheb_poly(H, coef, psi),
+                           tbpm.corr_dos(H, bes, psi, T, chk_thr=1e-4)]
+    for a, b in zip(res[True][:3], res[False][:3]):
+        np.testing.assert_array_equal(a, b)
+    assert np.max(np.abs(res[True][3] - res[False][3])) < 1e-13
+    return res[True][3]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("K", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("L1,L2,field,W,tile", [
+    (5, 4, 0.0, 0.0, 0.5),        # blocks that wrap around the sample
+    (48, 31, 0.0, 0.6, 0.9),      # four entries a row
+    (40, 52, 30.0, 0.0, 1.7),     # three complex entries a row
+    (33, 47, 30.0, 0.6, 30.0)])   # one tile: split into blocks
+def test_states_bitwise(handle, prec, K, L1, L2, field, W, tile):
+    s, (ip, ix, dt) = _sample(L1, L2, field, 0.02 if L1 > 8 else 0.0, W)
+    order, tiles = s.tile_order(tile, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision=prec, handle=handle, order=order,
+                         tiles=tiles)
+    bes = tbpm.bessel_series(tau_of(s), 1e-15)
+    psi = _states(s.num_orb, K)
+    c = _agree(handle, H, bes, psi)
+    ref = oracle.orc_tbpm_dos(ip, ix, dt, bes, psi[:1], 9)
+    assert np.max(np.abs(c[:1] - ref)) < (1e-12 if prec == "fp64" else 2e-5)
+    H.close()
+
+
+@pytest.mark.parametrize("nterms", [3, 4, 22, 34, 60])
+def test_series_lengths(handle, nterms):
+    """Passes of uneven length: short series, one term over a pass, more
+    terms than one pass may have."""
+    s, (ip, ix, dt) = _sample(60, 60)
+    order, tiles = s.tile_order(1.3, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision="fp64", handle=handle, order=order,
+                         tiles=tiles)
+    tau = {3: 0.2, 4: 0.4, 22: 3.2, 34: 9.0, 60: 27.0}[nterms]
+    bes = np.array([float(x) for x in tbpm.bessel_series(tau, 1e-30)[:nterms]])
+    psi = _states(s.num_orb, 2)
+    _agree(handle, H, bes, psi, T=3)
+    H.close()
+
+
+@pytest.mark.parametrize("prec,K,tile", [("fp32", 8, 4.8), ("fp64", 8, 3.2), ("fp64", 1, 7.5),
+                                         ("fp32", 12, 3.8), ("fp32", 64, 1.5), ("fp32", 1, 16.0)])
+def test_large_blocks(handle, prec, K, tile):
+    """262,144 orbitals: blocks at the limits of a workgroup's LDS and
+    registers, several per compute unit."""
+    s, (ip, ix, dt) = _sample(300, 437, vac=0.0, W=0.0)
+    order, tiles = s.tile_order(tile, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision=prec, handle=handle, order=order,
+                         tiles=tiles)
+    _agree(handle, H, tbpm.bessel_series(tau_of(s), 1e-15), _states(s.num_orb, K), T=5)
+    H.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_wide_rows_and_scattered_tiles(handle, prec):
+    """A random sparse Hermitian matrix (rows of ~9 entries) with tiles that
+    are not spatial: every ring reaches the whole matrix."""
+    rng = np.random.default_rng(31)
+    n, m = 700, 2800
+    hi, hj = rng.integers(0, n, m), rng.integers(0, n, m)
+    keep = hi != hj
+    hi, hj = hi[keep], hj[keep]
+    hv = (rng.normal(size=len(hi)) + 1j * rng.normal(size=len(hi))) * 0.05
+    ip, ix, dt = oracle.build_ham_csr(rng.uniform(-0.2, 0.2, n), hi, hj, hv)
+    order = rng.permutation(n).astype(np.int64)
+    H = tbpm.Hamiltonian(n, ip, ix, dt, precision=prec, handle=handle, order=order,
+                         tiles=np.r_[np.arange(0, n, 32), n].astype(np.int64))
+    bes = tbpm.bessel_series(math.pi, 1e-14)
+    psi = _states(n, 3, seed=24)
+    c = _agree(handle, H, bes, psi)
+    ref = oracle.orc_tbpm_dos(ip, ix, dt, bes, psi, 9)
+    assert np.max(np.abs(c - ref)) < (1e-12 if prec == "fp64" else 2e-5)
+    H.close()
+
+
+@pytest.mark.parametrize("prec,K", [("fp64", 1), ("fp32", 3), ("fp32", 4)])
+def test_batch(handle, prec, K):
+    """Uneven instances, one of them complex; correlations stay per instance."""
+    hams, psis, refs = [], [], []
+    bes = None
+    for i, (L1, L2) in enumerate([(9, 14), (30, 22), (5, 5), (41, 17)]):
+        s, (ip, ix, dt) = _sample(L1, L2, 25.0 if i == 3 else 0.0, 0.02 * (i % 2), 0.3 * i,
+                                  seed=40 + i)
+        bes = tbpm.bessel_series(tau_of(s), 1e-15)
+        order, tiles = s.tile_order(0.8, return_tiles=True)
+        hams.append(tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision=prec, handle=handle,
+                                     order=order, tiles=tiles))
+        psis.append(_states(s.num_orb, K, seed=400 + i))
+        refs.append(oracle.orc_tbpm_dos(ip, ix, dt, bes, psis[-1], 20))
+    handle.set_resident(True)
+    out = tbpm.corr_dos_batch(hams, bes, psis, 20, chk_thr=1e-4)
+    again = tbpm.corr_dos_batch(hams, bes, psis, 20, chk_thr=1e-4)
+    for o, a, r in zip(out, again, refs):
+        np.testing.assert_array_equal(o, a)
+        assert np.max(np.abs(o - r)) < (1e-12 if prec == "fp64" else 2e-5)
+    for H in hams:
+        H.close()
+
+
+@pytest.mark.parametrize("what", ["ac", "dc"])
+def test_conductivity_fixtures(handle, what):
+    """The reference's AC and DC correlations on its own states."""
+    g = golden(f"ref_{what}.npz")
+    n = len(g["indptr"]) - 1
+    handle.set_resident(True)
+    H = tbpm.Hamiltonian(n, g["indptr"], g["indices"], g["hop"], g["dx"], g["dy"],
+                         cur_scale=float(g["rescale"]), precision="fp64", handle=handle,
+                         tiles=np.r_[np.arange(0, n, 32), n].astype(np.int64))
+    if what == "ac":
+        cF, cO = (tbpm.fermi_cheb_coef(2 ** 15, float(g["beta_re"]), float(g["mu_re"]), om, 1e-12)
+                  for om in (False, True))
+        avg = np.mean(tbpm.corr_ac(H, g["bes"], cF, cO, g["psi0"], int(g["T"])), axis=0)
+        ref = g["corr"]
+        assert np.max(np.abs(avg - ref)) < 1e-11 * max(1.0, np.max(np.abs(ref)))
+    else:
+        dos, dc = tbpm.corr_dc(H, g["bes"], g["psi0"], int(g["T"]), float(g["t_step"]),
+                               g["energies"], g["en_inds"])
+        ne = len(g["en_inds"])
+        assert np.max(np.abs(dos.mean(axis=0) - g["dos"])) < 1e-12
+        assert np.max(np.abs(dc.mean(axis=0) - g["dc"][:, :ne])) < \
+            1e-10 * max(1.0, np.max(np.abs(g["dc"])))
+    H.close()
+
+
+def test_graph_replay_and_timing(handle):
+    """Replayed steps equal launched ones; the step counter and the norm
+    check work with resident passes."""
+    s, (ip, ix, dt) = _sample(40, 40)
+    order, tiles = s.tile_order(1.0, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision="fp32", handle=handle, order=order,
+                         tiles=tiles)
+    bes = tbpm.bessel_series(tau_of(s), 1e-15)
+    psi = _states(s.num_orb, 4)
+    handle.set_resident(True)
+    out = []
+    for graph in (True, True, False):
+        handle.set_graph(graph)
+        out.append(tbpm.corr_dos(H, bes, psi, 70, chk_thr=1e-4))
+    np.testing.assert_array_equal(out[0], out[1])
+    np.testing.assert_array_equal(out[0], out[2])
+    with pytest.raises(tb._lib.NormError):
+        tbpm.corr_dos(H, bes, psi, 20, chk_step=10, chk_thr=1e-30)
+    H.close()
