@@ -805,10 +805,13 @@ def dc_workload(args):
     ne = len(inds)
 
     def bytes_of(kind):
-        if kind == "dc_qe":    # psi(+t), psi(-t), psi0 read; QE read and written (FP64)
-            return 3 * per * n * 8 + 2 * ne * per * n * 16
+        # one launch works on the states of a block of up to 16 steps
+        if kind == "dc_qe":    # psi(+t), psi(-t) read; QE read and written (FP64)
+            steps = Tp / math.ceil(Tp / 16)
+            return steps * 2 * per * n * 8 + 2 * ne * per * n * 16
         if kind == "dc_dot":   # J_a psi(t) read, J_a QE read (FP64)
-            return 2 * per * n * 8 + 2 * ne * per * n * 16
+            steps = Tp / (1 + math.ceil((Tp - 1) / 16))
+            return steps * 2 * per * n * 8 + 2 * ne * per * n * 16
         return pass_bytes_fn(sched, n, nnz, 2 * per, 8, real)(kind)
     value = 2 * K * (2 * T - 1) / dt
     return {"metric": "DC correlation step·vectors/s (disordered field-threaded graphene)",

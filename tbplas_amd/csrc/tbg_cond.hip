@@ -159,107 +159,133 @@ k_accorr(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ 
     }
 }
 
-// QE(r, e, s) initialised to psi0 (FP64, tbpm.f90:600-603).
-// psi0 is in the caller's row order; layout row r holds caller row perm[r].
-__global__ void k_qe_init(const double2* __restrict__ psi0, int64_t n, int K, int n_en,
-                          int64_t n_pad, const int* __restrict__ perm, double2* __restrict__ qe) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nq = (int64_t)n_en * K;
-    if (i >= n_pad * nq) return;
-    const int64_t r = i / nq;
-    const int q = (int)(i - r * nq);
-    const int s = q % K;
-    const int64_t c = r < n ? (perm ? (int64_t)perm[r] : r) : 0;
-    qe[i] = r < n ? psi0[(int64_t)s * n + c] : make_double2(0.0, 0.0);
+// The DC run keeps the outputs of S (up to 16) steps and works on them at
+// once: the quasi-eigenstates are read and written, and the vectors Y read,
+// once per S steps instead of at every step.  With 28 energies of 8 states
+// on 0.5M orbitals the quasi-eigenstates are 1.9 GB and Y 3.8 GB: a step's
+// update took 786 us and its correlations 637 us, both at 5 TB/s; 16 steps
+// together take 1119 and 1134 us.
+constexpr int kDcSteps = 16;
+struct DcStates {
+    const void* p[kDcSteps];   // states after the block's steps
+};
+
+// FP64 vectors of K states for several energies: state s of row r for energy
+// e at e * K * n_pad + lay.at(r, s), laid out as the first K slots of the
+// run's states are (QLay::lin: those K slots are the first K * n_pad
+// elements of a state buffer, slots K .. 2K the next), else row by row.
+struct QLay {
+    Lay lay{1};
+    int64_t stride = 0;
+    bool lin = false;
+    __host__ __device__ __forceinline__ int64_t at(int64_t e, int64_t r, int s) const {
+        return e * stride + lay.at(r, s);
+    }
+};
+
+static QLay q_layout(const Lay& x, int K, int64_t n_pad) {
+    QLay q;
+    q.stride = K * n_pad;
+    q.lin = x.sh >= 0 && K % x.unit() == 0;
+    q.lay = q.lin ? Lay(K, x.sh, x.plane) : Lay(K);
+    return q;
 }
 
-// After step t (counter = t): DOS correlation <psi0|psi(+t)> and the
-// quasi-eigenstate update (tbpm.f90:616-638).
-template <typename R>
+// QE(e, r, s) initialised to psi0 (FP64, tbpm.f90:600-603); psi0 is in the
+// caller's row order, layout row r holds caller row perm[r].
+__global__ void k_qe_init(const double2* __restrict__ psi0, int64_t n, int K, int64_t n_pad,
+                          const int* __restrict__ perm, QLay ql, int n_en,
+                          double2* __restrict__ qe) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_pad * K) return;
+    const int s = (int)(i / n_pad);
+    const int64_t r = i - s * n_pad;
+    const int64_t c = r < n ? (perm ? (int64_t)perm[r] : r) : 0;
+    const double2 v = r < n ? psi0[(int64_t)s * n + c] : make_double2(0.0, 0.0);
+    for (int e = blockIdx.y; e < n_en; e += gridDim.y) qe[ql.at(e, r, s)] = v;
+}
+
+// The quasi-eigenstate update (tbpm.f90:616-638) of `count` steps, the last
+// of them step *counter: QE_e += W(t) (P(t, e) psi(t) + conj(P(t, e)) psi(-t))
+// in the order of the steps, with pw(t, e) = W(t) P(t, e).  A thread keeps
+// EC energies of one state of one row in registers over the block's steps;
+// pw's rows are `pitch` (a multiple of EC) wide, zeros behind the n_en.
+// Bound by HBM: QE read and written, the states once per EC energies: 16
+// steps at 28 energies of 8 FP32 states, 0.5M orbitals, move 5.9 GB in 1119
+// us (5.3 TB/s; 16 single steps took 12.6 ms).  EC = 16 holds 64 registers
+// of sums; fewer would read the states more often.
+template <typename R, bool LIN, int EC>
 __global__ void __launch_bounds__(256)
-k_qe(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, Lay lay,
-     int K, const typename CplxT<R>::T* __restrict__ psi, double2* __restrict__ qe, int n_en,
-     const double2* __restrict__ ptab, const double* __restrict__ wtab,
-     const int* __restrict__ counter, double* __restrict__ part) {
-    __shared__ double sh[256 * 2];
-    const int c = remap_chunk(blockIdx.x, gridDim.x);
-    const int64_t r0 = chunk[c] * 64, r1 = chunk[c + 1] * 64;
-    const int t = *counter;
-    const double W = wtab[t - 1];
-    const double2* P = ptab + (int64_t)(t - 1) * n_en;
-    const int ng = 256 / K;
-    const int s = threadIdx.x % K, grp = threadIdx.x / K;
-    const int64_t nq = (int64_t)n_en * K;
-    double dr = 0.0, di = 0.0;
-    if (grp < ng) {
-        for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const auto p = X[lay.at(r, s)];
-            const auto q = X[lay.at(r, K + s)];
-            const auto z = psi[lay.at(r, s)];
-            const double pr = p.x, pi = p.y, qr = q.x, qi = q.y;
-            dr = fma((double)z.x, pr, fma((double)z.y, pi, dr));
-            di = fma((double)z.x, pi, fma(-(double)z.y, pr, di));
-            double2* row = qe + r * nq + s;
-            for (int e = 0; e < n_en; ++e) {
-                const double2 Pe = P[e];
-                double2 v = row[(int64_t)e * K];
-                // QE = QE + P*pos*W; QE = QE + conj(P)*neg*W
-                const double ar = Pe.x * pr - Pe.y * pi, ai = Pe.x * pi + Pe.y * pr;
-                v.x = v.x + ar * W;
-                v.y = v.y + ai * W;
-                const double br = Pe.x * qr + Pe.y * qi, bi = Pe.x * qi - Pe.y * qr;
-                v.x = v.x + br * W;
-                v.y = v.y + bi * W;
-                row[(int64_t)e * K] = v;
-            }
+k_qe(DcStates xs, int count, Lay lay, int K, int64_t n_pad, QLay ql, double2* __restrict__ qe,
+     int n_en, int pitch, const double2* __restrict__ pw, const int* __restrict__ counter) {
+    using C = typename CplxT<R>::T;
+    const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (m >= n_pad * K) return;
+    const int e0 = blockIdx.y * EC;
+    const int ne = min(EC, n_en - e0);
+    int64_t ip, iq, io;   // psi(t), psi(-t) and the energies' vectors
+    if constexpr (LIN) {
+        ip = io = m;
+        iq = m + n_pad * K;
+    } else {
+        const int64_t r = m / K;
+        const int s = (int)(m - r * K);
+        ip = lay.at(r, s);
+        iq = lay.at(r, K + s);
+        io = ql.lay.at(r, s);
+    }
+    double2* out = qe + (int64_t)e0 * ql.stride + io;
+    double2 v[EC];
+#pragma unroll
+    for (int e = 0; e < EC; ++e)
+        v[e] = e < ne ? out[e * ql.stride] : make_double2(0.0, 0.0);
+    const double2* w = pw + (int64_t)(*counter - count) * pitch + e0;
+    for (int j = 0; j < count; ++j, w += pitch) {
+        const C* X = reinterpret_cast<const C*>(xs.p[j]);
+        const C p = X[ip], q = X[iq];
+        const double pr = p.x, pi = p.y, qr = q.x, qi = q.y;
+#pragma unroll
+        for (int e = 0; e < EC; ++e) {
+            const double2 P = w[e];
+            v[e].x = fma(P.x, pr, fma(-P.y, pi, v[e].x));
+            v[e].y = fma(P.x, pi, fma(P.y, pr, v[e].y));
+            v[e].x = fma(P.x, qr, fma(P.y, qi, v[e].x));
+            v[e].y = fma(P.x, qi, fma(-P.y, qr, v[e].y));
         }
     }
-    sh[threadIdx.x * 2 + 0] = dr;
-    sh[threadIdx.x * 2 + 1] = di;
-    __syncthreads();
-    if (threadIdx.x < 2 * K) {
-        const int s2 = threadIdx.x / 2, q = threadIdx.x % 2;
-        double acc = 0.0;
-        for (int g = 0; g < ng; ++g) acc += sh[(g * K + s2) * 2 + q];
-        part[(int64_t)c * 2 * K + s2 * 2 + q] = acc;
-    }
+#pragma unroll
+    for (int e = 0; e < EC; ++e)
+        if (e < ne) out[e * ql.stride] = v[e];
 }
 
 // Per quasi-eigenstate q = e*K + s: <psi0_s|QE_q> (re, im) and |QE_q|^2.
-// Grid (chunks, q tiles of 256); part[c][q][3].
+// Grid x: chunks; part[c][q][3].
 __global__ void __launch_bounds__(256)
-k_qe_stats(const int64_t* __restrict__ chunk, const double2* __restrict__ qe, int64_t nq, int K,
-           const double2* __restrict__ psi0, int64_t n, const int* __restrict__ perm,
+k_qe_stats(const int64_t* __restrict__ chunk, const double2* __restrict__ qe, QLay ql, int64_t nq,
+           int K, const double2* __restrict__ psi0, int64_t n, const int* __restrict__ perm,
            double* __restrict__ part) {
-    __shared__ double sh[256 * 3];
-    const int c = remap_chunk(blockIdx.x, gridDim.x);
-    const int64_t r0 = chunk[c] * 64, r1 = std::min<int64_t>(chunk[c + 1] * 64, n);
-    const int64_t qb = (int64_t)blockIdx.y * 256;
-    const int nqt = (int)std::min<int64_t>(256, nq - qb);
-    const int ng = 256 / nqt;
-    const int qi = threadIdx.x % nqt, grp = threadIdx.x / nqt;
-    const int64_t q = qb + qi;
+    __shared__ double sh[4][3];
+    const int64_t r0 = chunk[blockIdx.x] * 64,
+                  r1 = std::min<int64_t>(chunk[blockIdx.x + 1] * 64, n);
+    for (int64_t q = blockIdx.y; q < nq; q += gridDim.y) {
     const int s = (int)(q % K);
-    double dr = 0, di = 0, nn = 0;
-    if (grp < ng) {
-        for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const double2 v = qe[r * nq + q];
-            const double2 z = psi0[(int64_t)s * n + (perm ? (int64_t)perm[r] : r)];
-            dr = fma(z.x, v.x, fma(z.y, v.y, dr));
-            di = fma(z.x, v.y, fma(-z.y, v.x, di));
-            nn = fma(v.x, v.x, fma(v.y, v.y, nn));
-        }
+    double d[3] = {0.0, 0.0, 0.0};
+    for (int64_t r = r0 + threadIdx.x; r < r1; r += 256) {
+        const double2 v = qe[ql.at(q / K, r, s)];
+        const double2 z = psi0[(int64_t)s * n + (perm ? (int64_t)perm[r] : r)];
+        d[0] = fma(z.x, v.x, fma(z.y, v.y, d[0]));
+        d[1] = fma(z.x, v.y, fma(-z.y, v.x, d[1]));
+        d[2] = fma(v.x, v.x, fma(v.y, v.y, d[2]));
     }
-    sh[threadIdx.x * 3 + 0] = dr;
-    sh[threadIdx.x * 3 + 1] = di;
-    sh[threadIdx.x * 3 + 2] = nn;
+    for (int o = 1; o < 64; o <<= 1)
+        for (int k = 0; k < 3; ++k) d[k] += __shfl_xor(d[k], o);
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 3; ++k) sh[threadIdx.x >> 6][k] = d[k];
     __syncthreads();
-    // nqt * 3 sums (up to 768) over 256 threads
-    for (int o = threadIdx.x; o < nqt * 3; o += blockDim.x) {
-        const int q2 = o / 3, k = o % 3;
-        double acc = 0.0;
-        for (int g = 0; g < ng; ++g) acc += sh[(g * nqt + q2) * 3 + k];
-        part[((int64_t)c * nq + qb + q2) * 3 + k] = acc;
+    if (threadIdx.x < 3)
+        part[((int64_t)blockIdx.x * nq + q) * 3 + threadIdx.x] =
+            ((sh[0][threadIdx.x] + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
+    __syncthreads();
     }
 }
 
@@ -273,102 +299,143 @@ __global__ void k_sum_rows(const double* __restrict__ part, int nchunks, int64_t
     out[q] = acc;
 }
 
-// |QE(r, e, s)|^2 in the caller's row order: out[(s * n_en + e) * n + perm[r]]
-// (tbpm.f90:820-825, one sample per state s).
-__global__ void k_qe_abs2(const double2* __restrict__ qe, int64_t n, int K, int n_en,
-                          const int* __restrict__ perm, double* __restrict__ out) {
-    const int64_t nq = (int64_t)n_en * K;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * nq) return;
-    const int64_t r = i / nq;
-    const int q = (int)(i - r * nq);
-    const int e = q / K, s = q - e * K;
-    const double2 v = qe[i];
+// |QE(e, r, s) / div(e, s)|^2 in the caller's row order:
+// out[(s * n_en + e) * n + perm[r]] (tbpm.f90:820-825, one sample per state
+// s).
+__global__ void k_qe_abs2(const double2* __restrict__ qe, QLay ql, int64_t n, int K, int n_en,
+                          const double* __restrict__ div, const int* __restrict__ perm,
+                          double* __restrict__ out) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n) return;
     const int64_t c = perm ? (int64_t)perm[r] : r;
-    out[((int64_t)s * n_en + e) * n + c] = v.x * v.x + v.y * v.y;
-}
-
-__global__ void k_qe_scale(double2* __restrict__ qe, int64_t total, int64_t nq,
-                           const double* __restrict__ div) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const double d = div[i % nq];
-    double2 v = qe[i];
-    v.x = v.x / d;
-    v.y = v.y / d;
-    qe[i] = v;
-}
-
-// Y[r][a*nq + q] = sum_j J_a[r,j] (QE[col][q] / adiv[q])  (tbpm.f90:680-684)
-template <typename R>
-__global__ void k_dc_y(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ jx,
-                       const typename CplxT<R>::T* __restrict__ jy,
-                       const int64_t* __restrict__ soff, const int* __restrict__ sw, int64_t n_pad,
-                       const double2* __restrict__ qe, int64_t nq, const double* __restrict__ adiv,
-                       double2* __restrict__ Y) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_pad * 2 * nq) return;
-    const int64_t r = i / (2 * nq);
-    const int64_t q2 = i - r * 2 * nq;
-    const int a = q2 >= nq ? 1 : 0;
-    const int64_t q = q2 - a * nq;
-    const typename CplxT<R>::T* J = a ? jy : jx;
-    const int64_t sl = r >> 6;
-    const int lr = (int)(r & 63);
-    const int64_t off = soff[sl];
-    const int w = sw[sl];
-    const double dv = adiv[q];
-    double yr = 0.0, yi = 0.0;
-    for (int j = 0; j < w; ++j) {
-        const int64_t e = off + (int64_t)j * 64 + lr;
-        const int col = cols[e];
-        const auto h = J[e];
-        const double2 v = qe[(int64_t)col * nq + q];
-        const double vr = v.x / dv, vi = v.y / dv;
-        const double hr = h.x, hi = h.y;
-        yr = hr * vr - hi * vi + yr;
-        yi = hr * vi + hi * vr + yi;
+    for (int64_t q = blockIdx.y; q < (int64_t)n_en * K; q += gridDim.y) {
+        const int64_t e = q / K, s = q - e * K;
+        const double2 v = qe[ql.at(e, r, (int)s)];
+        const double x = v.x / div[q], y = v.y / div[q];
+        out[(s * n_en + e) * n + c] = x * x + y * y;
     }
-    Y[i] = make_double2(yr, yi);
 }
 
-// dc[a][q] = <X2[a*K + s] | Y[a*nq + q]>, q = e*K + s.  Grid (chunks, tiles).
+// Y_a(e, r, s) = sum_j J_a[r,j] (QE(e, col, s) / div(e, s)), a = x, y
+// (tbpm.f90:680-684), both currents from one gather.
 template <typename R>
 __global__ void __launch_bounds__(256)
-k_dcdot(const int64_t* __restrict__ chunk, const typename CplxT<R>::T* __restrict__ X, Lay lay,
-        int K, const double2* __restrict__ Y, int64_t nq2, int64_t nq,
-        double* __restrict__ part) {
-    __shared__ double sh[256 * 2];
-    const int c = remap_chunk(blockIdx.x, gridDim.x);
-    const int64_t r0 = chunk[c] * 64, r1 = chunk[c + 1] * 64;
-    const int64_t qb = (int64_t)blockIdx.y * 256;
-    const int nqt = (int)std::min<int64_t>(256, nq2 - qb);
-    const int ng = 256 / nqt;
-    const int qi = threadIdx.x % nqt, grp = threadIdx.x / nqt;
-    const int64_t q2 = qb + qi;
-    const int a = q2 >= nq ? 1 : 0;
-    const int s = (int)((q2 - a * nq) % K);
-    const int slot = a * K + s;
-    double dr = 0, di = 0;
-    if (grp < ng) {
-        for (int64_t r = r0 + grp; r < r1; r += ng) {
-            const auto x = X[lay.at(r, slot)];
-            const double2 y = Y[r * nq2 + q2];
-            const double xr = x.x, xi = x.y;
-            dr = fma(xr, y.x, fma(xi, y.y, dr));
-            di = fma(xr, y.y, fma(-xi, y.x, di));
+k_dc_y(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ jx,
+       const typename CplxT<R>::T* __restrict__ jy, const int64_t* __restrict__ soff,
+       const int* __restrict__ sw, int64_t n_pad, const double2* __restrict__ qe, QLay ql, int K,
+       int n_en, const double* __restrict__ div, double2* __restrict__ Y) {
+    const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (m >= n_pad * K) return;
+    const int unit = ql.lay.unit();    // consecutive threads: a row's unit, then the next row
+    const int64_t g = m / (n_pad * unit), in = m - g * n_pad * unit;
+    const int64_t r = in / unit;
+    const int s = (int)(g * unit + (in - r * unit));
+    const int64_t off = soff[r >> 6] + (r & 63);
+    const int w = sw[r >> 6];
+    for (int e = blockIdx.y; e < n_en; e += gridDim.y) {
+    const double dv = div[(int64_t)e * K + s];
+    double xr = 0.0, xi = 0.0, yr = 0.0, yi = 0.0;
+    for (int j = 0; j < w; ++j) {
+        const int64_t o = off + (int64_t)j * 64;
+        const double2 v = qe[ql.at(e, cols[o], s)];
+        const auto a = jx[o];
+        const auto b = jy[o];
+        const double vr = v.x / dv, vi = v.y / dv;
+        const double ar = a.x, ai = a.y, br = b.x, bi = b.y;
+        xr = ar * vr - ai * vi + xr;
+        xi = ar * vi + ai * vr + xi;
+        yr = br * vr - bi * vi + yr;
+        yi = br * vi + bi * vr + yi;
+    }
+    Y[ql.at(e, r, s)] = make_double2(xr, xi);
+    Y[ql.at((int64_t)n_en + e, r, s)] = make_double2(yr, yi);
+    }
+}
+
+// The DC correlations of `count` <= 16 steps: for each current a, state s:
+// part[z][tile][v][j][e] = sum_{rows of split z} conj(X_j(aK + s)) Y_a(e, s),
+// a 16 x n_en product over the rows on the FP64 matrix cores (complex: four
+// v_mfma_f64_16x16x4f64 per four rows).  A wave owns one tile (current, unit
+// of VU states, 16 energies) and one split of the rows and reads both
+// operands as it multiplies: lane i + 16 k holds step i and energy i of row
+// k, neighbouring rows of a step or an energy are contiguous.  Bound by HBM:
+// Y once per 16 steps (3.8 GB at 28 energies, 8 states, 0.5M rows: 1134 us,
+// where 16 single steps on the vector ALU took 10.2 ms).
+typedef double dc_d4 __attribute__((ext_vector_type(4)));
+template <typename R, int VU>
+__global__ void __launch_bounds__(256)
+k_dcdot(DcStates xs, int count, Lay lay, int K, int64_t n_pad, const double2* __restrict__ Y,
+        QLay ql, int n_en, int64_t split, double2* __restrict__ part) {
+    using C = typename CplxT<R>::T;
+    const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
+    const int et = (n_en + 15) / 16, units = K / VU, tiles = 2 * units * et;
+    // blocks b, b + 8, ...: one XCD; the tiles of the same rows follow each
+    // other there, for they read the same lines of states and of Y
+    const int xcd = blockIdx.x % 8, b = blockIdx.x / 8, tile = b % tiles;
+    const int64_t z = (int64_t)(b / tiles * 8 + xcd) * 4 + (threadIdx.x >> 6);
+    const int a = tile / (units * et), u = tile / et % units;
+    const int e = min((tile % et) * 16 + i, n_en - 1);
+    const int64_t r0 = z * split, r1 = min(r0 + split, n_pad);
+    const C* X = reinterpret_cast<const C*>(xs.p[min(i, count - 1)]);
+    const double2* Yp = Y + ((int64_t)a * n_en + e) * ql.stride;
+    dc_d4 re[VU], im[VU];
+#pragma unroll
+    for (int v = 0; v < VU; ++v) {
+        re[v] = dc_d4{0.0, 0.0, 0.0, 0.0};
+        im[v] = dc_d4{0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll 4
+    for (int64_t rb = r0; rb < r1; rb += 4) {   // (n_pad and split: multiples of 64)
+        const int64_t r = rb + k;
+        C x[VU];
+        double2 y[VU];
+        const int64_t ix = lay.at(r, a * K + u * VU), iy = ql.lay.at(r, u * VU);
+        if constexpr (VU == 2 && sizeof(R) == 4) {
+            const float4 t = *reinterpret_cast<const float4*>(X + ix);
+            x[0] = make_float2(t.x, t.y);
+            x[1] = make_float2(t.z, t.w);
+        } else {
+#pragma unroll
+            for (int v = 0; v < VU; ++v) x[v] = X[ix + v];
+        }
+#pragma unroll
+        for (int v = 0; v < VU; ++v) y[v] = Yp[iy + v];
+#pragma unroll
+        for (int v = 0; v < VU; ++v) {
+            const double xr = x[v].x, xi = x[v].y;
+            re[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, y[v].x, re[v], 0, 0, 0);
+            im[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, y[v].y, im[v], 0, 0, 0);
+            re[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(xi, y[v].y, re[v], 0, 0, 0);
+            im[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(-xi, y[v].x, im[v], 0, 0, 0);
         }
     }
-    sh[threadIdx.x * 2 + 0] = dr;
-    sh[threadIdx.x * 2 + 1] = di;
-    __syncthreads();
-    // nqt * 2 sums (up to 512) over 256 threads
-    for (int o = threadIdx.x; o < nqt * 2; o += blockDim.x) {
-        const int qq = o / 2, k = o % 2;
-        double acc = 0.0;
-        for (int g = 0; g < ng; ++g) acc += sh[(g * nqt + qq) * 2 + k];
-        part[((int64_t)c * nq2 + qb + qq) * 2 + k] = acc;
+    // D[step][energy] sits in lane energy + 16 (step % 4), element step / 4
+    double2* out = part + (z * tiles + tile) * VU * 256;
+#pragma unroll
+    for (int v = 0; v < VU; ++v)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            out[v * 256 + (k + 4 * q) * 16 + i] = make_double2(re[v][q], im[v][q]);
+}
+
+// The splits' sums in order, step j of the block to row *counter - count +
+// 1 + j of out: out[row][a nq + e K + s].
+template <int VU>
+__global__ void __launch_bounds__(256)
+k_dcsum(const double2* __restrict__ part, int nz, int count, int K, int n_en,
+        const int* __restrict__ counter, double2* __restrict__ out) {
+    const int et = (n_en + 15) / 16, units = K / VU;
+    const int tile = blockIdx.x, v = blockIdx.y, o = threadIdx.x, j = o >> 4;
+    const int a = tile / (units * et), u = tile / et % units, e = (tile % et) * 16 + (o & 15);
+    if (j >= count || e >= n_en) return;
+    double2 t = make_double2(0.0, 0.0);
+    for (int z = 0; z < nz; ++z) {
+        const double2 p = part[(((int64_t)z * gridDim.x + tile) * VU + v) * 256 + o];
+        t.x += p.x;
+        t.y += p.y;
     }
+    const int64_t nq = (int64_t)n_en * K;
+    out[(int64_t)(*counter - count + 1 + j) * 2 * nq + a * nq + (int64_t)e * K + u * VU + v] = t;
 }
 
 // Dynamic polarisation, per sample s: slots s (psi1), K+s (psi2):
@@ -623,44 +690,54 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     launch_pack<R>(psi0, K, n, psi.p, e.lay, 0, H->perm_ptr(), st);
     launch_pack<R>(psi0, K, n, e.X.p, e.lay, 0, H->perm_ptr(), st);
     launch_pack<R>(psi0, K, n, e.X.p, e.lay, K, H->perm_ptr(), st);
+    // the kept states leave room for the quasi-eigenstates, Y and the sums
+    if (nq > 0) {
+        size_t room = 0, total = 0;
+        TBG_HIP(hipMemGetInfo(&room, &total));
+        const size_t rest = (size_t)n_pad * nq * 3 * sizeof(double2) + ((size_t)1 << 29);
+        e.keep_history(T, room > rest ? (room - rest) / 2 : 0);
+    }
+    const QLay ql = q_layout(e.lay, K, n_pad);
     uint64_t bwd = 0;
     for (int k = K; k < 2 * K; ++k) bwd |= 1ull << k;
+    const unsigned nbm = nblk(n_pad * K), ny = (unsigned)std::min(n_en, 32768),
+                   nyq = (unsigned)std::min<int64_t>(nq, 32768);
+    // energies a thread of k_qe keeps, in even chunks
+    const int chunks = std::max((n_en + 15) / 16, 1), even = (n_en + chunks - 1) / chunks;
+    const int ec = even <= 2 ? 2 : even <= 8 ? 8 : 16;
+    const int nec = (n_en + ec - 1) / ec, pitch = nec * ec;
     DevBuf qe((size_t)std::max<int64_t>(n_pad * nq, 1) * sizeof(double2));
     if (nq > 0)
-        hipLaunchKernelGGL(k_qe_init, dim3(nblk(n_pad * nq)), dim3(256), 0, st,
-                           reinterpret_cast<const double2*>(psi0), n, K, n_en, n_pad,
-                           H->perm_ptr(), qe.as<double2>());
-    // Phase tables P(t, e) = exp(i E t dt), W(t) = Hanning (tbpm.f90:625-629).
-    std::vector<double> ptab((size_t)T * std::max(n_en, 1) * 2), wtab(T);
+        hipLaunchKernelGGL(k_qe_init, dim3(nbm, ny), dim3(256), 0, st,
+                           reinterpret_cast<const double2*>(psi0), n, K, n_pad, H->perm_ptr(), ql,
+                           n_en, qe.as<double2>());
+    // W(t) P(t, e): phases exp(i E t dt) and the Hanning window
+    // (tbpm.f90:625-629).
+    std::vector<double> ptab((size_t)T * std::max(pitch, 1) * 2, 0.0);
     const double pi = 3.14159265358979323846;
     for (int t = 1; t <= T; ++t) {
-        wtab[t - 1] = 0.5 * (1 + std::cos(pi * t / T));
+        const double W = 0.5 * (1 + std::cos(pi * t / T));
         for (int i = 0; i < n_en; ++i) {
             const double th = energies[en_inds[i]] * t * t_step;
-            ptab[((size_t)(t - 1) * n_en + i) * 2 + 0] = std::cos(th);
-            ptab[((size_t)(t - 1) * n_en + i) * 2 + 1] = std::sin(th);
+            ptab[((size_t)(t - 1) * pitch + i) * 2 + 0] = W * std::cos(th);
+            ptab[((size_t)(t - 1) * pitch + i) * 2 + 1] = W * std::sin(th);
         }
     }
-    DevBuf dptab(ptab.size() * sizeof(double)), dwtab(wtab.size() * sizeof(double));
+    DevBuf dptab(ptab.size() * sizeof(double));
     TBG_HIP(hipMemcpyAsync(dptab.p, ptab.data(), ptab.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    TBG_HIP(hipMemcpyAsync(dwtab.p, wtab.data(), wtab.size() * sizeof(double), hipMemcpyHostToDevice, st));
     const int nvn = 3 * Kp;
     DevBuf nbuf((size_t)(T + 1) * nvn * sizeof(double));
-    DevBuf dbuf((size_t)T * 2 * K * sizeof(double));
     DevBuf counter(sizeof(int));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
     launch_dotnorm<R>(e.plan, e.X.p, e.X.p, e.lay, Kp, e.part.template as<double>(), st);
     launch_reduce(e.part.template as<double>(), nvn, e.plan.inst_chunk_dev.template as<int>(), 1,
                   nbuf.as<double>(), 0, counter.as<int>(), 0, st);
     const StepPoly sp = time_poly(bes, nb);
+    std::vector<double> hn((size_t)(T + 1) * nvn);   // <psi0|psi(t)> and |psi(t)|^2 per slot
     // Check at t == chk_step on psi(+-) after chk_step-1 steps vs <psi0|psi0>
     // (tbpm.f90:608-611, 772-775).
     auto check_norms = [&]() {
         if (chk_step < 1 || chk_step > T) return;
-        std::vector<double> hn((size_t)(T + 1) * nvn);
-        TBG_HIP(hipMemcpyAsync(hn.data(), nbuf.p, hn.size() * sizeof(double),
-                               hipMemcpyDeviceToHost, st));
-        TBG_HIP(hipStreamSynchronize(st));
         for (int k = 0; k < 2 * K; ++k) {
             const double ref = hn[k * 3 + 2];
             const double nn = hn[(size_t)(chk_step - 1) * nvn + k * 3 + 2];
@@ -673,70 +750,84 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
             }
         }
     };
+    // the states of the last `count` of the `done` steps enqueued or captured
+    // (whole rounds of the buffers), the run's input being state `base`
+    int done = 0, base = 0;
+    auto kept = [&](int count) {
+        DcStates xs;
+        for (int j = 0; j < kDcSteps; ++j)
+            xs.p[j] = e.history(base + done - count + 1 + std::min(j, count - 1));
+        return xs;
+    };
+    auto qe_update = [&](int count) {
+        const DcStates xs = kept(count);
+#define TBG_QE(LIN, EC)                                                                     \
+    hipLaunchKernelGGL((k_qe<R, LIN, EC>), dim3(nbm, (unsigned)nec),                         \
+                       dim3(256), 0, st, xs, count, e.lay, K, n_pad, ql, qe.as<double2>(),   \
+                       n_en, pitch, dptab.as<double2>(), counter.as<int>())
+        timed_launch(h, kTimeQe, [&] {
+            if (ql.lin) {
+                if (ec == 2) TBG_QE(true, 2);
+                else if (ec == 8) TBG_QE(true, 8);
+                else TBG_QE(true, 16);
+            } else {
+                if (ec == 2) TBG_QE(false, 2);
+                else if (ec == 8) TBG_QE(false, 8);
+                else TBG_QE(false, 16);
+            }
+            TBG_HIP(hipGetLastError());
+        });
+#undef TBG_QE
+    };
     auto after1 = [&]() {
         launch_reduce(e.part.template as<double>(), nvn, e.epi_range(), 1, nbuf.as<double>(), 0,
                       counter.as<int>(), 0, st);
-        timed_launch(h, kTimeQe, [&] {
-            hipLaunchKernelGGL(k_qe<R>, dim3(e.plan.nchunks), dim3(256), 0, st,
-                               e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay, K,
-                               psi.as<C>(), qe.as<double2>(), n_en, dptab.as<double2>(),
-                               dwtab.as<double>(), counter.as<int>(),
-                               e.part.template as<double>());
-        });
-        launch_reduce(e.part.template as<double>(), 2 * K, e.plan.inst_chunk_dev.template as<int>(),
-                      1, dbuf.as<double>(), 0, counter.as<int>(), -1, st);
+        ++done;
+        if (nq > 0 && done % e.hist() == 0) qe_update(e.hist());
     };
-    e.run(T, sp, bwd, 0, F_NORM, nullptr, counter.as<int>(), after1);
-    // Normalise the quasi-eigenstates (tbpm.f90:642-647) and form
-    // a = |<psi0|QE>| on the normalised states (tbpm.f90:667).
-    std::vector<double> adiv(std::max<int64_t>(nq, 1));
-    DevBuf dadiv(adiv.size() * sizeof(double));
+    e.run(T, sp, bwd, 0, F_DOT | F_NORM, psi.p, counter.as<int>(), after1);
+    if (nq > 0 && done % e.hist() != 0) qe_update(done % e.hist());
+    TBG_HIP(hipMemcpyAsync(hn.data(), nbuf.p, hn.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    // |QE| and a = |<psi0|QE>| (tbpm.f90:642-647, 667): the currents act on
+    // QE / |QE| / (a / |QE|) = QE / a.
+    std::vector<double> div(std::max<int64_t>(nq, 1));
+    DevBuf ddiv(div.size() * sizeof(double));
     if (nq > 0) {
-        const int64_t ntiles = (nq + 255) / 256;
         DevBuf qpart((size_t)e.plan.nchunks * nq * 3 * sizeof(double));
         DevBuf qsum((size_t)nq * 3 * sizeof(double));
         std::vector<double> hs((size_t)nq * 3);
-        for (int pass = 0; pass < 2; ++pass) {
-            hipLaunchKernelGGL(k_qe_stats, dim3(e.plan.nchunks, (unsigned)ntiles), dim3(256), 0, st,
-                               e.plan.chunk.template as<int64_t>(), qe.as<double2>(), nq, K,
-                               reinterpret_cast<const double2*>(psi0), n, H->perm_ptr(),
-                               qpart.as<double>());
+        hipLaunchKernelGGL(k_qe_stats, dim3(e.plan.nchunks, nyq), dim3(256), 0, st,
+                           e.plan.chunk.template as<int64_t>(), qe.as<double2>(), ql, nq, K,
+                           reinterpret_cast<const double2*>(psi0), n, H->perm_ptr(),
+                           qpart.as<double>());
+        TBG_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_sum_rows, dim3(nblk(nq * 3)), dim3(256), 0, st, qpart.as<double>(),
+                           e.plan.nchunks, nq * 3, qsum.as<double>());
+        TBG_HIP(hipGetLastError());
+        TBG_HIP(hipMemcpyAsync(hs.data(), qsum.p, hs.size() * sizeof(double),
+                               hipMemcpyDeviceToHost, st));
+        TBG_HIP(hipStreamSynchronize(st));
+        for (int64_t q = 0; q < nq; ++q)
+            div[q] = qe_abs2 != nullptr ? std::sqrt(hs[q * 3 + 2])
+                                        : std::hypot(hs[q * 3 + 0], hs[q * 3 + 1]);
+        TBG_HIP(hipMemcpyAsync(ddiv.p, div.data(), nq * sizeof(double), hipMemcpyHostToDevice, st));
+        if (qe_abs2 != nullptr) {   // quasi-eigenstates: done after normalising
+            hipLaunchKernelGGL(k_qe_abs2, dim3(nblk(n), nyq), dim3(256), 0, st,
+                               qe.as<double2>(), ql, n, K, n_en, ddiv.as<double>(),
+                               H->perm_ptr(), qe_abs2);
             TBG_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_sum_rows, dim3(nblk(nq * 3)), dim3(256), 0, st, qpart.as<double>(),
-                               e.plan.nchunks, nq * 3, qsum.as<double>());
-            TBG_HIP(hipGetLastError());
-            TBG_HIP(hipMemcpyAsync(hs.data(), qsum.p, hs.size() * sizeof(double),
-                                   hipMemcpyDeviceToHost, st));
             TBG_HIP(hipStreamSynchronize(st));
-            if (pass == 0) {
-                for (int64_t q = 0; q < nq; ++q) adiv[q] = std::sqrt(hs[q * 3 + 2]);
-                TBG_HIP(hipMemcpyAsync(dadiv.p, adiv.data(), nq * sizeof(double),
-                                       hipMemcpyHostToDevice, st));
-                hipLaunchKernelGGL(k_qe_scale, dim3(nblk(n_pad * nq)), dim3(256), 0, st,
-                                   qe.as<double2>(), n_pad * nq, nq, dadiv.as<double>());
-                TBG_HIP(hipGetLastError());
-                if (qe_abs2 != nullptr) {   // quasi-eigenstates: done after normalising
-                    hipLaunchKernelGGL(k_qe_abs2, dim3(nblk(n * nq)), dim3(256), 0, st,
-                                       qe.as<double2>(), n, K, n_en, H->perm_ptr(), qe_abs2);
-                    TBG_HIP(hipGetLastError());
-                    TBG_HIP(hipStreamSynchronize(st));
-                    check_norms();
-                    return;
-                }
-            } else {
-                for (int64_t q = 0; q < nq; ++q) adiv[q] = std::hypot(hs[q * 3 + 0], hs[q * 3 + 1]);
-                TBG_HIP(hipMemcpyAsync(dadiv.p, adiv.data(), nq * sizeof(double),
-                                       hipMemcpyHostToDevice, st));
-            }
+            check_norms();
+            return;
         }
     }
     // Y_a = J_a (QE / a), time independent.
     DevBuf Y((size_t)std::max<int64_t>(n_pad * 2 * nq, 1) * sizeof(double2));
     if (nq > 0) {
-        hipLaunchKernelGGL(k_dc_y<R>, dim3(nblk(n_pad * 2 * nq)), dim3(256), 0, st,
-                           H->cols.as<int>(), H->jx.as<C>(), H->jy.as<C>(),
-                           H->slice_off.as<int64_t>(), H->slice_w.as<int>(), n_pad,
-                           qe.as<double2>(), nq, dadiv.as<double>(), Y.as<double2>());
+        hipLaunchKernelGGL(k_dc_y<R>, dim3(nbm, ny), dim3(256), 0, st, H->cols.as<int>(),
+                           H->jx.as<C>(), H->jy.as<C>(), H->slice_off.as<int64_t>(),
+                           H->slice_w.as<int>(), n_pad, qe.as<double2>(), ql, K, n_en,
+                           ddiv.as<double>(), Y.as<double2>());
         TBG_HIP(hipGetLastError());
     }
     qe.release();
@@ -747,23 +838,53 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     launch_spmv<R>(H, H->jy.p, psi.p, e.lay, 0, e.X.p, e.lay, K, K, st);
     const int64_t nq2 = 2 * nq;
     DevBuf cbuf((size_t)std::max<int64_t>(T * nq2 * 2, 1) * sizeof(double));
-    DevBuf cpart((size_t)std::max<int64_t>((int64_t)e.plan.nchunks * nq2 * 2, 1) * sizeof(double));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-    const int64_t ntiles2 = (nq2 + 255) / 256;
-    auto after2 = [&]() {
-        if (nq2 == 0) return;
+    // splits of the rows: about 16 waves a compute unit over all tiles
+    const bool pairs = sizeof(R) == 4 && ql.lin && ql.lay.sh == 1;
+    const int VU = pairs ? 2 : 1;
+    const int tiles = 2 * (K / VU) * ((n_en + 15) / 16);
+    int64_t split = 0, nz = 0;
+    DevBuf dpart;
+    if (nq2 > 0) {
+        const int64_t want = (16 * (int64_t)h->num_cus / tiles + 31) / 32 * 32;
+        split = std::max<int64_t>(64, ((n_pad + want - 1) / want + 63) / 64 * 64);
+        nz = ((n_pad + split - 1) / split + 31) / 32 * 32;   // 4 waves a block, 8 XCDs
+        dpart.alloc((size_t)nz * tiles * VU * 256 * sizeof(double2));
+    }
+    auto correlate = [&](int count) {
+        const DcStates xs = kept(count);
         timed_launch(h, kTimeDcDot, [&] {
-            hipLaunchKernelGGL(k_dcdot<R>, dim3(e.plan.nchunks, (unsigned)ntiles2), dim3(256), 0,
-                               st, e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay,
-                               K, Y.as<double2>(), nq2, nq, cpart.as<double>());
+            const dim3 grid((unsigned)(nz / 4 * tiles));
+            if (pairs) {
+                if constexpr (sizeof(R) == 4)
+                    hipLaunchKernelGGL((k_dcdot<R, 2>), grid, dim3(256), 0, st, xs, count, e.lay,
+                                       K, n_pad, Y.as<double2>(), ql, n_en, split,
+                                       dpart.as<double2>());
+            } else {
+                hipLaunchKernelGGL((k_dcdot<R, 1>), grid, dim3(256), 0, st, xs, count, e.lay, K,
+                                   n_pad, Y.as<double2>(), ql, n_en, split, dpart.as<double2>());
+            }
+            TBG_HIP(hipGetLastError());
         });
-        launch_reduce(cpart.as<double>(), (int)(nq2 * 2), e.plan.inst_chunk_dev.template as<int>(),
-                      1, cbuf.as<double>(), 0, counter.as<int>(), 0, st);
+        const dim3 grid((unsigned)tiles, VU);
+        if (pairs)
+            hipLaunchKernelGGL(k_dcsum<2>, grid, dim3(256), 0, st, dpart.as<double2>(), (int)nz,
+                               count, K, n_en, counter.as<int>(), cbuf.as<double2>());
+        else
+            hipLaunchKernelGGL(k_dcsum<1>, grid, dim3(256), 0, st, dpart.as<double2>(), (int)nz,
+                               count, K, n_en, counter.as<int>(), cbuf.as<double2>());
+        TBG_HIP(hipGetLastError());
     };
-    after2();  // t = 1, unpropagated
+    base = e.cur;
+    done = 0;
+    if (nq2 > 0) correlate(1);   // t = 1, unpropagated
+    auto after2 = [&]() {
+        ++done;
+        if (nq2 > 0 && done % e.hist() == 0) correlate(e.hist());
+    };
     if (T >= 2) e.run(T - 1, sp, 0, 0, 0, nullptr, counter.as<int>(), after2);
-    std::vector<double> hd((size_t)T * 2 * K), hc((size_t)T * nq2 * 2);
-    TBG_HIP(hipMemcpyAsync(hd.data(), dbuf.p, hd.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    if (nq2 > 0 && done % e.hist() != 0) correlate(done % e.hist());
+    std::vector<double> hc((size_t)T * nq2 * 2);
     if (nq2 > 0)
         TBG_HIP(hipMemcpyAsync(hc.data(), cbuf.p, hc.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     TBG_HIP(hipStreamSynchronize(st));
@@ -771,7 +892,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     for (int s = 0; s < K; ++s)
         for (int t = 0; t < T; ++t)
             for (int ri = 0; ri < 2; ++ri)
-                od[((size_t)s * T + t) * 2 + ri] = hd[(size_t)t * 2 * K + s * 2 + ri];
+                od[((size_t)s * T + t) * 2 + ri] = hn[(size_t)(t + 1) * nvn + s * 3 + ri];
     for (int s = 0; s < K; ++s)
         for (int a = 0; a < 2; ++a)
             for (int i = 0; i < n_en; ++i)

@@ -261,7 +261,7 @@ struct Engine {
         void* b0 = P.p;
         void* b1 = Q.p;
         void* b2 = S.p;
-        void* b3 = X.p;
+        void* b3 = free0();
         pass(PM_M1, T, 1, nullptr, X.p, b0, b1);
         int m = T + 1;
         const int rem = N - m;   // terms m .. N-1, at least one (N >= T + 2)
@@ -360,7 +360,7 @@ struct Engine {
                 b0 = P.p;
                 b1 = Q.p;
                 b2 = S.p;
-                b3 = X.p;
+                b3 = free0();
             } else {
                 std::swap(b0, b2);
                 std::swap(b1, b3);
@@ -371,8 +371,62 @@ struct Engine {
         parity ^= 1;
     }
 
+    // Keeps the outputs of the last hist() steps: the state `k` steps after
+    // the call lies in buffer k % hist() until hist() steps later.  Buffers of
+    // their own, as many as fit in `room` bytes: 16 at most (the steps of a
+    // captured graph, which then holds whole rounds of them), no more than
+    // `steps` need, or none: then only the last output is there.
+    std::vector<DevBuf> slot;
+    DevBuf spare;   // the recurrence buffer that X is where nothing is kept
+    int cur = 0;
+    int hist() const { return slot.empty() ? 1 : (int)slot.size(); }
+    void keep_history(int steps, size_t room) {
+        const bool need_spare = !(ring && S.p == nullptr);   // two passes leave X as it is
+        int want = 16;
+        while (want > 1 && want / 2 >= steps) want /= 2;
+        for (; want >= 2; want /= 2) {
+            if ((size_t)(want - 2 + need_spare) * vbytes > room) continue;
+            try {
+                slot.resize((size_t)want);
+                for (int i = 2; i < want; ++i) {   // X and Y are the other two
+                    slot[i].alloc(vbytes);
+                    launch_fill_zero(slot[i].p, vbytes, h->stream);
+                }
+                if (need_spare) {
+                    spare.alloc(vbytes);
+                    launch_fill_zero(spare.p, vbytes, h->stream);
+                }
+                std::swap(slot[1], Y);
+                cur = 0;
+                return;
+            } catch (const Error& e) {
+                slot.clear();
+                if (e.code != TBG_EOOM) throw;
+            }
+        }
+    }
+    const void* history(int k) const {
+        const int i = k % hist();
+        return slot.empty() || i == cur ? X.p : slot[i].p;
+    }
+    // v_0's buffer once the recurrence has passed it
+    void* free0() const { return slot.empty() ? X.p : spare.p; }
+
     // One step: X holds the input, the result is left in X (buffers swap).
     void step(const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi, const void* psi0,
+              int* counter) {
+        if (slot.empty()) {
+            step_once(sp, bwd, cls, epi, psi0, counter);
+            return;
+        }
+        const int next = (cur + 1) % (int)slot.size();
+        std::swap(Y, slot[next]);
+        step_once(sp, bwd, cls, epi, psi0, counter);
+        std::swap(Y, slot[cur]);
+        cur = next;
+    }
+
+    void step_once(const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi, const void* psi0,
               int* counter) {
         const int N = sp.N;
         TBG_REQUIRE(N >= 3, "at least 3 expansion terms are required");
@@ -384,7 +438,7 @@ struct Engine {
             step_blocked(sp, bwd, cls, epi, psi0, counter);
             return;
         }
-        auto buf = [&](int j) { return (j % 2 == 0) ? X.p : P.p; };
+        auto buf = [&](int j) { return j == 0 ? X.p : j % 2 == 0 ? free0() : P.p; };
         for (int m = 1; m < N; ++m) {
             TermArgs a = base_args(bwd, cls);
             a.acc = Y.p;
@@ -489,7 +543,8 @@ struct Engine {
              const void* psi0, int* counter, F&& after) {
         int done = 0;
         if (h->use_graph && !h->timing) {
-            const int per = std::min(16, nsteps & ~1);
+            // (with kept outputs a graph holds whole rounds of their buffers)
+            const int per = slot.empty() ? std::min(16, nsteps & ~1) : nsteps >= 16 ? 16 : 0;
             if (graph_steps == 0 && per >= 2) capture(per, sp, bwd, cls, epi, psi0, counter, after);
             if (graph_steps > 0 && parity != graph_parity && nsteps > 0) {
                 // one launched step restores the buffer roles of the graph

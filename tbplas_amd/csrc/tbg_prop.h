@@ -15,7 +15,7 @@ struct Lay {
     Lay(int K_) : K(K_) {}
     Lay(int K_, int sh_, int64_t plane_) : K(K_), sh(sh_), plane(plane_) {}
     // complex elements from one row to the next
-    int unit() const { return sh < 0 ? K : 1 << sh; }
+    __host__ __device__ int unit() const { return sh < 0 ? K : 1 << sh; }
     __host__ __device__ __forceinline__ int64_t at(int64_t r, int k) const {
         return sh < 0 ? r * K + k : (int64_t)(k >> sh) * plane + (r << sh) + (k & ((1 << sh) - 1));
     }

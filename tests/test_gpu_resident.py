@@ -194,3 +194,37 @@ def test_graph_replay_and_timing(handle):
     with pytest.raises(tb._lib.NormError):
         tbpm.corr_dos(H, bes, psi, 20, chk_step=10, chk_thr=1e-30)
     H.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-10), ("fp32", 2e-4)])
+@pytest.mark.parametrize("resident", [True, False])
+@pytest.mark.parametrize("T,n_en,K", [(1, 1, 1), (2, 3, 2), (7, 16, 3), (16, 2, 4), (17, 17, 2),
+                                      (33, 9, 5), (50, 33, 1)])
+def test_dc_step_blocks_vs_oracle(handle, prec, tol, resident, T, n_en, K):
+    """The quasi-eigenstates and the DC correlations are summed over blocks
+    of up to 16 kept steps: block lengths and remainders, energies around the
+    16 of a tile, states in planes and row by row.  Tolerances as in the
+    other comparisons of corr_dc with the oracle; the chosen energies keep
+    |<psi0|QE>| away from zero in both."""
+    s, _ = _sample(9, 14)
+    ip, ix, hop, dx, dy = oracle.build_ham_dxy_loop(s.orb_eng, s.hop_i, s.hop_j, s.hop_v, s.dr)
+    bes = tbpm.bessel_series(tau_of(s), 1e-14)
+    psi = _states(s.num_orb, K)
+    t_step = 2 * math.pi / 18.0
+    en = np.linspace(-2.6, 2.6, 64)
+    inds = np.unique(np.linspace(3, 60, n_en).astype(int))
+    assert len(inds) == n_en
+    handle.set_blocking(False)
+    handle.set_resident(resident)
+    order, tiles = s.tile_order(1.3, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, hop, dx, dy, cur_scale=9.0, precision=prec,
+                         handle=handle, order=order if resident else None,
+                         tiles=tiles if resident else None)
+    d, c = tbpm.corr_dc(H, bes, psi, T, t_step, en, inds)
+    rd, rc = oracle.orc_tbpm_dccond(ip, ix, hop, dx, dy, 9.0, bes, psi, T, t_step, en, inds)
+    assert np.max(np.abs(d - rd)) < tol
+    assert np.max(np.abs(c - rc)) < tol * max(1.0, np.max(np.abs(rc)))
+    g = tbpm.quasi_eigenstates(H, bes, psi, T, t_step, list(en[inds]))
+    r = oracle.orc_quasi_eigenstates(ip, ix, hop, bes, psi, T, t_step, list(en[inds]))
+    assert np.max(np.abs(g - r)) < tol * max(1.0, np.max(r))
+    H.close()
