@@ -327,6 +327,12 @@ int tbg_haydock_coef(tbg_handle *h, const tbg_ham *H, const double *psi0,
 int tbg_hall_mu(tbg_handle *h, const tbg_ham *H, const double *psi0, int K,
                 int n_kernel, int direction, double *mu);
 
+/* tbg_hall_mu with each state in row-major order (element (i, j) at
+ * s*N*N + i*N + j), the order of the Python arrays: transposing 2048^2
+ * moments on the host took longer than computing them. */
+int tbg_hall_mu_rows(tbg_handle *h, const tbg_ham *H, const double *psi0, int K,
+                     int n_kernel, int direction, double *mu);
+
 /* Replaces f2py tbpm_eigenstates (tbplas/fortran/tbpm.f90:721-830; called
  * from tbplas/tbpm/solver.py:472-505).  energies: host, n_en energies (eV,
  * with t_step in hbar/eV as for tbg_corr_dc).  qe: device float64

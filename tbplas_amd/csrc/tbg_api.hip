@@ -1058,8 +1058,8 @@ int tbg_haydock_coef(tbg_handle* h, const tbg_ham* H, const double* psi0, int K,
     });
 }
 
-int tbg_hall_mu(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int n_kernel,
-                int direction, double* mu) {
+static int hall_mu(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int n_kernel,
+                   int direction, bool rows_first, double* mu) {
     return guard([&] {
         check_handle(h);
         check_psi_args(H, psi0, K, 1);
@@ -1067,8 +1067,18 @@ int tbg_hall_mu(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int 
         TBG_REQUIRE(H->precision == TBG_FP64, "the Hall moments need a complex128 Hamiltonian");
         TBG_REQUIRE(n_kernel >= 1 && mu != nullptr, "need n_kernel >= 1 and an output");
         TBG_REQUIRE(direction == 1 || direction == 2, "direction must be 1 (xx) or 2 (xy)");
-        hall_mu_impl(h, H, psi0, K, n_kernel, direction, mu);
+        hall_mu_impl(h, H, psi0, K, n_kernel, direction, rows_first, mu);
     });
+}
+
+int tbg_hall_mu(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int n_kernel,
+                int direction, double* mu) {
+    return hall_mu(h, H, psi0, K, n_kernel, direction, false, mu);
+}
+
+int tbg_hall_mu_rows(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int n_kernel,
+                     int direction, double* mu) {
+    return hall_mu(h, H, psi0, K, n_kernel, direction, true, mu);
 }
 
 int tbg_quasi_eigenstates(tbg_handle* h, const tbg_ham* H, const double* bes, int n_bes,

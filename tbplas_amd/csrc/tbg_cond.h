@@ -32,7 +32,7 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
 void haydock_impl(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int depth,
                   double rescale, double* coefa, double* coefb);
 void hall_mu_impl(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, int N, int dir,
-                  double* mu);
+                  bool rows_first, double* mu);
 
 template <typename R>
 void dyn_pol_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, const double* cF,

@@ -334,10 +334,9 @@ def hall_mu(H, psi0, n_kernel, direction=1):
     if n != H.n:
         raise ValueError("state length does not match the Hamiltonian")
     out = torch.empty((K, n_kernel, n_kernel), dtype=torch.complex128, device=f"cuda:{dv}")
-    _lib.check(_lib.lib().tbg_hall_mu(H.handle.ptr, H.ptr, _lib.ptr(p), K, int(n_kernel),
-                                      int(direction), _lib.ptr(out)))
-    # each state is column-major (i + j N): the array read row-major is [s, j, i]
-    return out.cpu().numpy().transpose(0, 2, 1).copy()
+    _lib.check(_lib.lib().tbg_hall_mu_rows(H.handle.ptr, H.ptr, _lib.ptr(p), K, int(n_kernel),
+                                           int(direction), _lib.ptr(out)))
+    return out.cpu().numpy()
 
 
 def quasi_eigenstates(H, bes, psi0, n_timestep, t_step, energies, chk_step=128, chk_thr=1e-9):
