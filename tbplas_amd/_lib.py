@@ -258,6 +258,15 @@ def dev(a, dtype=None, device=0):
     return torch.from_numpy(a).to(f"cuda:{device}")
 
 
+def host(t):
+    """numpy copy of a device tensor.  NumPy advises huge pages for its large
+    arrays and torch does not: 64 MB arrive in 6.7 ms instead of 16 ms, most
+    of which were the page faults of the destination."""
+    torch = torch_cuda()
+    out = torch.from_numpy(np.empty(t.shape, dtype=str(t.dtype)[6:]))
+    return out.copy_(t).numpy()
+
+
 def ptr(t):
     return ctypes.c_void_p(t.data_ptr() if t is not None and t.numel() > 0 else 0)
 

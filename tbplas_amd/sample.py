@@ -349,7 +349,7 @@ class Sample:
         """
         if algo not in ("fast", "safe"):
             raise ValueError(f"unknown algo {algo}")
-        out = [t.cpu().numpy() for t in self.build_ham_dxy_device(orb_eng_cutoff)]
+        out = [_lib.host(t) for t in self.build_ham_dxy_device(orb_eng_cutoff)]
         if sort_col:
             indptr, indices, hop, dx, dy = out
             for r in range(len(indptr) - 1):

@@ -219,7 +219,7 @@ def corr_dos(H, bes, psi0, n_timestep, chk_step=128, chk_thr=1e-9):
                                  K, int(n_timestep), int(chk_step), float(chk_thr),
                                  _lib.ptr(out), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def ldos_states(psi, site_indices):
@@ -248,7 +248,7 @@ def corr_ldos(H, bes, psi0, n_timestep, chk_step=128, chk_thr=1e-9):
                                   K, int(n_timestep), int(chk_step), float(chk_thr),
                                   _lib.ptr(out), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def psi_t(H, bes, psi0, time_log, n_timestep, chk_step=128, chk_thr=1e-9):
@@ -268,7 +268,7 @@ def psi_t(H, bes, psi0, time_log, n_timestep, chk_step=128, chk_thr=1e-9):
                               tl.ctypes.data, len(tl), int(n_timestep), int(chk_step),
                               float(chk_thr), _lib.ptr(out), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def corr_dyn_pol(H, bes, coef_F, coef_omF, psi0, n_timestep, q_points, orb_pos,
@@ -296,7 +296,7 @@ def corr_dyn_pol(H, bes, coef_F, coef_omF, psi0, n_timestep, q_points, orb_pos,
                                      pos.ctypes.data, int(chk_step), float(chk_thr),
                                      _lib.ptr(out), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def haydock_coef(H, psi0, depth, rescale):
@@ -336,7 +336,7 @@ def hall_mu(H, psi0, n_kernel, direction=1):
     out = torch.empty((K, n_kernel, n_kernel), dtype=torch.complex128, device=f"cuda:{dv}")
     _lib.check(_lib.lib().tbg_hall_mu_rows(H.handle.ptr, H.ptr, _lib.ptr(p), K, int(n_kernel),
                                            int(direction), _lib.ptr(out)))
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def quasi_eigenstates(H, bes, psi0, n_timestep, t_step, energies, chk_step=128, chk_thr=1e-9):
@@ -357,7 +357,7 @@ def quasi_eigenstates(H, bes, psi0, n_timestep, t_step, energies, chk_step=128, 
                                           en.ctypes.data, len(en), int(chk_step),
                                           float(chk_thr), _lib.ptr(out), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def corr_dos_batch(hams, bes, psi0_list, n_timestep, chk_step=128, chk_thr=1e-9):
@@ -386,7 +386,7 @@ def corr_dos_batch(hams, bes, psi0_list, n_timestep, chk_step=128, chk_thr=1e-9)
                                        int(n_timestep), int(chk_step), float(chk_thr), oarr,
                                        ctypes.byref(fi), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return [o.cpu().numpy() for o in outs]
+    return [_lib.host(o) for o in outs]
 
 
 class DosRun:
@@ -453,7 +453,7 @@ class DosRun:
         rc = _lib.lib().tbg_dos_end(self._r, int(chk_step), float(chk_thr), oarr,
                                     ctypes.byref(fi), ctypes.byref(fs))
         _lib.check(rc, fs)
-        res = [o.cpu().numpy() for o in outs]
+        res = [_lib.host(o) for o in outs]
         return res if len(res) > 1 else res[0]
 
     def close(self):
@@ -483,7 +483,7 @@ def corr_ac(H, bes, coef_F, coef_omF, psi0, n_timestep, chk_step=128, chk_thr=1e
                                 int(n_timestep), int(chk_step), float(chk_thr), _lib.ptr(out),
                                 ctypes.byref(fs))
     _lib.check(rc, fs)
-    return out.cpu().numpy()
+    return _lib.host(out)
 
 
 def corr_dc(H, bes, psi0, n_timestep, t_step, energies, en_inds, chk_step=128,
@@ -506,7 +506,7 @@ def corr_dc(H, bes, psi0, n_timestep, t_step, energies, en_inds, chk_step=128,
                                 en_inds.ctypes.data, n_en, int(chk_step), float(chk_thr),
                                 _lib.ptr(dos), _lib.ptr(dc), ctypes.byref(fs))
     _lib.check(rc, fs)
-    return dos.cpu().numpy(), dc.cpu().numpy()[:, :, :n_en, :]
+    return _lib.host(dos), _lib.host(dc)[:, :, :n_en, :]
 
 
 def cheb_step(H, bes, psi, fwd=True):
@@ -516,7 +516,7 @@ def cheb_step(H, bes, psi, fwd=True):
     bes = np.ascontiguousarray(bes, dtype=np.float64)
     _lib.check(_lib.lib().tbg_cheb_step(H.handle.ptr, H.ptr, bes.ctypes.data, len(bes),
                                         _lib.ptr(p), K, 1 if fwd else 0))
-    return p.cpu().numpy()
+    return _lib.host(p)
 
 
 def cheb_poly(H, coef, psi):
@@ -526,4 +526,4 @@ def cheb_poly(H, coef, psi):
     coef = np.ascontiguousarray(coef, dtype=np.float64)
     _lib.check(_lib.lib().tbg_cheb_poly(H.handle.ptr, H.ptr, coef.ctypes.data, len(coef),
                                         _lib.ptr(p), K))
-    return p.cpu().numpy()
+    return _lib.host(p)
