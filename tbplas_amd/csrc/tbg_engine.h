@@ -309,7 +309,6 @@ struct Engine {
         a.plane = lay.plane;
         a.depth = ring->depth;
         a.groups = Kp / ring_v;
-        a.lds_rows = ring->rows_max;
         // the two recurrences there are: time steps (alpha = -2i, beta = 1)
         // and Chebyshev polynomials (2, -1), which run as u_m = (-i)^m T_m
         const bool time = sp.ar == 0.0 && sp.ar1 == 0.0 && sp.ai == -2.0 && sp.ai1 == -1.0 &&

@@ -14,6 +14,9 @@ namespace tbg {
 constexpr int kRingMax = 32;      // terms of one resident pass at most
 constexpr int kRingLanes = 512;   // lanes of a workgroup (two on a compute unit:
 constexpr int kRingPerCu = 2;     // 128 registers a lane)
+// byte offset beyond every plane, which has less than kRingPlane bytes
+constexpr unsigned kRingNowhere = 0xffffff00u;
+constexpr uint64_t kRingPlane = 0xfffffe00u;
 
 // Rows per lane of a resident pass: a lane keeps v_{m-2}, the table (two
 // words of positions and the values) and, of its owned rows, the output in
@@ -88,7 +91,6 @@ struct RingArgs {
     void* acc;               // step output
     int64_t plane;           // complex elements of one group's states
     int depth, T, groups, first;
-    int lds_rows;
     // v_m = i ai H v_{m-1} + v_{m-2}: of the first term and of the others,
     // forward and backward.  exp(-i H tau): ai = -1, -2.  Chebyshev
     // polynomials T_m run as u_m = (-i)^m T_m, which obey the same

@@ -183,6 +183,8 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
                                  const std::vector<std::vector<int64_t>>& segs, int real_bytes,
                                  int V, int groups, int terms, bool real_vals) {
     const int unit_bytes = V * 2 * real_bytes;
+    // (a plane is addressed with 32-bit byte offsets)
+    if ((uint64_t)src.nslices * 64 * unit_bytes > kRingPlane) return nullptr;
     const int64_t n = src.nrows;
     const size_t vsz = src.vsz;
     Csr A;
@@ -587,10 +589,10 @@ void launch_ring(const RingArgs<R>& a, const Ring& r, int V, bool real_vals, hip
     if (r.rows_lane != ring_rows(sizeof(R), V, real_vals, r.width) ||
         r.owned_lane != ring_owned(sizeof(R), V, real_vals, r.width) ||
         r.rows_max > r.rows_lane * kRingLanes || r.owned_max > r.owned_lane * kRingLanes ||
-        a.lds_rows < r.rows_max)
+        (uint64_t)a.plane * sizeof(typename CplxT<R>::T) > kRingPlane)
         throw Error{TBG_EINVAL, "internal: resident pass beyond its workgroup"};
     if ((a.q1 == nullptr) != (a.q2 == nullptr) || a.acc == nullptr || a.p1 == nullptr ||
-        (!a.first && a.p0 == nullptr))
+        (!a.first && a.p0 == nullptr) || (a.q1 != nullptr && a.part != nullptr))
         throw Error{TBG_EINVAL, "internal: resident pass without its vectors"};
 #define TBG_RING_RV(VV)                                                        \
     do {                                                                       \

@@ -70,6 +70,35 @@ struct RingRow {
     }
 };
 
+// The unit of row `row` of a plane (of less than 4 GiB): a scalar base and a
+// 32-bit offset a lane, so that no lane holds addresses.
+template <typename R, int V>
+__device__ __forceinline__ Vec<R, V> unit_at(const void* plane, int row) {
+    return vld<R, V>(reinterpret_cast<const unsigned char*>(plane) +
+                         (unsigned)row * (unsigned)sizeof(Vec<R, V>), 0);
+}
+
+// Stores the unit of row `row`, or nothing for row -1 (beyond the buffer).
+template <typename R, int V>
+__device__ __forceinline__ void unit_to(BufRsrc plane, int row, const Vec<R, V>& o) {
+    const unsigned at = row < 0 ? kRingNowhere : (unsigned)row * (unsigned)sizeof(Vec<R, V>);
+    R t[2 * V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        t[2 * v] = o.re[v];
+        t[2 * v + 1] = o.im[v];
+    }
+    if constexpr (sizeof(o) == 16) {
+        buf_u4 u;
+        __builtin_memcpy(&u, t, 16);
+        __builtin_amdgcn_raw_buffer_store_b128(u, plane, at, 0, 0);
+    } else {
+        buf_u2 u;
+        __builtin_memcpy(&u, t, 8);
+        __builtin_amdgcn_raw_buffer_store_b64(u, plane, at, 0, 0);
+    }
+}
+
 // The unit at LDS byte offset o.  The dynamic LDS is all the LDS that the
 // kernel has, so it starts at offset 0 and the offset is the address.
 template <typename R, int V>
@@ -111,7 +140,8 @@ __device__ __forceinline__ Vec<R, V> lds_unit(unsigned o) {
 // gaps.  Reading the entries from L2 at every term instead of holding them
 // (which allows 5120 rows a block) took 122 against 92 ms for 256 steps of
 // one complex128 state on 4.2M orbitals: its tables then miss L2 at every
-// term; 16-wave workgroups, one a compute unit, 113.
+// term; 16-wave workgroups, one a compute unit, 113 (both before the loads
+// lost their branches, which took the 92 to 81).
 template <typename R, int V, bool RV, int W, bool POLY, int NT, int NR, int NRO>
 struct RingPass {
     using C = typename CplxT<R>::T;
@@ -229,7 +259,14 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
     const int* ends = ends_ + (int64_t)b * (a.depth + 1);
     const int nL = ends[a.T], nC = ends[a.T - 1], n0 = ends[0];
     const int tid = threadIdx.x;
-    const int* rows = rows_ + m.offR;
+    const BufRsrc rowb = buffer_of(rows_ + m.offR, (unsigned)nL * 4u);
+    RingPass<R, V, RV, W, POLY, NT, NR, NRO> P;
+    P.lds = lds;
+    P.tid = tid;
+    P.wide = m.w;
+    P.pad = m.pad;
+    P.idx = idx_ + (W ? m.offT * 4 : m.offE);
+    P.vals = vals_ + (W ? m.offT * W : m.offE) * (RV ? sizeof(R) : sizeof(C));
     const C* p1 = reinterpret_cast<const C*>(a.p1) + g * a.plane;
     const C* p0 = reinterpret_cast<const C*>(a.p0) + g * a.plane;
     C* accp = reinterpret_cast<C*>(a.acc) + g * a.plane;
@@ -240,62 +277,60 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
         cl[v] = (int)((a.cls_mask >> (g * V + v)) & 1ull);
         bw[v] = ((a.bwd_mask >> (g * V + v)) & 1ull) != 0;
     }
-    RingPass<R, V, RV, W, POLY, NT, NR, NRO> P;
-    P.lds = lds;
-    P.tid = tid;
-    P.wide = m.w;
-    P.pad = m.pad;
-    P.idx = idx_ + (W ? m.offT * 4 : m.offE);
-    P.vals = vals_ + (W ? m.offT * W : m.offE) * (RV ? sizeof(R) : sizeof(C));
-#pragma unroll
-    for (int i = 0; i < NR; ++i) P.prev[i] = vzero<R, V>();
-#pragma unroll
-    for (int i = 0; i < NRO; ++i) P.acc[i] = vzero<R, V>();
-    // v_{m-1} of every row to LDS, v_{m-2} and the output to registers
+    // v_{m-1} of every row to LDS, v_{m-2} and the output to registers.
+    // No branches around single loads (lanes beyond the block read row 0; a
+    // block of few rows skips the upper half): with one each, every load
+    // waited for the one before, and this phase took 36,000 of a block's
+    // 75,000 cycles (8.4M rows, four complex64 groups: 334 ms for 128 steps,
+    // 265 without; 4.2M rows, one complex128 state: 96 and 81 for 256).  All
+    // loads at once, the entries first, or v_{m-1} loaded straight to LDS
+    // measured 0 to 8% slower; so did a workgroup that takes several groups
+    // in turn and keeps the entries (they come from L2, and fewer, longer
+    // workgroups balance worse).
     {
         int row[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            row[i] = 0;
-            if (i * NT < nL) row[i] = rows[min(i * NT + tid, nL - 1)];
-        }
+        for (int i = 0; i < NR; ++i)
+            row[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rowb, tid * 4u, i * NT * 4, 0);
         constexpr int HB = (NR + 1) / 2;
 #pragma unroll
         for (int hb = 0; hb < NR; hb += HB) {
+            if (hb * NT >= nL) break;
             VT x[HB];
 #pragma unroll
-            for (int q = 0; q < HB; ++q)
-                if (hb + q < NR && (hb + q) * NT < nL)
-                    x[q] = vld<R, V>(p1, (int64_t)row[hb + q] * V);
+            for (int q = 0; q < HB && hb + q < NR; ++q) x[q] = unit_at<R, V>(p1, row[hb + q]);
 #pragma unroll
-            for (int q = 0; q < HB; ++q) {
+            for (int q = 0; q < HB && hb + q < NR; ++q) {
                 const int i = hb + q;
-                if (i < NR && i * NT < nL) {
-                    if (i * NT + tid < nL) vst<R, V>(lds, (int64_t)(i * NT + tid) * V, x[q]);
-                    if (i < NRO && a.first) {
-                        R c0[V];
-#pragma unroll
-                        for (int v = 0; v < V; ++v) c0[v] = a.c0[cl[v]];
-                        axpy<R, V>(P.acc[i < NRO ? i : 0], c0, x[q]);
-                    }
-                }
+                vst<R, V>(lds, (int64_t)(i * NT + tid) * V, x[q]);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (!a.first) {
 #pragma unroll
-            for (int i = 0; i < NR; ++i)
-                if (i * NT < nC) P.prev[i] = vld<R, V>(p0, (int64_t)row[i] * V);
+            for (int i = 0; i < NR; ++i) P.prev[i] = unit_at<R, V>(p0, row[i]);
 #pragma unroll
-            for (int i = 0; i < NRO; ++i)
-                if (i * NT < n0) P.acc[i] = vld<R, V>(accp, (int64_t)row[i] * V);
+            for (int i = 0; i < NRO; ++i) P.acc[i] = unit_at<R, V>(accp, row[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) P.prev[i] = vzero<R, V>();
         }
     }
     if constexpr (W > 0) {
-        const BufRsrc idx = buffer_of(P.idx, (unsigned)m.pad * 8u);
-        const BufRsrc val = buffer_of(P.vals, (unsigned)(m.pad * RingRow<R, RV, W>::VB));
+        const BufRsrc idx = buffer_of(P.idx, (unsigned)P.pad * 8u);
+        const BufRsrc val = buffer_of(P.vals, (unsigned)(P.pad * RingRow<R, RV, W>::VB));
 #pragma unroll
-        for (int i = 0; i < NR; ++i)
-            if (i * NT < nC) P.tab[i].load(idx, val, i * NT, (unsigned)tid);
+        for (int i = 0; i < NR; ++i) P.tab[i].load(idx, val, i * NT, (unsigned)tid);
+    }
+    if (a.first) {
+        R c0[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) c0[v] = a.c0[cl[v]];
+#pragma unroll
+        for (int i = 0; i < NRO; ++i) {
+            P.acc[i] = vzero<R, V>();
+            axpy<R, V>(P.acc[i], c0, vld<R, V>(lds, (int64_t)(i * NT + tid) * V));
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -305,36 +340,50 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
     int t = 0, na = nC;
     P.template terms<NR>(a, ends, cl, bw, t, na);
     // owned rows: the output, the last two terms (the last one in LDS, where
-    // the same lane wrote it) and the epilogue's sums
+    // the same lane wrote it) and the epilogue's sums.  No branches here
+    // either: the stores of lanes without a row go nowhere.
     double dre[V], dim_[V], nrm[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) { dre[v] = 0.0; dim_[v] = 0.0; nrm[v] = 0.0; }
+    {
+        int at[NRO];
 #pragma unroll
-    for (int i = 0; i < NRO; ++i) {
-        const int l = i * NT + tid;
-        if (l < n0) {
-            const int64_t at = (int64_t)rows[l] * V;
-            const VT o = P.acc[i];
-            vst<R, V>(accp, at, o);
-            if (a.q1 != nullptr) {
-                vst<R, V>(reinterpret_cast<C*>(a.q1) + g * a.plane, at, P.prev[i]);
-                vst<R, V>(reinterpret_cast<C*>(a.q2) + g * a.plane, at,
-                          vld<R, V>(lds, (int64_t)l * V));
+        for (int i = 0; i < NRO; ++i)
+            at[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rowb, tid * 4u, i * NT * 4, 0);
+        const unsigned bytes = (unsigned)(a.plane * (int64_t)sizeof(C));
+        const BufRsrc accb = buffer_of(accp, bytes);
+#pragma unroll
+        for (int i = 0; i < NRO; ++i) at[i] = i * NT + tid < n0 ? at[i] : -1;
+#pragma unroll
+        for (int i = 0; i < NRO; ++i) unit_to<R, V>(accb, at[i], P.acc[i]);
+        if (a.q1 != nullptr) {
+            const BufRsrc q1 = buffer_of(reinterpret_cast<C*>(a.q1) + g * a.plane, bytes);
+            const BufRsrc q2 = buffer_of(reinterpret_cast<C*>(a.q2) + g * a.plane, bytes);
+#pragma unroll
+            for (int i = 0; i < NRO; ++i) {
+                unit_to<R, V>(q1, at[i], P.prev[i]);
+                unit_to<R, V>(q2, at[i], vld<R, V>(lds, (int64_t)(i * NT + tid) * V));
             }
-            if (a.part != nullptr) {
-                if (a.psi0 != nullptr) {
-                    const VT p = vld<R, V>(reinterpret_cast<const C*>(a.psi0) + g * a.plane, at);
+        } else if (a.part != nullptr) {
+            VT p[NRO];
+#pragma unroll
+            for (int i = 0; i < NRO; ++i) p[i] = vzero<R, V>();
+            if (a.psi0 != nullptr) {
+                const C* psi0 = reinterpret_cast<const C*>(a.psi0) + g * a.plane;
+#pragma unroll
+                for (int i = 0; i < NRO; ++i) p[i] = unit_at<R, V>(psi0, max(at[i], 0));
+            }
+#pragma unroll
+            for (int i = 0; i < NRO; ++i) {
+                if (i * NT + tid < n0) {
 #pragma unroll
                     for (int v = 0; v < V; ++v) {
-                        const double pr = p.re[v], pi = p.im[v], orr = o.re[v], oi = o.im[v];
+                        const double pr = p[i].re[v], pi = p[i].im[v];
+                        const double orr = P.acc[i].re[v], oi = P.acc[i].im[v];
                         dre[v] = fma(pr, orr, fma(pi, oi, dre[v]));
                         dim_[v] = fma(pr, oi, fma(-pi, orr, dim_[v]));
+                        nrm[v] = fma(orr, orr, fma(oi, oi, nrm[v]));
                     }
-                }
-#pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    const double orr = o.re[v], oi = o.im[v];
-                    nrm[v] = fma(orr, orr, fma(oi, oi, nrm[v]));
                 }
             }
         }
@@ -373,8 +422,10 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
 
 template <typename R, int V, bool RV, int W, bool POLY>
 static void launch_ring_w(const RingArgs<R>& a, const Ring& r, hipStream_t s) {
-    const size_t lds = std::max<size_t>((size_t)a.lds_rows * V * sizeof(typename CplxT<R>::T),
-                                        (size_t)(kRingLanes / 64) * 3 * V * sizeof(double));
+    // every lane has its rows' places, used or not
+    constexpr size_t lds = (size_t)ring_rows(sizeof(R), V, RV, W) * kRingLanes * V *
+                           sizeof(typename CplxT<R>::T);
+    static_assert(lds >= (kRingLanes / 64) * 3 * V * sizeof(double), "the sums' place");
     hipLaunchKernelGGL((k_ring<R, V, RV, W, POLY, kRingLanes, ring_rows(sizeof(R), V, RV, W), ring_owned(sizeof(R), V, RV, W)>),
                        dim3(r.nblocks * a.groups), dim3(kRingLanes), lds, s, a, r.meta.as<RingMeta>(),
                        r.ends.as<int>(), r.rows.as<int>(), r.idx.as<uint16_t>(),
