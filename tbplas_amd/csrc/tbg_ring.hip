@@ -238,17 +238,21 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
         growth /= std::max(cnt, 1);
     }
 
-    // Depth and owned rows: the least estimated cycles of a compute unit per
-    // owned row and step.  A row of three
-    // entries costs about 0.9 cycles a term (LDS: its entries, its own
-    // value twice); bytes
-    // from HBM pass at about 10 a cycle; of tables that several groups read,
-    // two thirds come from L2.  With two workgroups a compute unit most of
-    // the lesser of the two hides behind the other.  Measured, one pass a
-    // step against two (ms a step): 8.4M rows, four complex64 groups 2.26 /
-    // 2.21; 0.9M rows, eight complex128 groups 0.71 / 0.57; 0.5M rows, six
-    // complex64 groups (15 terms) 0.25 / 0.30; 4.2M rows, one complex128
-    // group 0.36 / 0.37.
+    // Depth and owned rows: the least estimated cycles of a step.  A row of
+    // three entries costs a compute unit about 0.9 cycles a term (LDS: its
+    // entries, its own value twice); bytes pass at about 16 a cycle (of
+    // tables that several groups read, two thirds come from L2); with two
+    // workgroups a compute unit most of the lesser of the two hides behind
+    // the other; a launch takes about 5000.  A sample too small to fill the
+    // chip with full blocks gets one workgroup a compute unit, which is alone
+    // there, rather than two with more halo between them, and two only where
+    // one would be too large (us a step, one / two a unit: 131k rows, one
+    // complex128 state 24 / 31; 65k rows 21 / 31; 32k rows, four states
+    // 26 / 44; 131k rows, four complex64 states 40 / 54).  One pass a step
+    // against two (ms a step): 8.4M rows, four complex64 groups 2.68 / 2.07;
+    // 0.9M rows, eight complex128 groups 0.72 / 0.54; 4.2M rows, one
+    // complex128 group 0.38 / 0.32; 0.5M rows, six complex64 groups (15
+    // terms) 0.29 / 0.32; 0.2M rows, twelve complex128 groups 0.32 / 0.30.
     const int64_t cap = std::min<int64_t>((int64_t)nr * kRingLanes,
                                           (int64_t)h->max_lds / kRingPerCu / unit_bytes);
     const int64_t own_cap = (int64_t)nro * kRingLanes;
@@ -262,10 +266,19 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
         if (d > kRingMax || (passes > 1 && d < 3)) continue;
         const double side = std::sqrt(fill * cap) - growth * d;
         if (side < 8.0) continue;
-        const double slots = (double)h->num_cus * kRingPerCu;
-        double own = std::min<double>((double)own_cap, side * side);
-        // a small sample: a block for every workgroup that runs at once
-        own = std::min(own, std::max(64.0, (double)covered * groups / (0.9 * slots)));
+        const double cus = (double)h->num_cus, rows = (double)covered * groups;
+        const double most = std::min<double>((double)own_cap, side * side);
+        // a small sample: one workgroup a compute unit, or two
+        double own = std::max(64.0, rows / (0.84 * cus));
+        int each = 1;
+        if (own > most) {
+            own = rows / (0.84 * kRingPerCu * cus);
+            each = kRingPerCu;
+        }
+        if (own > most) {
+            own = most;
+            each = 0;
+        }
         double comp = 0.0;
         for (int k = 0; k < d; ++k) {
             const double s = std::sqrt(own) + growth * k;
@@ -276,8 +289,12 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
         const double bytes = all * (4.0 + unit_bytes * (passes > 1 ? 2 : 1)) +
                              all * (groups > 1 ? table / 3.0 : table) +
                              own * unit_bytes * (passes > 1 ? 4 : 3);
-        const double mem = bytes / 10.0 + 2000.0;
-        const double cost = passes * (std::max(comp, mem) + 0.4 * std::min(comp, mem)) / own;
+        const double mem = bytes / 16.0 + 2000.0;
+        const double pair = std::max(comp, mem) + 0.4 * std::min(comp, mem);
+        const double cost =
+            passes * (5000.0 + (each == 1   ? comp + mem
+                                : each == 2 ? 2.0 * pair
+                                            : rows / (0.9 * own * cus) * pair));
         if (best == 0.0 || cost < best) {
             best = cost;
             depth = d;
