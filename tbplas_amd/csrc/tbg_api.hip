@@ -171,6 +171,7 @@ struct DosRun : tbg_run {
         if (ni > 1 && !ring) pre = batch_blocking<R>(h, ni, hams, cat, inst_slices, K);
         e.init(h, mv, inst_slices, K, chunk_target(h, mv.nslices), ni == 1 ? hams[0] : nullptr,
                pre, nb - 1, 0, ring);
+        e.keep_sums();
         const int Kp = e.Kp;
         nv = 3 * Kp;
         psi.alloc(e.vbytes);
@@ -188,21 +189,17 @@ struct DosRun : tbg_run {
         TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), h->stream));
         // t = 0: <psi0|psi0> (tbpm.f90:58-62)
         launch_dotnorm<R>(e.plan, psi.p, psi.p, e.lay, Kp, e.part.template as<double>(), h->stream);
-        reduce(e.plan.inst_chunk_dev.template as<int>());
+        launch_reduce(e.part.template as<double>(), nv, e.plan.inst_chunk_dev.template as<int>(),
+                      n_inst, cbuf.as<double>(), stride, counter.as<int>(), 0, h->stream);
         sp = time_poly(bes, nb);
         TBG_HIP(hipStreamSynchronize(h->stream));
-    }
-
-    // sums the partial rows of ranges[inst] .. ranges[inst + 1] per instance
-    void reduce(const int* ranges) {
-        launch_reduce(e.part.template as<double>(), nv, ranges, n_inst, cbuf.as<double>(), stride,
-                      counter.as<int>(), 0, h->stream);
     }
 
     void advance(int nsteps) override {
         TBG_REQUIRE(nsteps >= 0 && done + nsteps <= T, "advancing past the last time step");
         e.run(nsteps, sp, 0, 0, F_DOT | F_NORM, psi.p, counter.as<int>(),
-              [&]() { reduce(e.epi_range()); });
+              [&]() { e.add_sums(nv, n_inst, cbuf.as<double>(), stride, counter.as<int>()); },
+              [&]() { e.add_rest(nv, n_inst, cbuf.as<double>(), stride, counter.as<int>()); });
         done += nsteps;
     }
 

@@ -504,6 +504,7 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     Engine<R> e;
     e.init(h, view_of(H), {0, H->nslices}, 3 * K, chunks_for(h, H->nslices), H, nullptr, nb - 1,
            std::max(nF, nO) - 1);
+    e.keep_sums();
     const int Kp = e.Kp;
     const hipStream_t st = h->stream;
     DevBuf psi(e.vbytes);
@@ -532,21 +533,30 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     launch_reduce(e.part.template as<double>(), nvn, e.plan.inst_chunk_dev.template as<int>(), 1,
                   nbuf.as<double>(), 0, counter.as<int>(), 0, st);
     const StepPoly sp = time_poly(bes, nb);
+    const int64_t astride = (int64_t)e.plan.nchunks * 8 * K;
+    DevBuf apart((size_t)e.part_steps * astride * sizeof(double));
+    auto reduce_corr = [&](int steps) {
+        if (steps > 0)
+            launch_reduce(apart.as<double>(), 8 * K, e.plan.inst_chunk_dev.template as<int>(), 1,
+                          abuf.as<double>(), 0, counter.as<int>(), 0, st, steps, astride);
+    };
     auto after = [&]() {
-        launch_reduce(e.part.template as<double>(), nvn, e.epi_range(), 1, nbuf.as<double>(), 0,
-                      counter.as<int>(), 0, st);
         timed_launch(h, kTimeAcCorr, [&] {
             hipLaunchKernelGGL(k_accorr<R>, dim3(e.plan.nchunks), dim3(256), 0, st,
                                H->cols.as<int>(), H->jx.as<C>(), H->jy.as<C>(),
                                H->slice_off.as<int64_t>(), H->slice_w.as<int>(),
                                e.plan.chunk.template as<int64_t>(), e.X.template as<C>(), e.lay, K,
-                               e.part.template as<double>());
+                               apart.as<double>() + e.part_at * astride);
         });
-        launch_reduce(e.part.template as<double>(), 8 * K, e.plan.inst_chunk_dev.template as<int>(),
-                      1, abuf.as<double>(), 0, counter.as<int>(), 0, st);
+        e.add_sums(nvn, 1, nbuf.as<double>(), 0, counter.as<int>());
+        if (e.part_at == 0) reduce_corr(e.part_steps);
+    };
+    auto rest = [&]() {
+        reduce_corr(e.part_at);
+        e.add_rest(nvn, 1, nbuf.as<double>(), 0, counter.as<int>());
     };
     // t = 2..T (tbpm.f90:308-345); t = 1 is never stored.
-    if (T >= 2) e.run(T - 1, sp, 0, 0, F_NORM, nullptr, counter.as<int>(), after);
+    if (T >= 2) e.run(T - 1, sp, 0, 0, F_NORM, nullptr, counter.as<int>(), after, rest);
     std::vector<double> ha((size_t)T * 8 * K), hn((size_t)T * nvn);
     TBG_HIP(hipMemcpyAsync(ha.data(), abuf.p, ha.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     TBG_HIP(hipMemcpyAsync(hn.data(), nbuf.p, hn.size() * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -682,6 +692,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     const hipStream_t st = h->stream;
     Engine<R> e;
     e.init(h, view_of(H), {0, H->nslices}, 2 * K, chunks_for(h, H->nslices), H, nullptr, nb - 1);
+    e.keep_sums();
     const int Kp = e.Kp;
     const int64_t n = H->n, n_pad = e.n_pad;
     const int64_t nq = (int64_t)n_en * K;
@@ -780,12 +791,12 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
 #undef TBG_QE
     };
     auto after1 = [&]() {
-        launch_reduce(e.part.template as<double>(), nvn, e.epi_range(), 1, nbuf.as<double>(), 0,
-                      counter.as<int>(), 0, st);
+        e.add_sums(nvn, 1, nbuf.as<double>(), 0, counter.as<int>());
         ++done;
         if (nq > 0 && done % e.hist() == 0) qe_update(e.hist());
     };
-    e.run(T, sp, bwd, 0, F_DOT | F_NORM, psi.p, counter.as<int>(), after1);
+    e.run(T, sp, bwd, 0, F_DOT | F_NORM, psi.p, counter.as<int>(), after1,
+          [&]() { e.add_rest(nvn, 1, nbuf.as<double>(), 0, counter.as<int>()); });
     if (nq > 0 && done % e.hist() != 0) qe_update(done % e.hist());
     TBG_HIP(hipMemcpyAsync(hn.data(), nbuf.p, hn.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     // |QE| and a = |<psi0|QE>| (tbpm.f90:642-647, 667): the currents act on

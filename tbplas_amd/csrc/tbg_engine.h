@@ -180,6 +180,30 @@ struct Engine {
         TBG_HIP(hipStreamSynchronize(h->stream));
     }
 
+    // The epilogue's partial sums of up to part_steps steps, kept apart until
+    // one launch adds them (keep_sums; 16 as a captured graph has steps).
+    int part_steps = 1, part_at = 0;
+    int64_t part_stride = 0;
+    double* part_now() const { return part.template as<double>() + part_at * part_stride; }
+    void keep_sums() {
+        if (part.bytes > ((size_t)4 << 20)) return;   // (a step is long enough)
+        part_stride = (int64_t)(part.bytes / sizeof(double));
+        part_steps = 16;
+        part.alloc((size_t)part_steps * part_stride * sizeof(double));
+    }
+    // After a step that formed sums of nv values: adds them to row *counter
+    // of out, at once or (add_rest) at the end of a run.
+    void add_sums(int nv, int ninst, double* out, int64_t inst_stride, const int* counter) {
+        if (++part_at < part_steps) return;
+        add_rest(nv, ninst, out, inst_stride, counter);
+    }
+    void add_rest(int nv, int ninst, double* out, int64_t inst_stride, const int* counter) {
+        if (part_at == 0) return;
+        launch_reduce(part.template as<double>(), nv, epi_range(), ninst, out, inst_stride, counter,
+                      0, h->stream, part_at, part_stride);
+        part_at = 0;
+    }
+
     // The partial-row range (per instance) that the last step's F_DOT /
     // F_NORM epilogue wrote into part: the chunks of the one-term kernel, or
     // the tiles [0, nblocks) when a pair pass ended the step.
@@ -250,7 +274,7 @@ struct Engine {
             if (mode == PM_M1) t.counter = counter;
             if (mode == PM_NORM || mode == PM_DOTNORM) {
                 t.psi0 = psi0;
-                t.part = part.as<double>();
+                t.part = part_now();
             }
             timed_launch(h, kTimePass + 10 * mode + terms, [&] {
                 launch_pass<R>(mode, terms, M.real_vals != 0, t, *blk, h->stream);
@@ -283,7 +307,7 @@ struct Engine {
             a.cc[0] = sp.c[0][m];
             a.cc[1] = sp.c[1][m];
             a.psi0 = psi0;
-            a.part = part.as<double>();
+            a.part = part_now();
             timed_launch(h, kTimeTerm, [&] {
                 launch_term<R>(F_PREV | F_ACC | F_ACCRMW | epi, a, plan.nchunks, h->stream);
             });
@@ -347,7 +371,7 @@ struct Engine {
             a.q1 = last ? nullptr : b2;
             a.q2 = last ? nullptr : b3;
             if (last && (epi & (F_DOT | F_NORM))) {
-                a.part = part.template as<double>();
+                a.part = part_now();
                 a.psi0 = (epi & F_DOT) ? psi0 : nullptr;
             }
             const int kind = kTimeRing + 100 * ((a.first ? 1 : 0) + (last ? 2 : 0)) + a.T;
@@ -480,7 +504,7 @@ struct Engine {
                 if (last) {
                     fl |= epi;
                     a.psi0 = psi0;
-                    a.part = part.as<double>();
+                    a.part = part_now();
                 }
             }
             timed_launch(h, kTimeTerm, [&] { launch_term<R>(fl, a, plan.nchunks, h->stream); });
@@ -509,9 +533,9 @@ struct Engine {
     }
     ~Engine() { drop_graph(); }
 
-    template <typename F>
+    template <typename F, typename G>
     void capture(int per, const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi,
-                 const void* psi0, int* counter, F&& after) {
+                 const void* psi0, int* counter, F&& after, G&& rest) {
         drop_graph();
         graph_parity = parity;
         TBG_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
@@ -520,6 +544,7 @@ struct Engine {
                 step(sp, bwd, cls, epi, psi0, counter);
                 after();
             }
+            rest();
         } catch (...) {
             hipGraph_t dummy = nullptr;
             (void)hipStreamEndCapture(h->stream, &dummy);
@@ -536,19 +561,27 @@ struct Engine {
     }
 
     // Enqueue nsteps steps, each followed by `after` (reductions etc.),
-    // replaying the captured graph where possible.
+    // replaying the captured graph where possible.  `rest` ends what after
+    // has put off: at the end of the graph, before a replay that follows a
+    // launched step, and at the end.
     template <typename F>
     void run(int nsteps, const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi,
              const void* psi0, int* counter, F&& after) {
+        run(nsteps, sp, bwd, cls, epi, psi0, counter, after, [] {});
+    }
+    template <typename F, typename G>
+    void run(int nsteps, const StepPoly& sp, uint64_t bwd, uint64_t cls, int epi,
+             const void* psi0, int* counter, F&& after, G&& rest) {
         int done = 0;
         if (h->use_graph && !h->timing) {
             // (with kept outputs a graph holds whole rounds of their buffers)
             const int per = slot.empty() ? std::min(16, nsteps & ~1) : nsteps >= 16 ? 16 : 0;
-            if (graph_steps == 0 && per >= 2) capture(per, sp, bwd, cls, epi, psi0, counter, after);
+            if (graph_steps == 0 && per >= 2) capture(per, sp, bwd, cls, epi, psi0, counter, after, rest);
             if (graph_steps > 0 && parity != graph_parity && nsteps > 0) {
                 // one launched step restores the buffer roles of the graph
                 step(sp, bwd, cls, epi, psi0, counter);
                 after();
+                rest();
                 ++done;
             }
             if (graph_steps > 0) {
@@ -561,6 +594,7 @@ struct Engine {
             step(sp, bwd, cls, epi, psi0, counter);
             after();
         }
+        rest();
     }
 };
 

@@ -105,7 +105,8 @@ template <typename R> void launch_term(int flags, const TermArgs& a, int nchunks
 // Sum partial rows per instance: out[i][(*counter + toff) * nv + q].
 void launch_reduce(const double* part, int nv, const int* inst_chunk, int ninst,
                    double* out, int64_t inst_stride, const int* counter, int toff,
-                   hipStream_t s);
+                   hipStream_t s, int steps = 1,
+                   int64_t part_stride = 0);
 // pack complex128 (K, n) -> complex<R> rows of layout lay at a slot offset;
 // with perm (layout row -> caller row) layout row r takes caller row perm[r].
 template <typename R> void launch_pack(const double* src, int K, int64_t n,

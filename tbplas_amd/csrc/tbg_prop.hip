@@ -167,13 +167,18 @@ __global__ void __launch_bounds__(256) k_term(TermArgs a) {
     }
 }
 
-// Fixed-order reduction of partial rows: block (q, inst) sums value q over
-// the instance's chunks (strided per thread, then an LDS tree).
+// Fixed-order reduction of partial rows: block (q, inst, j) sums value q over
+// the instance's chunks (strided per thread, then an LDS tree) of step j of
+// the gridDim.z kept ones, the last of them step *counter.  A launch takes 3
+// to 5 us whatever it sums, as long as a fifth of a small sample's step;
+// sixteen steps at once take 4 to 8.
 __global__ void __launch_bounds__(256)
 k_reduce(const double* part, int nv, const int* inst_chunk, double* out,
-         int64_t inst_stride, const int* counter, int toff) {
+         int64_t inst_stride, const int* counter, int toff, int64_t part_stride) {
     __shared__ double sh[256];
     const int q = blockIdx.x, inst = blockIdx.y;
+    part += blockIdx.z * part_stride;
+    toff -= (int)(gridDim.z - 1 - blockIdx.z);
     const int c0 = inst_chunk[inst], c1 = inst_chunk[inst + 1];
     double acc = 0.0;
     for (int c = c0 + threadIdx.x; c < c1; c += 256) acc += part[(int64_t)c * nv + q];
@@ -364,9 +369,10 @@ template void launch_term<float>(int, const TermArgs&, int, hipStream_t);
 template void launch_term<double>(int, const TermArgs&, int, hipStream_t);
 
 void launch_reduce(const double* part, int nv, const int* inst_chunk, int ninst, double* out,
-                   int64_t inst_stride, const int* counter, int toff, hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce, dim3(nv, ninst), dim3(256), 0, s, part, nv, inst_chunk, out,
-                       inst_stride, counter, toff);
+                   int64_t inst_stride, const int* counter, int toff, hipStream_t s, int steps,
+                   int64_t part_stride) {
+    hipLaunchKernelGGL(k_reduce, dim3(nv, ninst, steps), dim3(256), 0, s, part, nv, inst_chunk,
+                       out, inst_stride, counter, toff, part_stride);
     TBG_HIP(hipGetLastError());
 }
 

@@ -228,3 +228,31 @@ def test_dc_step_blocks_vs_oracle(handle, prec, tol, resident, T, n_en, K):
     r = oracle.orc_quasi_eigenstates(ip, ix, hop, bes, psi, T, t_step, list(en[inds]))
     assert np.max(np.abs(g - r)) < tol * max(1.0, np.max(r))
     H.close()
+
+
+@pytest.mark.parametrize("resident", [True, False])
+@pytest.mark.parametrize("cuts", [[1] * 5, [15, 1, 16, 17], [16, 33], [3, 40, 5], [64], [2, 2, 2]])
+def test_sums_kept_over_steps_equal_sums_of_single_steps(handle, resident, cuts):
+    """The partial sums of up to 16 steps are added by one launch: a run cut
+    anywhere (graphs of any length, rests) has the rows of a run whose steps
+    are launched and summed one by one, bit for bit."""
+    s, csr = _sample(12, 17)
+    order, tiles = s.tile_order(1.0, return_tiles=True)
+    handle.set_blocking(False)
+    handle.set_resident(resident)
+    H = tbpm.Hamiltonian(s.num_orb, *csr, precision="fp64", handle=handle, order=order,
+                         tiles=tiles)
+    bes, psi, T = tbpm.bessel_series(tau_of(s), 1e-14), _states(s.num_orb, 2), sum(cuts)
+    run = tbpm.DosRun(H, bes, psi, T)
+    for c in cuts:
+        run.advance(c)
+    got = run.result()
+    run.close()
+    handle.set_graph(False)
+    single = tbpm.DosRun(H, bes, psi, T)
+    for _ in range(T):
+        single.advance(1)
+    want = single.result()
+    single.close()
+    np.testing.assert_array_equal(got, want)
+    H.close()
