@@ -503,8 +503,7 @@ int tbg_ham_dxy_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng
     return guard([&] {
         check_handle(h);
         TBG_REQUIRE(orb_eng && indptr && nnz && (m == 0 || (hop_i && hop_j)), "null argument");
-        DevBuf tmp;
-        *nnz = place_count(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, indptr, tmp);
+        *nnz = dxy_count(h, n, m, orb_eng, cutoff, hop_i, hop_j, indptr);
     });
 }
 

@@ -8,11 +8,10 @@ namespace tbg {
 void scan_i64(tbg_handle* h, const int64_t* in, int64_t n, int64_t* out, bool exclusive,
               DevBuf& tmp);
 
-// Row pointer of the emission stream (diag_mode 1: |orb_eng| >= cutoff,
-// 2: orb_eng != 0, 0: no diagonal).  Returns the entry count.
-int64_t place_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, int diag_mode,
-                    double cutoff, const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr,
-                    DevBuf& tmp);
+// Row pointer of the emission stream with the diagonals |orb_eng| >= cutoff.
+// Returns the entry count.
+int64_t dxy_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, double cutoff,
+                  const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr);
 
 void dxy_fill(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, const int64_t* hop_i,
               const int64_t* hop_j, const double* hop_v, const double* dr, double cutoff,

@@ -311,11 +311,36 @@ __global__ void k_check_hops(int64_t m, const int64_t* hop_i, const int64_t* hop
         atomicOr(bad, 1);
 }
 
+// One allocation for a builder call's scratch arrays: nine pairs of hipMalloc
+// and hipFree, each a wait for the device, took 3 of the 19 ms of assembling
+// 2M orbitals twice.  What does not fit is allocated by itself.
+struct Scratch {
+    DevBuf all;
+    size_t used = 0;
+    explicit Scratch(size_t bytes) : all(bytes) {}
+    void give(DevBuf& d, size_t bytes) {
+        const size_t at = (used + 255) / 256 * 256;
+        if (at + bytes > all.bytes) {
+            d.alloc(bytes);
+            return;
+        }
+        d.borrow(all.as<unsigned char>() + at, bytes);
+        used = at + bytes;
+    }
+};
+
+// n + 1 counts or offsets, `rows` times, the scan's sums, flags and cursors
+static size_t scratch_bytes(int64_t n, int rows) {
+    return (size_t)(n + 1) * (8 * rows + 4) + (size_t)(n / kScanTile + 2) * 8 +
+           (size_t)(rows + 8) * 256;
+}
+
 // Every hop index must lie in [0, n) before any kernel scatters by it.
 static void check_hop_indices(tbg_handle* h, int64_t n, int64_t m, const int64_t* hop_i,
-                              const int64_t* hop_j) {
+                              const int64_t* hop_j, Scratch& w) {
     if (m == 0) return;
-    DevBuf bad(sizeof(int));
+    DevBuf bad;
+    w.give(bad, sizeof(int));
     TBG_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), h->stream));
     hipLaunchKernelGGL(k_check_hops, dim3(blocks_for(m)), dim3(256), 0, h->stream, m, hop_i,
                        hop_j, n, bad.as<int>());
@@ -326,13 +351,39 @@ static void check_hop_indices(tbg_handle* h, int64_t n, int64_t m, const int64_t
     TBG_REQUIRE(hb == 0, "hop_i/hop_j index out of range [0, n)");
 }
 
-// indptr (n+1) from the emission stream; returns nnz.
-int64_t place_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, int diag_mode,
-                    double cutoff, const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr,
-                    DevBuf& tmp) {
+// The caller's indptr must be the one that the hops give: compared where both
+// are (reading both back and comparing them on the host took half of an
+// assembly: 33 MB and their pages at 2M orbitals).
+__global__ void k_differ(int64_t n, const int64_t* __restrict__ a, const int64_t* __restrict__ b,
+                         int* bad) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && a[i] != b[i]) atomicOr(bad, 1);
+}
+
+static bool same_indptr(tbg_handle* h, int64_t n, const int64_t* a, const int64_t* b,
+                        Scratch& w) {
+    DevBuf bad;
+    w.give(bad, sizeof(int));
+    TBG_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), h->stream));
+    hipLaunchKernelGGL(k_differ, dim3(blocks_for(n + 1)), dim3(256), 0, h->stream, n + 1, a, b,
+                       bad.as<int>());
+    TBG_HIP(hipGetLastError());
+    int hb = 0;
+    TBG_HIP(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    TBG_HIP(hipStreamSynchronize(h->stream));
+    return hb == 0;
+}
+
+// indptr (n+1) from the emission stream (diag_mode 1: |orb_eng| >= cutoff,
+// 2: orb_eng != 0, 0: no diagonal); returns nnz.
+static int64_t place_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
+                           int diag_mode, double cutoff, const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr,
+                    Scratch& w) {
     check_hops(n, m);
-    check_hop_indices(h, n, m, hop_i, hop_j);
-    DevBuf cnt((size_t)(n + 1) * sizeof(int64_t));
+    check_hop_indices(h, n, m, hop_i, hop_j, w);
+    DevBuf cnt, tmp;
+    w.give(cnt, (size_t)(n + 1) * sizeof(int64_t));
+    w.give(tmp, (size_t)(n / kScanTile + 2) * sizeof(int64_t));
     TBG_HIP(hipMemsetAsync(cnt.p, 0, (size_t)(n + 1) * sizeof(int64_t), h->stream));
     const int64_t mx = std::max(n, m);
     hipLaunchKernelGGL(k_count, dim3(blocks_for(mx)), dim3(256), 0, h->stream, n, m, orb_eng,
@@ -347,8 +398,9 @@ int64_t place_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, 
 
 void place_keys(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, int diag_mode,
                 double cutoff, const int64_t* hop_i, const int64_t* hop_j, const int64_t* indptr,
-                int64_t* keys) {
-    DevBuf cursor((size_t)n * sizeof(unsigned int));
+                int64_t* keys, Scratch& w) {
+    DevBuf cursor;
+    w.give(cursor, (size_t)n * sizeof(unsigned int));
     TBG_HIP(hipMemsetAsync(cursor.p, 0, (size_t)n * sizeof(unsigned int), h->stream));
     const int64_t mx = std::max(n, m);
     hipLaunchKernelGGL(k_place, dim3(blocks_for(mx)), dim3(256), 0, h->stream, n, m, orb_eng,
@@ -356,26 +408,28 @@ void place_keys(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, int 
     TBG_HIP(hipGetLastError());
 }
 
+int64_t dxy_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, double cutoff,
+                  const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr) {
+    check_hops(n, m);
+    Scratch w(scratch_bytes(n, 1));
+    return place_count(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, indptr, w);
+}
+
 void dxy_fill(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng, const int64_t* hop_i,
               const int64_t* hop_j, const double* hop_v, const double* dr, double cutoff,
               const int64_t* indptr, int64_t* indices, double* hop, double* dx, double* dy) {
     check_hops(n, m);
-    check_hop_indices(h, n, m, hop_i, hop_j);
+    Scratch w(scratch_bytes(n, 2));
     // The caller's indptr must match the stream (it comes from the count
     // call); verify before scattering into the caller's arrays.
     {
-        DevBuf tmp;
-        DevBuf ref((size_t)(n + 1) * sizeof(int64_t));
-        place_count(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, ref.as<int64_t>(), tmp);
-        std::vector<int64_t> a(n + 1), b(n + 1);
-        TBG_HIP(hipMemcpyAsync(a.data(), ref.p, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost,
-                               h->stream));
-        TBG_HIP(hipMemcpyAsync(b.data(), indptr, (n + 1) * sizeof(int64_t),
-                               hipMemcpyDeviceToHost, h->stream));
-        TBG_HIP(hipStreamSynchronize(h->stream));
-        TBG_REQUIRE(a == b, "indptr does not match the hop list (call tbg_ham_dxy_count first)");
+        DevBuf ref;
+        w.give(ref, (size_t)(n + 1) * sizeof(int64_t));
+        place_count(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, ref.as<int64_t>(), w);
+        TBG_REQUIRE(same_indptr(h, n, ref.as<int64_t>(), indptr, w),
+                    "indptr does not match the hop list (call tbg_ham_dxy_count first)");
     }
-    place_keys(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, indptr, indices);
+    place_keys(h, n, m, orb_eng, 1, cutoff, hop_i, hop_j, indptr, indices, w);
     hipLaunchKernelGGL(k_dxy_fill, dim3(blocks_for(n)), dim3(256), 0, h->stream, n, orb_eng,
                        hop_i, hop_j, reinterpret_cast<const double2*>(hop_v), dr, indptr, indices,
                        reinterpret_cast<double2*>(hop), dx, dy);
@@ -389,13 +443,19 @@ int64_t canon_build(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
                     const int64_t* hop_i, const int64_t* hop_j, const double* hop_v,
                     int64_t* indptr_out, const int64_t* indptr_in, int64_t* indices,
                     double* data) {
-    DevBuf tmp;
-    DevBuf tptr((size_t)(n + 1) * sizeof(int64_t));
-    const int64_t ntmp = place_count(h, n, m, orb_eng, 2, 0.0, hop_i, hop_j, tptr.as<int64_t>(), tmp);
-    DevBuf keys((size_t)std::max<int64_t>(ntmp, 1) * sizeof(int64_t));
-    DevBuf vals((size_t)std::max<int64_t>(ntmp, 1) * sizeof(double2));
-    place_keys(h, n, m, orb_eng, 2, 0.0, hop_i, hop_j, tptr.as<int64_t>(), keys.as<int64_t>());
-    DevBuf cnt((size_t)(n + 1) * sizeof(int64_t));
+    check_hops(n, m);
+    Scratch w(scratch_bytes(n, 4));
+    DevBuf tptr, cnt, tmp;
+    w.give(tptr, (size_t)(n + 1) * sizeof(int64_t));
+    const int64_t ntmp = place_count(h, n, m, orb_eng, 2, 0.0, hop_i, hop_j, tptr.as<int64_t>(), w);
+    const size_t most = (size_t)std::max<int64_t>(ntmp, 1);
+    DevBuf entries(most * (sizeof(int64_t) + sizeof(double2)));
+    DevBuf keys, vals;
+    vals.borrow(entries.p, most * sizeof(double2));
+    keys.borrow(entries.as<double2>() + most, most * sizeof(int64_t));
+    place_keys(h, n, m, orb_eng, 2, 0.0, hop_i, hop_j, tptr.as<int64_t>(), keys.as<int64_t>(), w);
+    w.give(cnt, (size_t)(n + 1) * sizeof(int64_t));
+    w.give(tmp, (size_t)(n / kScanTile + 2) * sizeof(int64_t));
     TBG_HIP(hipMemsetAsync(cnt.p, 0, sizeof(int64_t), h->stream));
     hipLaunchKernelGGL(k_canon_merge, dim3(blocks_for(n)), dim3(256), 0, h->stream, n, orb_eng,
                        hop_i, hop_j, reinterpret_cast<const double2*>(hop_v), tptr.as<int64_t>(),
@@ -405,19 +465,14 @@ int64_t canon_build(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
     DevBuf own;
     int64_t* ip = indptr_out;
     if (!ip) {
-        own.alloc((size_t)(n + 1) * sizeof(int64_t));
+        w.give(own, (size_t)(n + 1) * sizeof(int64_t));
         ip = own.as<int64_t>();
     }
     scan_i64(h, cnt.as<int64_t>(), n + 1, ip, false, tmp);
     TBG_HIP(hipMemcpyAsync(&nnz, ip + n, sizeof(int64_t), hipMemcpyDeviceToHost, h->stream));
     if (indices) {
-        std::vector<int64_t> a(n + 1), b(n + 1);
-        TBG_HIP(hipMemcpyAsync(a.data(), ip, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost,
-                               h->stream));
-        TBG_HIP(hipMemcpyAsync(b.data(), indptr_in, (n + 1) * sizeof(int64_t),
-                               hipMemcpyDeviceToHost, h->stream));
-        TBG_HIP(hipStreamSynchronize(h->stream));
-        TBG_REQUIRE(a == b, "indptr does not match the hop list (call tbg_ham_csr_count first)");
+        TBG_REQUIRE(same_indptr(h, n, ip, indptr_in, w),
+                    "indptr does not match the hop list (call tbg_ham_csr_count first)");
         hipLaunchKernelGGL(k_canon_compact, dim3(blocks_for(n)), dim3(256), 0, h->stream, n,
                            tptr.as<int64_t>(), keys.as<int64_t>(), vals.as<double2>(), indptr_in,
                            indices, reinterpret_cast<double2*>(data));
@@ -429,12 +484,15 @@ int64_t canon_build(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
 
 double get_rescale(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
                    const int64_t* hop_i, const int64_t* hop_j, const double* hop_v) {
-    DevBuf tmp;
-    DevBuf tptr((size_t)(n + 1) * sizeof(int64_t));
-    const int64_t ntmp = place_count(h, n, m, orb_eng, 0, 0.0, hop_i, hop_j, tptr.as<int64_t>(), tmp);
+    check_hops(n, m);
+    Scratch w(scratch_bytes(n, 3));
+    DevBuf tptr;
+    w.give(tptr, (size_t)(n + 1) * sizeof(int64_t));
+    const int64_t ntmp = place_count(h, n, m, orb_eng, 0, 0.0, hop_i, hop_j, tptr.as<int64_t>(), w);
     DevBuf keys((size_t)std::max<int64_t>(ntmp, 1) * sizeof(int64_t));
-    place_keys(h, n, m, orb_eng, 0, 0.0, hop_i, hop_j, tptr.as<int64_t>(), keys.as<int64_t>());
-    DevBuf rs((size_t)n * sizeof(double));
+    place_keys(h, n, m, orb_eng, 0, 0.0, hop_i, hop_j, tptr.as<int64_t>(), keys.as<int64_t>(), w);
+    DevBuf rs;
+    w.give(rs, (size_t)n * sizeof(double));
     hipLaunchKernelGGL(k_rowabs, dim3(blocks_for(n)), dim3(256), 0, h->stream, n, orb_eng,
                        reinterpret_cast<const double2*>(hop_v), tptr.as<int64_t>(),
                        keys.as<int64_t>(), rs.as<double>());

@@ -117,3 +117,41 @@ def test_large_sample_properties(gpu):
     assert np.all(cd == s.hop_v[0])
     # dx is antisymmetric: the pair (r, c) and (c, r) carry opposite signs
     assert abs(np.sum(dx)) < 1e-6 and abs(np.sum(dy)) < 1e-6
+
+
+@pytest.mark.parametrize("at", [0, 1, 255, 256, -2, -1])
+def test_fill_refuses_an_indptr_of_other_hops(gpu, at):
+    """The comparison of the caller's indptr with the hops' own, at the edges
+    of its blocks and ends; the unchanged one passes."""
+    import ctypes
+    import torch
+    s = tb.make_graphene_sample(17, 31)
+    s.init_orb_eng()
+    L, h = tb._lib, tb._lib.default_handle(0)
+    d = tb.sample._DevHops(s, 0, with_dr=True)
+    n, m = s.num_orb, s.num_hop
+    ip = torch.empty(n + 1, dtype=torch.int64, device="cuda:0")
+    nnz = ctypes.c_int64(0)
+    hops = [L.ptr(x) for x in (d.orb_eng, d.hop_i, d.hop_j)]
+    for csr in (False, True):
+        if csr:
+            L.check(L.lib().tbg_ham_csr_count(h.ptr, n, m, *hops, L.ptr(d.hop_v), L.ptr(ip),
+                                              ctypes.byref(nnz)))
+        else:
+            L.check(L.lib().tbg_ham_dxy_count(h.ptr, n, m, *hops, 1e-5, L.ptr(ip),
+                                              ctypes.byref(nnz)))
+        ix = torch.empty(nnz.value, dtype=torch.int64, device="cuda:0")
+        v = torch.empty(nnz.value, dtype=torch.complex128, device="cuda:0")
+        x, y = (torch.empty(nnz.value, dtype=torch.float64, device="cuda:0") for _ in range(2))
+
+        def fill():
+            if csr:
+                return L.lib().tbg_ham_csr_fill(h.ptr, n, m, *hops, L.ptr(d.hop_v), L.ptr(ip),
+                                                L.ptr(ix), L.ptr(v))
+            return L.lib().tbg_ham_dxy_fill(h.ptr, n, m, *hops, L.ptr(d.hop_v), L.ptr(d.dr), 1e-5,
+                                            L.ptr(ip), L.ptr(ix), L.ptr(v), L.ptr(x), L.ptr(y))
+        assert fill() == 0
+        ip[at] += 1
+        torch.cuda.synchronize()
+        with pytest.raises(L.TBGError, match="does not match the hop list"):
+            L.check(fill())
