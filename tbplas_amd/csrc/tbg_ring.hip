@@ -567,9 +567,6 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     up(R->meta, meta.data(), meta.size() * sizeof(RingMeta));
     up(R->ends, ends.data(), ends.size() * sizeof(int));
     up(R->rows, rows.data(), rows.size() * sizeof(int));
-    // (a group of rows past the last table stays inside the allocation)
-    idx.resize(idx.size() + kRingLanes * 4);
-    vals.resize(vals.size() + kRingLanes * 4 * vsz);
     up(R->idx, idx.data(), idx.size() * sizeof(uint16_t));
     up(R->vals, vals.data(), vals.size());
     TBG_HIP(hipStreamSynchronize(h->stream));

@@ -15,26 +15,38 @@ typedef unsigned buf_u3 __attribute__((ext_vector_type(3)));
 typedef unsigned buf_u4 __attribute__((ext_vector_type(4)));
 
 // A buffer of `bytes` bytes at p (the same for every lane); loads beyond it
-// return zeros.
+// return zeros.  Only a load's lane offset is compared with `bytes`, its
+// scalar offset is not: the loads here have a scalar offset of 0, and what
+// comes before a group of rows is taken off the buffer (buffer_from).
 __device__ __forceinline__ BufRsrc buffer_of(const void* p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
+// The part of that buffer from byte `skip` on, empty when it ends before:
+// scalar arithmetic, and the lanes' offsets are the same for every group.
+__device__ __forceinline__ BufRsrc buffer_from(const void* p, unsigned bytes, unsigned skip) {
+    const unsigned s = skip < bytes ? skip : bytes;
+    return buffer_of(static_cast<const unsigned char*>(p) + s, bytes - s);
+}
 
 // The W <= 4 entries of one row: positions in the block and values.  Rows
-// are addressed as a scalar offset (the rows before this group of rows) plus
-// one 32-bit offset a lane, so that no lane holds addresses.
+// are addressed as a scalar base (that of their group) plus one 32-bit
+// offset a lane, so that no lane holds addresses.
 template <typename R, bool RV, int W>
 struct RingRow {
     static constexpr int VB = W * (int)(RV ? sizeof(R) : 2 * sizeof(R));   // value bytes
     static constexpr int NW = VB / 4 > 0 ? VB / 4 : 1;
     buf_u2 c;
     unsigned v[NW];
-    __device__ __forceinline__ void load(BufRsrc idx, BufRsrc vals, int r0, unsigned lane) {
-        c = __builtin_amdgcn_raw_buffer_load_b64(idx, lane * 8u, r0 * 8, 0);
+    // row r0 + lane of the tables of `rows` rows
+    __device__ __forceinline__ void load(const void* idx_, const void* vals_, unsigned rows,
+                                         unsigned r0, unsigned lane) {
+        const BufRsrc idx = buffer_from(idx_, rows * 8u, r0 * 8u);
+        const BufRsrc vals = buffer_from(vals_, rows * (unsigned)VB, r0 * (unsigned)VB);
+        c = __builtin_amdgcn_raw_buffer_load_b64(idx, lane * 8u, 0, 0);
 #pragma unroll
         for (int q = 0; q + 4 <= NW; q += 4) {
             const buf_u4 t =
-                __builtin_amdgcn_raw_buffer_load_b128(vals, lane * VB + q * 4u, r0 * VB, 0);
+                __builtin_amdgcn_raw_buffer_load_b128(vals, lane * VB + q * 4u, 0, 0);
             v[q] = t.x;
             v[q + 1] = t.y;
             v[q + 2] = t.z;
@@ -43,13 +55,13 @@ struct RingRow {
         constexpr int q = NW / 4 * 4;
         if constexpr (NW % 4 == 3) {
             const buf_u3 t =
-                __builtin_amdgcn_raw_buffer_load_b96(vals, lane * VB + q * 4u, r0 * VB, 0);
+                __builtin_amdgcn_raw_buffer_load_b96(vals, lane * VB + q * 4u, 0, 0);
             v[q] = t.x;
             v[q + 1] = t.y;
             v[q + 2] = t.z;
         } else if constexpr (NW % 4 == 2) {
             const buf_u2 t =
-                __builtin_amdgcn_raw_buffer_load_b64(vals, lane * VB + q * 4u, r0 * VB, 0);
+                __builtin_amdgcn_raw_buffer_load_b64(vals, lane * VB + q * 4u, 0, 0);
             v[q] = t.x;
             v[q + 1] = t.y;
         }
@@ -259,7 +271,11 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
     const int* ends = ends_ + (int64_t)b * (a.depth + 1);
     const int nL = ends[a.T], nC = ends[a.T - 1], n0 = ends[0];
     const int tid = threadIdx.x;
-    const BufRsrc rowb = buffer_of(rows_ + m.offR, (unsigned)nL * 4u);
+    // the layout row of row i NT + lane of the block (beyond the block: row 0)
+    auto layout_row = [&](int i, unsigned lane) {
+        return (int)__builtin_amdgcn_raw_buffer_load_b32(
+            buffer_from(rows_ + m.offR, (unsigned)nL * 4u, i * NT * 4u), lane * 4u, 0, 0);
+    };
     RingPass<R, V, RV, W, POLY, NT, NR, NRO> P;
     P.lds = lds;
     P.tid = tid;
@@ -289,9 +305,10 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
     // workgroups balance worse).
     {
         int row[NR];
+        unsigned ln = tid;   // (a copy: no offset made from it outlives the loads)
+        asm volatile("" : "+v"(ln));
 #pragma unroll
-        for (int i = 0; i < NR; ++i)
-            row[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rowb, tid * 4u, i * NT * 4, 0);
+        for (int i = 0; i < NR; ++i) row[i] = layout_row(i, ln);
         constexpr int HB = (NR + 1) / 2;
 #pragma unroll
         for (int hb = 0; hb < NR; hb += HB) {
@@ -317,10 +334,11 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
         }
     }
     if constexpr (W > 0) {
-        const BufRsrc idx = buffer_of(P.idx, (unsigned)P.pad * 8u);
-        const BufRsrc val = buffer_of(P.vals, (unsigned)(P.pad * RingRow<R, RV, W>::VB));
+        unsigned ln = tid;
+        asm volatile("" : "+v"(ln));
 #pragma unroll
-        for (int i = 0; i < NR; ++i) P.tab[i].load(idx, val, i * NT, (unsigned)tid);
+        for (int i = 0; i < NR; ++i)
+            P.tab[i].load(P.idx, P.vals, (unsigned)P.pad, i * NT, ln);
     }
     if (a.first) {
         R c0[V];
@@ -348,8 +366,7 @@ k_ring(RingArgs<R> a, const RingMeta* __restrict__ meta_, const int* __restrict_
     {
         int at[NRO];
 #pragma unroll
-        for (int i = 0; i < NRO; ++i)
-            at[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rowb, tid * 4u, i * NT * 4, 0);
+        for (int i = 0; i < NRO; ++i) at[i] = layout_row(i, tid);
         const unsigned bytes = (unsigned)(a.plane * (int64_t)sizeof(C));
         const BufRsrc accb = buffer_of(accp, bytes);
 #pragma unroll
