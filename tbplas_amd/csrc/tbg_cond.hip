@@ -17,6 +17,7 @@
 #include <cmath>
 
 #include "tbg_cond.h"
+#include "tbg_dc_split.h"
 
 namespace tbg {
 
@@ -352,9 +353,10 @@ k_dc_y(const int* __restrict__ cols, const typename CplxT<R>::T* __restrict__ jx
     }
 }
 
-// The DC correlations of `count` <= 16 steps: for each current a, state s:
-// part[z][tile][v][j][e] = sum_{rows of split z} conj(X_j(aK + s)) Y_a(e, s),
-// a 16 x n_en product over the rows on the FP64 matrix cores (complex: four
+// The DC correlations of `count` <= 16 steps at the energies e0 .. e0 + ne of
+// n_en (DcSplit): for each current a, state s: part[z][tile][v][j][e] =
+// sum_{rows of split z} conj(X_j(aK + s)) Y_a(e0 + e, s), a 16 x ne product
+// over the rows on the FP64 matrix cores (complex: four
 // v_mfma_f64_16x16x4f64 per four rows).  A wave owns one tile (current, unit
 // of VU states, 16 energies) and one split of the rows and reads both
 // operands as it multiplies: lane i + 16 k holds step i and energy i of row
@@ -365,16 +367,16 @@ typedef double dc_d4 __attribute__((ext_vector_type(4)));
 template <typename R, int VU>
 __global__ void __launch_bounds__(256)
 k_dcdot(DcStates xs, int count, Lay lay, int K, int64_t n_pad, const double2* __restrict__ Y,
-        QLay ql, int n_en, int64_t split, double2* __restrict__ part) {
+        QLay ql, int n_en, int e0, int ne, int64_t split, double2* __restrict__ part) {
     using C = typename CplxT<R>::T;
     const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
-    const int et = (n_en + 15) / 16, units = K / VU, tiles = 2 * units * et;
+    const int et = (ne + 15) / 16, units = K / VU, tiles = 2 * units * et;
     // blocks b, b + 8, ...: one XCD; the tiles of the same rows follow each
     // other there, for they read the same lines of states and of Y
     const int xcd = blockIdx.x % 8, b = blockIdx.x / 8, tile = b % tiles;
     const int64_t z = (int64_t)(b / tiles * 8 + xcd) * 4 + (threadIdx.x >> 6);
     const int a = tile / (units * et), u = tile / et % units;
-    const int e = min((tile % et) * 16 + i, n_en - 1);
+    const int e = e0 + min((tile % et) * 16 + i, ne - 1);
     const int64_t r0 = z * split, r1 = min(r0 + split, n_pad);
     const C* X = reinterpret_cast<const C*>(xs.p[min(i, count - 1)]);
     const double2* Yp = Y + ((int64_t)a * n_en + e) * ql.stride;
@@ -422,12 +424,13 @@ k_dcdot(DcStates xs, int count, Lay lay, int K, int64_t n_pad, const double2* __
 // 1 + j of out: out[row][a nq + e K + s].
 template <int VU>
 __global__ void __launch_bounds__(256)
-k_dcsum(const double2* __restrict__ part, int nz, int count, int K, int n_en,
+k_dcsum(const double2* __restrict__ part, int nz, int count, int K, int n_en, int e0, int ne,
         const int* __restrict__ counter, double2* __restrict__ out) {
-    const int et = (n_en + 15) / 16, units = K / VU;
+    const int et = (ne + 15) / 16, units = K / VU;
     const int tile = blockIdx.x, v = blockIdx.y, o = threadIdx.x, j = o >> 4;
-    const int a = tile / (units * et), u = tile / et % units, e = (tile % et) * 16 + (o & 15);
-    if (j >= count || e >= n_en) return;
+    const int a = tile / (units * et), u = tile / et % units, el = (tile % et) * 16 + (o & 15);
+    if (j >= count || el >= ne) return;
+    const int e = e0 + el;
     double2 t = make_double2(0.0, 0.0);
     for (int z = 0; z < nz; ++z) {
         const double2 p = part[(((int64_t)z * gridDim.x + tile) * VU + v) * 256 + o];
@@ -850,41 +853,44 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     const int64_t nq2 = 2 * nq;
     DevBuf cbuf((size_t)std::max<int64_t>(T * nq2 * 2, 1) * sizeof(double));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-    // splits of the rows: about 16 waves a compute unit over all tiles
     const bool pairs = sizeof(R) == 4 && ql.lin && ql.lay.sh == 1;
     const int VU = pairs ? 2 : 1;
-    const int tiles = 2 * (K / VU) * ((n_en + 15) / 16);
-    int64_t split = 0, nz = 0;
+    DcSplit ds{};
     DevBuf dpart;
     if (nq2 > 0) {
-        const int64_t want = (16 * (int64_t)h->num_cus / tiles + 31) / 32 * 32;
-        split = std::max<int64_t>(64, ((n_pad + want - 1) / want + 63) / 64 * 64);
-        nz = ((n_pad + split - 1) / split + 31) / 32 * 32;   // 4 waves a block, 8 XCDs
-        dpart.alloc((size_t)nz * tiles * VU * 256 * sizeof(double2));
+        ds = dc_split(K, VU, n_en, n_pad, h->num_cus);
+        dpart.alloc((size_t)ds.nz * ds.tiles * VU * 256 * sizeof(double2));
     }
     auto correlate = [&](int count) {
         const DcStates xs = kept(count);
-        timed_launch(h, kTimeDcDot, [&] {
-            const dim3 grid((unsigned)(nz / 4 * tiles));
-            if (pairs) {
-                if constexpr (sizeof(R) == 4)
-                    hipLaunchKernelGGL((k_dcdot<R, 2>), grid, dim3(256), 0, st, xs, count, e.lay,
-                                       K, n_pad, Y.as<double2>(), ql, n_en, split,
+        for (int e0 = 0; e0 < n_en; e0 += ds.ne) {
+            const int ne = std::min(ds.ne, n_en - e0);
+            const int tiles = 2 * (K / VU) * ((ne + 15) / 16);
+            timed_launch(h, kTimeDcDot, [&] {
+                const dim3 grid((unsigned)(ds.nz / 4 * tiles));
+                if (pairs) {
+                    if constexpr (sizeof(R) == 4)
+                        hipLaunchKernelGGL((k_dcdot<R, 2>), grid, dim3(256), 0, st, xs, count,
+                                           e.lay, K, n_pad, Y.as<double2>(), ql, n_en, e0, ne,
+                                           ds.split, dpart.as<double2>());
+                } else {
+                    hipLaunchKernelGGL((k_dcdot<R, 1>), grid, dim3(256), 0, st, xs, count, e.lay,
+                                       K, n_pad, Y.as<double2>(), ql, n_en, e0, ne, ds.split,
                                        dpart.as<double2>());
-            } else {
-                hipLaunchKernelGGL((k_dcdot<R, 1>), grid, dim3(256), 0, st, xs, count, e.lay, K,
-                                   n_pad, Y.as<double2>(), ql, n_en, split, dpart.as<double2>());
-            }
+                }
+                TBG_HIP(hipGetLastError());
+            });
+            const dim3 grid((unsigned)tiles, VU);
+            if (pairs)
+                hipLaunchKernelGGL(k_dcsum<2>, grid, dim3(256), 0, st, dpart.as<double2>(),
+                                   (int)ds.nz, count, K, n_en, e0, ne, counter.as<int>(),
+                                   cbuf.as<double2>());
+            else
+                hipLaunchKernelGGL(k_dcsum<1>, grid, dim3(256), 0, st, dpart.as<double2>(),
+                                   (int)ds.nz, count, K, n_en, e0, ne, counter.as<int>(),
+                                   cbuf.as<double2>());
             TBG_HIP(hipGetLastError());
-        });
-        const dim3 grid((unsigned)tiles, VU);
-        if (pairs)
-            hipLaunchKernelGGL(k_dcsum<2>, grid, dim3(256), 0, st, dpart.as<double2>(), (int)nz,
-                               count, K, n_en, counter.as<int>(), cbuf.as<double2>());
-        else
-            hipLaunchKernelGGL(k_dcsum<1>, grid, dim3(256), 0, st, dpart.as<double2>(), (int)nz,
-                               count, K, n_en, counter.as<int>(), cbuf.as<double2>());
-        TBG_HIP(hipGetLastError());
+        }
     };
     base = e.cur;
     done = 0;

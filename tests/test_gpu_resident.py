@@ -230,6 +230,35 @@ def test_dc_step_blocks_vs_oracle(handle, prec, tol, resident, T, n_en, K):
     H.close()
 
 
+@pytest.mark.parametrize("prec,resident,K,n_en", [
+    ("fp64", True, 32, 1024), ("fp64", True, 32, 1025), ("fp64", False, 32, 2100),
+    ("fp32", True, 32, 2049), ("fp64", False, 8, 4097)])
+def test_dc_many_energies(handle, prec, resident, K, n_en):
+    """More energies than one launch takes (its tiles of a current, a state
+    and 16 energies are at most 16 a compute unit; 1024 energies of 32 states
+    on 256 units): the same numbers as runs over parts of the energies, of
+    which each sum is independent (1e-12 of the largest: sums of 128 rows in
+    another grouping)."""
+    s, _ = _sample(6, 9, vac=0.0)
+    ip, ix, hop, dx, dy = oracle.build_ham_dxy_loop(s.orb_eng, s.hop_i, s.hop_j, s.hop_v, s.dr)
+    bes = tbpm.bessel_series(tau_of(s), 1e-14)
+    psi = _states(s.num_orb, K)
+    en = np.linspace(-2.6, 2.6, n_en)
+    handle.set_blocking(False)
+    handle.set_resident(resident)
+    order, tiles = s.tile_order(1.3, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, hop, dx, dy, cur_scale=9.0, precision=prec,
+                         handle=handle, order=order if resident else None,
+                         tiles=tiles if resident else None)
+    run = [tbpm.corr_dc(H, bes, psi, 3, 2 * math.pi / 18.0, en, inds)
+           for inds in (np.arange(n_en), np.arange(7), np.arange(n_en - 19, n_en))]
+    assert np.all(np.isfinite(run[0][1]))
+    np.testing.assert_array_equal(run[0][0], run[1][0])
+    for part, got in ((run[1][1], run[0][1][:, :, :7]), (run[2][1], run[0][1][:, :, -19:])):
+        assert np.max(np.abs(got - part)) < 1e-12 * max(1.0, np.max(np.abs(part)))
+    H.close()
+
+
 @pytest.mark.parametrize("resident", [True, False])
 @pytest.mark.parametrize("cuts", [[1] * 5, [15, 1, 16, 17], [16, 33], [3, 40, 5], [64], [2, 2, 2]])
 def test_sums_kept_over_steps_equal_sums_of_single_steps(handle, resident, cuts):
