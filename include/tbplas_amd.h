@@ -72,6 +72,12 @@ int tbg_set_blocking(tbg_handle *h, int enable, int max_rows);
  * counterpart. */
 int tbg_set_resident(tbg_handle *h, int enable);
 
+/* States that a DC or quasi-eigenstate run keeps between two updates of its
+ * energies: the power of two up to `most` (1 to 16, default 16) that fits
+ * the free memory.  Fewer need less memory and take longer; the results
+ * agree to rounding.  No reference counterpart. */
+int tbg_set_kept_steps(tbg_handle *h, int most);
+
 /* ---- CSR assembly --------------------------------------------------------
  * Replaces the Cython build_ham_dxy_fast (tbplas/cython/sample.pyx:148-257,
  * called from tbplas/builder/sample.py:452-458).  Insertion order: within a

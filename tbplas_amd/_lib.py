@@ -41,6 +41,7 @@ _SIGS = {
                                ctypes.POINTER(_P)],
     "tbg_set_blocking": [_P, _I, _I],
     "tbg_set_resident": [_P, _I],
+    "tbg_set_kept_steps": [_P, _I],
     "tbg_ham_blocking_info": [_P, _P, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_D)],
     "tbg_ham_blocking_launch": [_P, _P, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)],
     "tbg_ham_blocking_bytes": [_P, _P, _I, _I, _P],
@@ -192,6 +193,11 @@ class Handle:
         blocks that stay in LDS and registers, for Hamiltonians with spatial
         tiles (same states); set_blocking turns it off again."""
         check(lib().tbg_set_resident(self._h, 1 if enable else 0))
+
+    def set_kept_steps(self, most=16):
+        """States a DC or quasi-eigenstate run may keep between two updates
+        of its energies (1 to 16): fewer need less memory."""
+        check(lib().tbg_set_kept_steps(self._h, int(most)))
 
     def set_kernel_timing(self, enable=True):
         """Bracket every propagation and correlation launch by HIP events

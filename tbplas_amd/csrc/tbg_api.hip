@@ -444,6 +444,14 @@ int tbg_set_resident(tbg_handle* h, int enable) {
     });
 }
 
+int tbg_set_kept_steps(tbg_handle* h, int most) {
+    return guard([&] {
+        check_handle(h);
+        TBG_REQUIRE(most >= 1 && most <= 16, "kept steps must be in [1, 16]");
+        h->kept_steps = most;
+    });
+}
+
 int tbg_set_real_layout(tbg_handle* h, int enable) {
     return guard([&] {
         check_handle(h);

@@ -709,7 +709,7 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
         size_t room = 0, total = 0;
         TBG_HIP(hipMemGetInfo(&room, &total));
         const size_t rest = (size_t)n_pad * nq * 3 * sizeof(double2) + ((size_t)1 << 29);
-        e.keep_history(T, room > rest ? (room - rest) / 2 : 0);
+        e.keep_history(T, room > rest ? (room - rest) / 2 : 0, h->kept_steps);
     }
     const QLay ql = q_layout(e.lay, K, n_pad);
     uint64_t bwd = 0;

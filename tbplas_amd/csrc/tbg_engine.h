@@ -398,15 +398,16 @@ struct Engine {
     // the call lies in buffer k % hist() until hist() steps later.  Buffers of
     // their own, as many as fit in `room` bytes: 16 at most (the steps of a
     // captured graph, which then holds whole rounds of them), no more than
-    // `steps` need, or none: then only the last output is there.
+    // `steps` need or `most` allows, fewer where an allocation fails, or none:
+    // then only the last output is there.
     std::vector<DevBuf> slot;
     DevBuf spare;   // the recurrence buffer that X is where nothing is kept
     int cur = 0;
     int hist() const { return slot.empty() ? 1 : (int)slot.size(); }
-    void keep_history(int steps, size_t room) {
+    void keep_history(int steps, size_t room, int most = 16) {
         const bool need_spare = !(ring && S.p == nullptr);   // two passes leave X as it is
         int want = 16;
-        while (want > 1 && want / 2 >= steps) want /= 2;
+        while (want > 1 && (want / 2 >= steps || want > most)) want /= 2;
         for (; want >= 2; want /= 2) {
             if ((size_t)(want - 2 + need_spare) * vbytes > room) continue;
             try {

@@ -71,6 +71,7 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, b);
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();   // or the next launch's check would report it
             throw Error{TBG_EOOM, "hipMalloc(" + std::to_string(b) + " bytes) failed: " +
                                       hipGetErrorString(e)};
         }
@@ -122,6 +123,7 @@ struct tbg_handle {
     int blocking = 3;         // terms per pass where H has spatial tiles (3 to 5; 0: one)
     int resident = 0;         // resident passes where H has spatial tiles (over blocking)
     int block_rows = 0;       // cap on rows owned per workgroup (0: from LDS)
+    int kept_steps = 16;      // states that a DC run may keep (tbg_set_kept_steps)
     int max_lds = 65536;      // LDS bytes one workgroup may use
     tbg::DevBuf scratch;      // reduction partials and small tables
     tbg::DevBuf counter;      // step counter for graph-replayed reductions

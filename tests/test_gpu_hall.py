@@ -51,3 +51,22 @@ def test_hall_moments_tile_edges_vs_oracle(gpu, real, n, width, N, K):
     L.check(L.lib().tbg_hall_mu(H.handle.ptr, H.ptr, L.ptr(p), K, N, 2, L.ptr(out)))
     np.testing.assert_array_equal(out.cpu().numpy().transpose(0, 2, 1), g)   # (i + j N)
     H.close()
+
+
+def test_a_run_after_one_that_did_not_fit(gpu):
+    """An allocation that fails is an error of its own call only: 1.1 times
+    the device's memory in Chebyshev vectors, then a run that fits."""
+    ip, ix, hop, dx, dy = _random_ham(64, 3, True, 5)
+    psi = tb.states.random_states(64, tb.states.sample_seeds(3, 1))
+    small = tbpm.Hamiltonian(64, ip, ix, hop, dx, dy, precision="fp64")
+    want = tbpm.hall_mu(small, psi, 8, 1)
+    n, N = 4_000_000, 1 + int(1.1 * gpu.cuda.mem_get_info()[1] / (4_000_000 * 16))
+    e = np.arange(n + 1, dtype=np.int64)
+    z = np.zeros(n)
+    large = tbpm.Hamiltonian(n, e, e[:-1], z + 0.5, z, z, precision="fp64", handle=small.handle)
+    with pytest.raises(tb._lib.TBGError) as err:
+        tbpm.hall_mu(large, np.full((1, n), n ** -0.5 + 0j), N, 1)
+    assert err.value.code == tb._lib.TBG_EOOM
+    np.testing.assert_array_equal(tbpm.hall_mu(small, psi, 8, 1), want)
+    large.close()
+    small.close()

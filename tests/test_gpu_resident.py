@@ -230,6 +230,41 @@ def test_dc_step_blocks_vs_oracle(handle, prec, tol, resident, T, n_en, K):
     H.close()
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("resident", [True, False])
+@pytest.mark.parametrize("T", [7, 16, 37])
+def test_dc_kept_steps(handle, prec, resident, T):
+    """Runs that keep 1, 2, 4 or 8 states (less memory) give what runs that
+    keep 16 give: the same quasi-eigenstates bit for bit (each is summed step
+    by step in every block length), and correlations to the grouping of the
+    rows (1e-12 of the largest)."""
+    s, _ = _sample(9, 14)
+    ip, ix, hop, dx, dy = oracle.build_ham_dxy_loop(s.orb_eng, s.hop_i, s.hop_j, s.hop_v, s.dr)
+    bes = tbpm.bessel_series(tau_of(s), 1e-14)
+    psi = _states(s.num_orb, 3)
+    en = np.linspace(-2.6, 2.6, 18)
+    handle.set_blocking(False)
+    handle.set_resident(resident)
+    order, tiles = s.tile_order(1.3, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, hop, dx, dy, cur_scale=9.0, precision=prec,
+                         handle=handle, order=order if resident else None,
+                         tiles=tiles if resident else None)
+    res = {}
+    for most in (16, 8, 5, 2, 1):
+        handle.set_kept_steps(most)
+        d, c = tbpm.corr_dc(H, bes, psi, T, 2 * math.pi / 18.0, en, np.arange(18))
+        res[most] = d, c, tbpm.quasi_eigenstates(H, bes, psi, T, 2 * math.pi / 18.0, list(en))
+    d16, c16, q16 = res[16]
+    for d, c, q in res.values():
+        np.testing.assert_array_equal(d, d16)
+        np.testing.assert_array_equal(q, q16)
+        assert np.max(np.abs(c - c16)) < 1e-12 * max(1.0, np.max(np.abs(c16)))
+    for bad in (0, 17):
+        with pytest.raises(tb._lib.TBGError):
+            handle.set_kept_steps(bad)
+    H.close()
+
+
 @pytest.mark.parametrize("prec,resident,K,n_en", [
     ("fp64", True, 32, 1024), ("fp64", True, 32, 1025), ("fp64", False, 32, 2100),
     ("fp32", True, 32, 2049), ("fp64", False, 8, 4097)])

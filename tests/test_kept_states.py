@@ -1,0 +1,88 @@
+"""The states a DC run keeps, as many as memory gives: Engine::keep_history
+on the CPU, compiled against a stand-in for the HIP runtime whose allocations
+fail beyond a budget and leave their error for the next check, as HIP does."""
+import subprocess
+
+import pytest
+
+from tbplas_amd import build
+
+CODE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include "tbg_engine.h"
+
+static size_t budget = 0, used = 0;
+static std::map<void*, size_t> blocks;
+static hipError_t last = hipSuccess;
+hipError_t hipMalloc(void** p, size_t n) {
+    if (used + n > budget) return last = hipErrorOutOfMemory;
+    *p = std::malloc(n);
+    blocks[*p] = n;
+    used += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    used -= blocks.at(p);
+    blocks.erase(p);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipGetLastError() {
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
+const char* hipGetErrorString(hipError_t) { return "out of memory"; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+namespace tbg {
+void launch_fill_zero(void*, size_t, hipStream_t) { TBG_HIP(hipGetLastError()); }
+}
+int main(int, char** v) {
+    const int free_buffers = std::atoi(v[1]), steps = std::atoi(v[2]), room = std::atoi(v[3]),
+              most = std::atoi(v[4]);
+    try {
+        tbg_handle h;
+        tbg::Engine<double> e;
+        e.h = &h;
+        e.vbytes = 1000;
+        budget = 2000 + 1000 * (size_t)free_buffers;
+        e.X.alloc(1000);
+        e.Y.alloc(1000);
+        e.keep_history(steps, (size_t)room * 1000, most);
+        if (hipGetLastError() != hipSuccess) return 2;
+        std::printf("%d %zu\n", e.hist(), used / 1000);
+    } catch (const tbg::Error& e) {
+        std::printf("%s\n", e.msg.c_str());
+        return 1;
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    d = tmp_path_factory.mktemp("kept")
+    src, out = d / "t.cpp", d / "t"
+    src.write_text(CODE)
+    subprocess.run(["g++", "-std=c++17", "-O0", "-w", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-I", build.CSRC, str(src), "-o", str(out)],
+                   check=True)
+    return str(out)
+
+
+@pytest.mark.parametrize("free,steps,room,most,kept", [
+    (99, 500, 99, 16, 16), (99, 500, 99, 8, 8), (99, 500, 99, 7, 4), (99, 500, 99, 1, 1),
+    (99, 500, 14, 16, 8), (99, 500, 7, 16, 8), (99, 500, 6, 16, 4), (99, 500, 0, 16, 1),
+    (99, 1, 99, 16, 1), (99, 2, 99, 16, 2), (99, 8, 99, 16, 8), (99, 9, 99, 16, 16),
+    # the allocations fail where the free memory promised more
+    (15, 500, 99, 16, 16), (14, 500, 99, 16, 8), (6, 500, 99, 16, 4), (2, 500, 99, 16, 2),
+    (1, 500, 99, 16, 2), (0, 500, 99, 16, 1)])
+def test_as_many_states_as_memory_gives(exe, free, steps, room, most, kept):
+    """kept - 2 buffers beside the two of the engine, and a spare one."""
+    r = subprocess.run([exe, str(free), str(steps), str(room), str(most)], capture_output=True,
+                       text=True)
+    assert r.returncode == 0, r.stdout
+    assert r.stdout.split() == [str(kept), str(kept + 1 if kept > 1 else 2)]
