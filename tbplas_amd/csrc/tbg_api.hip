@@ -127,8 +127,7 @@ static std::shared_ptr<Ring> batch_ring(tbg_handle* h, int ni, const tbg_ham* co
         if (hams[i]->tiles.size() < 2) return nullptr;
     if (terms > kRingMax) terms = 20;
     const int Kp = slots_for(K), V = ring_vectors<R>(Kp);
-    std::string key = std::to_string(V) + "|" + std::to_string(Kp / V) + "|" +
-                      std::to_string(terms);
+    std::string key = ring_key((int)sizeof(R), V, Kp / V) + std::to_string(terms);
     for (int i = 0; i < ni; ++i) key += "|" + std::to_string(hams[i]->uid);
     for (const auto& kv : h->batch_ring)
         if (kv.first == key) return kv.second;
@@ -355,7 +354,7 @@ static void check_psi_args(const tbg_ham* H, const double* psi0, int K, int T) {
 static std::shared_ptr<Ring> ring_of(tbg_handle* h, const tbg_ham* H, int Kp, int real_bytes) {
     if (!h->resident) return nullptr;
     const int V = real_bytes == 4 ? ring_vectors<float>(Kp) : ring_vectors<double>(Kp);
-    const std::string want = std::to_string(V) + "|" + std::to_string(Kp / V) + "|";
+    const std::string want = ring_key(real_bytes, V, Kp / V);
     for (auto it = H->rings.rbegin(); it != H->rings.rend(); ++it)
         if (it->first.compare(0, want.size(), want) == 0) return it->second;
     return get_ring(h, H, real_bytes, V, Kp / V, 20);

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <memory>
+#include <string>
 #include <vector>
 
 #include "tbg_block.h"
@@ -76,7 +77,11 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
                                  const std::vector<std::vector<int64_t>>& segs, int real_bytes,
                                  int V, int groups, int terms, bool real_vals);
 
-// The tables of H for groups of V states (built on
+// What tables are made for, as a cache key that starts with everything but
+// the terms.
+std::string ring_key(int real_bytes, int V, int groups);
+
+// The tables of H for groups of V states of real_bytes-byte reals (built on
 // first use, the last few kept on H), or null when the handle does not ask
 // for resident passes, H has no tiles, or no block fits.
 std::shared_ptr<Ring> get_ring(tbg_handle* h, const tbg_ham* H, int real_bytes, int V, int groups,

@@ -573,12 +573,16 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     return R;
 }
 
+std::string ring_key(int real_bytes, int V, int groups) {
+    return std::to_string(real_bytes) + "|" + std::to_string(V) + "|" + std::to_string(groups) +
+           "|";
+}
+
 std::shared_ptr<Ring> get_ring(tbg_handle* h, const tbg_ham* H, int real_bytes, int V, int groups,
                                int terms) {
     if (!h->resident || H->tiles.size() < 2) return nullptr;
     if (terms > kRingMax) terms = 20;    // a long series: any depth divides it well
-    const std::string key = std::to_string(V) + "|" + std::to_string(groups) + "|" +
-                            std::to_string(terms);
+    const std::string key = ring_key(real_bytes, V, groups) + std::to_string(terms);
     for (const auto& kv : H->rings)
         if (kv.first == key) return kv.second;
     BlockSrc src;

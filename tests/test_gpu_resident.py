@@ -175,6 +175,28 @@ def test_conductivity_fixtures(handle, what):
     H.close()
 
 
+@pytest.mark.parametrize("prec,other", [("fp64", "fp32"), ("fp32", "fp64")])
+@pytest.mark.parametrize("K", [1, 3])
+def test_layout_queries_in_the_other_precision(handle, prec, other, K):
+    """What a run would look like in the other precision does not change what
+    runs: odd state counts have the same groups in both."""
+    s, (ip, ix, dt) = _sample(31, 24)
+    order, tiles = s.tile_order(1.3, return_tiles=True)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, dt, precision=prec, handle=handle, order=order,
+                         tiles=tiles)
+    bes = np.array([float(x) for x in tbpm.bessel_series(math.pi, 1e-30)[:21]])
+    psi = _states(s.num_orb, K)
+    handle.set_resident(True)
+    for query in (H.blocking_info, H.blocking_launch, H.blocking_bytes):
+        theirs, ours = query(K, other), query(K)
+        assert theirs and ours
+    got = tbpm.corr_dos(H, bes, psi, 6, chk_thr=1e-4)
+    handle.set_resident(False)
+    handle.set_blocking(False)
+    assert np.max(np.abs(got - tbpm.corr_dos(H, bes, psi, 6, chk_thr=1e-4))) < 1e-13
+    H.close()
+
+
 def test_graph_replay_and_timing(handle):
     """Replayed steps equal launched ones; the step counter and the norm
     check work with resident passes."""
