@@ -344,8 +344,9 @@ def counter_traffic(workload, kernel):
 
 
 def passes_terms(shape):
-    """Terms per pass of a tuner shape (1: one term per pass)."""
-    return max(1, int(shape[2])) if len(shape) > 2 else 1
+    """Terms per pass of a tuner shape (1: one term per pass; 32: resident
+    passes, whatever tile passes stand in for them)."""
+    return max(1, min(32, int(shape[2]))) if len(shape) > 2 else 1
 
 
 def passes_name(shape):

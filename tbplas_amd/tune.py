@@ -4,9 +4,10 @@ For a prepared Hamiltonian, a state count and a precision it times a few
 Chebyshev steps (HIP events on the library stream, after warm-up steps) for
 every candidate (persistent blocks per CU, LDS staging of the slice rows)
 and keeps the fastest; for a Hamiltonian with spatial tiles it then times
-the best shape with three, four and five terms per pass and keeps the
-fastest.  A shape is (blocks per CU, staging, terms per pass: 1, 3, 4 or
-5).
+the best shape with three, four and five terms per pass and with resident
+passes and keeps the fastest.  A shape is (blocks per CU, staging, terms per
+pass: 1, 3, 4, 5, or RESIDENT plus the terms per pass of runs whose tables do
+not fit resident passes; RESIDENT alone: five).
 Results are cached per (device name, library build, instances, rows, stored
 elements, widest slice, value layout, row order and tile count, states,
 precision) in memory and in a JSON file
@@ -26,7 +27,8 @@ CANDIDATES = [(bpc, stage) for bpc in (4, 8, 12, 16) for stage in (True, False)]
 # untuned: blocks per CU and staging; the terms per pass are those the
 # tiles of auto_tile_nm are sized for (sample.pass_terms)
 DEFAULT = (16, True)
-# "terms per pass" of a shape that runs resident passes (up to a whole step)
+# added to the terms per pass of a shape that runs resident passes (up to a
+# whole step)
 RESIDENT = 32
 
 _lock = threading.Lock()
@@ -78,7 +80,7 @@ def _key(hams, K):
 
 
 def autotune(H, K, bes, steps=6, warmup=2, candidates=None, use_cache=True):
-    """Pick (blocks_per_cu, stage, three terms per pass) for Hamiltonian H
+    """Pick (blocks_per_cu, stage, terms per pass) for Hamiltonian H
     (or a list of Hamiltonians run as one batch) and K states each; returns
     (best, timings) and leaves the handle set to the best shape."""
     from .tbpm import DosRun
@@ -131,19 +133,21 @@ def autotune(H, K, bes, steps=6, warmup=2, candidates=None, use_cache=True):
 def _set(handle, shape):
     handle.set_tuning(shape[0], shape[1])
     terms = int(shape[2])
-    handle.set_blocking(terms > 1, terms=5 if terms == RESIDENT else max(terms, 3))
-    handle.set_resident(terms == RESIDENT)
+    resident = terms >= RESIDENT
+    if resident:
+        terms = terms - RESIDENT or 5
+    handle.set_blocking(terms > 1, terms=max(terms, 3))
+    handle.set_resident(resident)
 
 
 def apply(H, K, bes, enabled=True):
-    """Tune when enabled, otherwise use the default shape (H: one
-    Hamiltonian or the list of a batch)."""
+    """Tune when enabled, otherwise use the default shape: resident passes
+    (H: one Hamiltonian or the list of a batch).  Returns the shape."""
     if enabled:
         return autotune(H, K, bes)[0]
     from .sample import pass_terms
     H0 = H[0] if isinstance(H, (list, tuple)) else H
     prec = "fp32" if H0.precision == _lib.TBG_FP32 else "fp64"
-    shape = DEFAULT + (pass_terms(K, prec),)
+    shape = DEFAULT + (RESIDENT + pass_terms(K, prec),)
     _set(H0.handle, shape)
-    H0.handle.set_resident(True)
     return shape
