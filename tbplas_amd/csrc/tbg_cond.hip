@@ -704,14 +704,18 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     launch_pack<R>(psi0, K, n, psi.p, e.lay, 0, H->perm_ptr(), st);
     launch_pack<R>(psi0, K, n, e.X.p, e.lay, 0, H->perm_ptr(), st);
     launch_pack<R>(psi0, K, n, e.X.p, e.lay, K, H->perm_ptr(), st);
-    // the kept states leave room for the quasi-eigenstates, Y and the sums
+    const QLay ql = q_layout(e.lay, K, n_pad);
+    const bool pairs = sizeof(R) == 4 && ql.lin && ql.lay.sh == 1;
+    const int VU = pairs ? 2 : 1;
+    DcSplit ds{};
+    // the kept states leave room for all that follows
     if (nq > 0) {
+        ds = dc_split(K, VU, n_en, n_pad, h->num_cus);
+        const size_t rest = dc_bytes(ds, K, VU, n_en, n_pad, T, e.plan.nchunks);
         size_t room = 0, total = 0;
         TBG_HIP(hipMemGetInfo(&room, &total));
-        const size_t rest = (size_t)n_pad * nq * 3 * sizeof(double2) + ((size_t)1 << 29);
         e.keep_history(T, room > rest ? (room - rest) / 2 : 0, h->kept_steps);
     }
-    const QLay ql = q_layout(e.lay, K, n_pad);
     uint64_t bwd = 0;
     for (int k = K; k < 2 * K; ++k) bwd |= 1ull << k;
     const unsigned nbm = nblk(n_pad * K), ny = (unsigned)std::min(n_en, 32768),
@@ -853,14 +857,8 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     const int64_t nq2 = 2 * nq;
     DevBuf cbuf((size_t)std::max<int64_t>(T * nq2 * 2, 1) * sizeof(double));
     TBG_HIP(hipMemsetAsync(counter.p, 0, sizeof(int), st));
-    const bool pairs = sizeof(R) == 4 && ql.lin && ql.lay.sh == 1;
-    const int VU = pairs ? 2 : 1;
-    DcSplit ds{};
     DevBuf dpart;
-    if (nq2 > 0) {
-        ds = dc_split(K, VU, n_en, n_pad, h->num_cus);
-        dpart.alloc((size_t)ds.nz * ds.tiles * VU * 256 * sizeof(double2));
-    }
+    if (nq2 > 0) dpart.alloc((size_t)ds.nz * ds.tiles * VU * 256 * sizeof(double2));
     auto correlate = [&](int count) {
         const DcStates xs = kept(count);
         for (int e0 = 0; e0 < n_en; e0 += ds.ne) {

@@ -2,6 +2,7 @@
 // waves (host arithmetic only, no HIP).
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include <algorithm>
@@ -32,6 +33,17 @@ inline DcSplit dc_split(int K, int VU, int n_en, int64_t n_pad, int num_cus) {
     d.split = std::max<int64_t>(64, ((n_pad + want - 1) / want + 63) / 64 * 64);
     d.nz = ((n_pad + d.split - 1) / d.split + 31) / 32 * 32;
     return d;
+}
+
+// Device bytes that a DC run allocates after it has chosen how many states it
+// keeps: the quasi-eigenstates and their two currents, the phase table, the
+// partial sums of their norms (`chunks` rows) and of the correlations, and
+// these themselves; 64 MB for what is small.
+inline size_t dc_bytes(const DcSplit& d, int K, int VU, int n_en, int64_t n_pad, int T,
+                       int chunks) {
+    const size_t nq = (size_t)n_en * K;
+    return 16 * (size_t)n_pad * nq * 3 + 16 * (size_t)T * (n_en + 15) + 24 * (size_t)chunks * nq +
+           4096 * (size_t)d.nz * d.tiles * VU + 32 * (size_t)T * nq + ((size_t)64 << 20);
 }
 
 }  // namespace tbg

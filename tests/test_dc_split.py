@@ -48,6 +48,11 @@ int main() {
                     }
             }
     std::printf("%ld\n", n);
+    // 8 complex128 states, 4097 energies, 8192 steps, 130,000 rows: the sums
+    // take more than half a GiB beside the energies' vectors
+    const tbg::DcSplit d = tbg::dc_split(8, 1, 4097, 130048, 256);
+    std::printf("%zu %lld %d\n", tbg::dc_bytes(d, 8, 1, 4097, 130048, 8192, 508), (long long)d.nz,
+                d.tiles);
 }
 """
 
@@ -61,4 +66,11 @@ def test_every_energy_and_row_is_covered(tmp_path):
                    check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
-    assert int(r.stdout) > 10000
+    first, second = r.stdout.splitlines()
+    assert int(first) > 10000
+    total, nz, tiles = (int(x) for x in second.split())
+    nq = 8 * 4097
+    vectors = 3 * 130048 * nq * 16
+    sums = 508 * nq * 3 * 8 + nz * tiles * 256 * 16 + 8192 * 2 * nq * 16 + 8192 * 4112 * 16
+    assert sums > 2 ** 29
+    assert 0 <= total - vectors - sums < 2 ** 27
