@@ -779,22 +779,27 @@ void corr_dc_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
     };
     auto qe_update = [&](int count) {
         const DcStates xs = kept(count);
+        // (y: the energies of a launch whose grid stays within 65535)
+        for (int y = 0; y < nec; y += 32768) {
+            const dim3 grid(nbm, (unsigned)std::min(nec - y, 32768));
+            const int e0 = y * ec;
 #define TBG_QE(LIN, EC)                                                                     \
-    hipLaunchKernelGGL((k_qe<R, LIN, EC>), dim3(nbm, (unsigned)nec),                         \
-                       dim3(256), 0, st, xs, count, e.lay, K, n_pad, ql, qe.as<double2>(),   \
-                       n_en, pitch, dptab.as<double2>(), counter.as<int>())
-        timed_launch(h, kTimeQe, [&] {
-            if (ql.lin) {
-                if (ec == 2) TBG_QE(true, 2);
-                else if (ec == 8) TBG_QE(true, 8);
-                else TBG_QE(true, 16);
-            } else {
-                if (ec == 2) TBG_QE(false, 2);
-                else if (ec == 8) TBG_QE(false, 8);
-                else TBG_QE(false, 16);
-            }
-            TBG_HIP(hipGetLastError());
-        });
+    hipLaunchKernelGGL((k_qe<R, LIN, EC>), grid, dim3(256), 0, st, xs, count, e.lay, K, n_pad, \
+                       ql, qe.as<double2>() + e0 * ql.stride, n_en - e0, pitch,              \
+                       dptab.as<double2>() + e0, counter.as<int>())
+            timed_launch(h, kTimeQe, [&] {
+                if (ql.lin) {
+                    if (ec == 2) TBG_QE(true, 2);
+                    else if (ec == 8) TBG_QE(true, 8);
+                    else TBG_QE(true, 16);
+                } else {
+                    if (ec == 2) TBG_QE(false, 2);
+                    else if (ec == 8) TBG_QE(false, 8);
+                    else TBG_QE(false, 16);
+                }
+                TBG_HIP(hipGetLastError());
+            });
+        }
 #undef TBG_QE
     };
     auto after1 = [&]() {

@@ -252,6 +252,24 @@ def test_dc_step_blocks_vs_oracle(handle, prec, tol, resident, T, n_en, K):
     H.close()
 
 
+def test_dc_more_energies_than_grid_rows(handle):
+    """1,050,000 energies are 65,625 groups of 16, more than a grid's 65,535
+    rows: the same numbers over and over (1e-12 of the largest: sums of 64
+    rows in another grouping)."""
+    s, _ = _sample(4, 8, vac=0.0)
+    ip, ix, hop, dx, dy = oracle.build_ham_dxy_loop(s.orb_eng, s.hop_i, s.hop_j, s.hop_v, s.dr)
+    bes = tbpm.bessel_series(tau_of(s), 1e-14)
+    psi = _states(s.num_orb, 1)
+    en = np.linspace(-2.6, 2.6, 16)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, hop, dx, dy, cur_scale=9.0, precision="fp64",
+                         handle=handle)
+    few = tbpm.corr_dc(H, bes, psi, 2, 2 * math.pi / 18.0, en, np.arange(16))[1]
+    many = tbpm.corr_dc(H, bes, psi, 2, 2 * math.pi / 18.0, en, np.arange(1_050_000) % 16)[1]
+    many = many.reshape(1, 2, -1, 16, 2)
+    assert np.max(np.abs(many - few[:, :, None])) < 1e-12 * max(1.0, np.max(np.abs(few)))
+    H.close()
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("resident", [True, False])
 @pytest.mark.parametrize("T", [7, 16, 37])
