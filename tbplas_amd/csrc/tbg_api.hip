@@ -129,13 +129,14 @@ static std::shared_ptr<Ring> batch_ring(tbg_handle* h, int ni, const tbg_ham* co
     const int Kp = slots_for(K), V = ring_vectors<R>(Kp);
     std::string key = ring_key((int)sizeof(R), V, Kp / V) + std::to_string(terms);
     for (int i = 0; i < ni; ++i) key += "|" + std::to_string(hams[i]->uid);
-    for (const auto& kv : h->batch_ring)
-        if (kv.first == key) return kv.second;
+    if (auto t = h->batch_ring.find(key))
+        if (!t->gone()) return t->ring();
     std::vector<std::vector<int64_t>> segs;
     const BlockSrc src = batch_src<R>(ni, hams, cat, inst_slices, segs);
     auto B = build_ring(h, src, segs, (int)sizeof(R), V, Kp / V, terms, cat.real_vals != 0);
-    h->batch_ring.emplace_back(key, B);
-    if (h->batch_ring.size() > 4) h->batch_ring.erase(h->batch_ring.begin());
+    // (a thirty-second of the memory: 9 GB, the tables of about 100M orbitals)
+    auto t = h->batch_ring.add(key, B, B ? B->bytes() : 0, h->memory / 32);
+    for (int i = 0; i < ni; ++i) hams[i]->batches.join(t);
     return B;
 }
 
@@ -383,6 +384,7 @@ int tbg_create(tbg_handle** out, int device) {
         TBG_HIP(hipGetDeviceProperties(&prop, device));
         h->num_cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
         h->max_lds = prop.sharedMemPerBlock > 0 ? (int)prop.sharedMemPerBlock : 65536;
+        h->memory = prop.totalGlobalMem;
         prepare_term3(h->max_lds);
         prepare_ring(h->max_lds);
         static_scratch_init(device);   // the allocation-free entry point's array

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/tbplas_amd.h"
+#include "tbg_batch_cache.h"
 
 namespace tbg {
 
@@ -125,12 +126,13 @@ struct tbg_handle {
     int block_rows = 0;       // cap on rows owned per workgroup (0: from LDS)
     int kept_steps = 16;      // states that a DC run may keep (tbg_set_kept_steps)
     int max_lds = 65536;      // LDS bytes one workgroup may use
+    size_t memory = 0;        // bytes of the device
     tbg::DevBuf scratch;      // reduction partials and small tables
     tbg::DevBuf counter;      // step counter for graph-replayed reductions
     // three-term tables of recent batches (key: state row bytes, limits and
     // the instances' ids); a null entry records tiles that do not fit
     std::vector<std::pair<std::string, std::shared_ptr<tbg::Blocking>>> batch_blk;
-    std::vector<std::pair<std::string, std::shared_ptr<tbg::Ring>>> batch_ring;   // the last four
+    tbg::BatchCache batch_ring;   // resident-pass tables of batches
     // Per-launch timing (tbg_set_kernel_timing): a pair of events around
     // every propagation and correlation launch, tagged with the launch kind
     // (tbg_kernel_times sums them); events are reused from ev_pool.
@@ -224,5 +226,6 @@ struct tbg_ham {
     mutable int blk_depth = 0;
     // tables of resident passes (tbg_ring.hip), the last two used
     mutable std::vector<std::pair<std::string, std::shared_ptr<tbg::Ring>>> rings;
+    mutable tbg::BatchShares batches;   // and those of batches it is in
     uint64_t uid = 0;         // unique per Hamiltonian created in the process
 };

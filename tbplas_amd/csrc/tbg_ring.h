@@ -61,6 +61,9 @@ struct Ring {
     // rows computed in the first term, rows owned
     int64_t sched[4] = {0, 0, 0, 0};
     DevBuf meta, ends, rows, idx, vals;
+    size_t bytes() const {
+        return meta.bytes + ends.bytes + rows.bytes + idx.bytes + vals.bytes;
+    }
 };
 
 // Vectors per lane (states of one workgroup) for Kp slots: 16-byte units

@@ -150,6 +150,37 @@ def test_batch(handle, prec, K):
         H.close()
 
 
+def test_batch_tables_go_with_the_hamiltonians(gpu, handle):
+    """Closing a batch's Hamiltonians gives its tables back (some 16 MB for
+    the 183,000 orbitals here; the pages of other allocations may stay)."""
+    s, csr = _sample(214, 214, vac=0.0)
+    order, tiles = s.tile_order(2.4, return_tiles=True)
+    bes, psi = tbpm.bessel_series(tau_of(s), 1e-15), _states(s.num_orb, 1)
+    handle.set_resident(True)
+
+    def free():
+        gpu.cuda.synchronize()
+        gpu.cuda.empty_cache()
+        return gpu.cuda.mem_get_info()[0]
+
+    def batch():
+        hams = [tbpm.Hamiltonian(s.num_orb, *csr, precision="fp64", handle=handle, order=order,
+                                 tiles=tiles) for _ in range(2)]
+        out = tbpm.corr_dos_batch(hams, bes, [psi, psi], 4)
+        with_tables = free()
+        for H in hams:
+            H.close()
+        return out, with_tables
+
+    first, _ = batch()
+    before = free()
+    for _ in range(3):
+        out, with_tables = batch()
+        np.testing.assert_array_equal(out, first)
+    assert with_tables < before - 16e6
+    assert free() >= before - 4e6
+
+
 @pytest.mark.parametrize("what", ["ac", "dc"])
 def test_conductivity_fixtures(handle, what):
     """The reference's AC and DC correlations on its own states."""
