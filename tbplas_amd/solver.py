@@ -136,6 +136,11 @@ class Solver:
             yield i, min(total, i + per)
             i += per
 
+    @staticmethod
+    def _all_steps(steps, total, per):
+        """Time steps of the runs over `total` samples, `per` at a time."""
+        return steps * -(-total // per)
+
     def _row_order(self, gpu, key, vectors=1, rule=auto_tile_nm):
         """(row order, tile offsets) of square tiles of gpu[key] nm ('auto':
         sized by `rule`, ``auto_tile_nm`` or ``ac_tile_nm``, for `vectors`
@@ -179,7 +184,8 @@ class Solver:
         psi0 = self._states(num_sample)
         chk, thr = self._chk()
         T = self._config.generic["nr_time_steps"]
-        tune.apply(H, min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(T, num_sample, per))
         corr = np.zeros(T + 1, dtype=np.complex128)
         for a, b in self._batches(num_sample, per):
             c = corr_dos(H, bes, psi0[a:b], T, chk, thr)
@@ -208,7 +214,8 @@ class Solver:
         psi0 = ldos_states(self._states(num_sample), self._config.LDOS["site_indices"])
         chk, thr = self._chk()
         T = self._config.generic["nr_time_steps"]
-        tune.apply(H, min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(T, num_sample, per))
         corr = np.zeros(T + 1, dtype=np.complex128)
         for a, b in self._batches(num_sample, per):
             c = corr_ldos(H, bes, psi0[a:b], T, chk, thr)
@@ -260,7 +267,8 @@ class Solver:
         psi0 = self._states(num_sample)
         chk, thr = self._chk()
         T = self._config.generic["nr_time_steps"]
-        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(T, num_sample, per))
         out = np.zeros((len(energies), self._sample.num_orb), dtype=np.float64)
         for a, b in self._batches(num_sample, per):
             q = quasi_eigenstates(H, bes, psi0[a:b], T, time_step, energies, chk, thr)
@@ -361,7 +369,8 @@ class Solver:
         psi0 = self._states(num_sample)
         chk, thr = self._chk()
         T = g["nr_time_steps"]
-        tune.apply(H, 3 * min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, 3 * min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(T, num_sample, per))
         corr = np.zeros((4, T), dtype=np.complex128)
         for a, b in self._batches(num_sample, per):
             c = corr_ac(H, bes, coef_F, coef_omF, psi0[a:b], T, chk, thr)
@@ -397,7 +406,8 @@ class Solver:
         chk, thr = self._chk()
         T = g["nr_time_steps"]
         per = max(1, min(32, int(gpu["max_vectors"])))
-        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(T * len(q_points), num_sample, per))
         corr = np.zeros((len(q_points), T), dtype=np.float64)
         for a, b in self._batches(num_sample, per):
             c = corr_dyn_pol(H, bes, coef_F, coef_omF, psi0[a:b], T, q_points, pos, chk, thr)
@@ -432,7 +442,8 @@ class Solver:
                         handle=h, order=order, tiles=tiles)
         psi0 = self._states(num_sample)
         chk, thr = self._chk()
-        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"])
+        tune.apply(H, 2 * min(per, num_sample), bes, gpu["autotune"],
+                   self._all_steps(2 * tnr, num_sample, per))
         corr_dos_ = np.zeros(tnr, dtype=np.complex128)
         corr_dc_ = np.zeros((2, len(energies_dos), tnr), dtype=np.complex128)
         n_en = len(qe_indices)

@@ -140,14 +140,33 @@ def _set(handle, shape):
     handle.set_resident(resident)
 
 
-def apply(H, K, bes, enabled=True):
+def _few_steps(n, K, prec, steps):
+    """Whether so few steps on a new Hamiltonian of n rows do not pay for the
+    tables of resident passes.  Below some 70,000 rows these take longer to
+    make than the tiles' (ms, one complex128 state: 0.8 / 0.3 at 2,100 rows,
+    1.7 / 0.5 at 8,300, 3.3 / 1.4 at 33,000; 5.5 / 5.4 at 131,600, and less
+    from there on), and a step gains 8 to 20 us.  Steps after which they are
+    even: 71, 116, 201 there, 60 to 245 for one complex64 state, 41 to 171
+    for four; 20 to 60 with more than 32 bytes a row (114 once), AC and DC
+    runs 10 to 90."""
+    from .sample import _row_bytes
+    return n < 70_000 and steps < (150 if _row_bytes(K, prec) <= 32 else 50)
+
+
+def apply(H, K, bes, enabled=True, steps=None):
     """Tune when enabled, otherwise use the default shape: resident passes
-    (H: one Hamiltonian or the list of a batch).  Returns the shape."""
-    if enabled:
-        return autotune(H, K, bes)[0]
+    (H: one Hamiltonian or the list of a batch).  With `steps`, the time
+    steps of all runs that H was made for, tile passes where these are too
+    few for the tables of resident passes.  Returns the shape."""
     from .sample import pass_terms
-    H0 = H[0] if isinstance(H, (list, tuple)) else H
-    prec = "fp32" if H0.precision == _lib.TBG_FP32 else "fp64"
-    shape = DEFAULT + (RESIDENT + pass_terms(K, prec),)
-    _set(H0.handle, shape)
+    hams = list(H) if isinstance(H, (list, tuple)) else [H]
+    prec = "fp32" if hams[0].precision == _lib.TBG_FP32 else "fp64"
+    if enabled:
+        shape = autotune(H, K, bes)[0]
+    else:
+        shape = DEFAULT + (RESIDENT + pass_terms(K, prec),)
+    if shape[2] >= RESIDENT and steps is not None and \
+            _few_steps(sum(Hi.n for Hi in hams), K, prec, steps):
+        shape = tuple(shape[:2]) + (shape[2] - RESIDENT or 5,)
+    _set(hams[0].handle, shape)
     return shape

@@ -115,3 +115,20 @@ def test_solver_norm_error_instead_of_stop(gpu, tmp_path):
     from tbplas_amd._lib import NormError
     with pytest.raises(NormError):
         solver.calc_corr_dos()
+
+
+@pytest.mark.parametrize("kind,factor", [("dos", 1), ("ac_cond", 1), ("dc_cond", 2)])
+def test_solver_states_the_steps_of_its_runs(gpu, tmp_path, monkeypatch, kind, factor):
+    """Three samples, two at a time: two runs (a DC run propagates twice)."""
+    from tbplas_amd import tune
+    seen, apply = [], tune.apply
+    monkeypatch.setattr(tune, "apply",
+                        lambda H, K, bes, on, steps: seen.append(steps) or apply(H, K, bes, on, steps))
+    s = tb.make_graphene_sample(6)
+    s.rescale_ham(9.0)
+    cfg = _config(16, 3)
+    cfg.gpu["max_vectors"] = 2
+    cfg.DC_conductivity["energy_limits"] = (-0.3, 0.3)
+    solver = tb.Solver(s, cfg, directory=str(tmp_path / "sim"), prefix="t", echo_details=False)
+    getattr(solver, "calc_corr_" + kind)()
+    assert seen == [16 * 2 * factor]

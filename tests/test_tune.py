@@ -23,8 +23,8 @@ class Handle:
 
 
 class Ham:
-    def __init__(self, precision):
-        self.handle, self.precision = Handle(), precision
+    def __init__(self, precision, n=1000):
+        self.handle, self.precision, self.n = Handle(), precision, n
 
 
 @pytest.mark.parametrize("precision", [_lib.TBG_FP64, _lib.TBG_FP32])
@@ -48,3 +48,27 @@ def test_shapes(terms, state):
     tune._set(h, (8, False, terms))
     assert (h.state["terms"], h.state["resident"]) == state
     assert (h.state["blocks"], h.state["stage"]) == (8, False)
+
+
+@pytest.mark.parametrize("n,K,steps,resident", [
+    (8000, 1, 64, False), (8000, 1, 149, False), (8000, 1, 150, True), (8000, 2, 64, False),
+    (8000, 4, 64, True), (8000, 4, 49, False), (69999, 1, 1, False), (70000, 1, 1, True),
+    (8000, 1, None, True), (2_000_000, 8, 1, True)])
+@pytest.mark.parametrize("tuned", [False, True])
+def test_few_steps_on_a_small_sample_take_tile_passes(n, K, steps, resident, tuned, monkeypatch):
+    """The tables of resident passes take longer than such a run gains, with
+    a shape from the tuner as well; a batch counts as a whole."""
+    monkeypatch.setattr(tune, "autotune", lambda H, K, bes: ((8, True, tune.RESIDENT), None))
+    for hams in (Ham(_lib.TBG_FP64, n), [Ham(_lib.TBG_FP64, n // 2), Ham(_lib.TBG_FP64, n - n // 2)]):
+        H0 = hams[0] if isinstance(hams, list) else hams
+        shape = tune.apply(hams, K, np.ones(5), tuned, steps)
+        assert H0.handle.state["resident"] == resident
+        assert H0.handle.state["terms"] == 5
+        assert (shape[2] >= tune.RESIDENT) == resident
+
+
+def test_a_shape_without_resident_passes_stays(monkeypatch):
+    monkeypatch.setattr(tune, "autotune", lambda H, K, bes: ((8, True, 1), None))
+    H = Ham(_lib.TBG_FP64)
+    assert tune.apply(H, 1, np.ones(5), True, 3) == (8, True, 1)
+    assert H.handle.state["terms"] == 0
