@@ -379,8 +379,13 @@ void hall_mu_impl(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, in
         }
         return best;
     };
-    const int64_t max_split = std::max(split_of(B), split_of(N % B ? N % B : B));
-    DevBuf gpart((size_t)max_split * B * N * sizeof(double2));
+    // The partial sums of as many splits (of B rows; a last block of fewer
+    // rows has more) as the vectors leave memory for: 200 MB at the size
+    // above, 4 GB for 20,000 moments.
+    const int tail = N % B ? N % B : B;
+    const int64_t units = std::max(split_of(B), (split_of(tail) * tail + B - 1) / B);
+    DevBuf gpart;
+    const int64_t gcols = alloc_units(gpart, (size_t)B * N * sizeof(double2), units) * B;
     for (int s = 0; s < K; ++s) {
         double2* cur = T0.as<double2>();   // T_j
         double2* oth = T1.as<double2>();   // T_{j-1}; T_{j+1} is formed in place over it
@@ -407,7 +412,7 @@ void hall_mu_impl(tbg_handle* h, const tbg_ham* H, const double* psi0, int K, in
             p1 = pi;
             if (i % B == B - 1 || i == N - 1) {
                 const int i0 = i - i % B, rows = i % B + 1;
-                const int64_t want = split_of(rows);
+                const int64_t want = std::min(split_of(rows), gcols / rows);
                 const int64_t kchunk = ((np + want - 1) / want + kGramK - 1) / kGramK * kGramK;
                 const int64_t nsplit = (np + kchunk - 1) / kchunk;
                 const dim3 grid((unsigned)(nsplit * ((N + kGramN - 1) / kGramN) *

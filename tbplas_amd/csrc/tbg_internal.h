@@ -96,6 +96,19 @@ struct DevBuf {
     template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// As many of `most` units of b bytes as there is memory for, by halves, one
+// at least: scratch that is worth having but not what a run must have.
+inline int64_t alloc_units(DevBuf& d, size_t b, int64_t most) {
+    for (;; most = (most + 1) / 2) {
+        try {
+            d.alloc(b * (size_t)most);
+            return most;
+        } catch (const Error& e) {
+            if (e.code != TBG_EOOM || most <= 1) throw;
+        }
+    }
+}
+
 // Complex storage type of a working precision.
 template <typename R> struct CplxT;
 template <> struct CplxT<float> { using T = float2; };

@@ -1,13 +1,13 @@
-"""The states a DC run keeps, as many as memory gives: Engine::keep_history
-on the CPU, compiled against a stand-in for the HIP runtime whose allocations
-fail beyond a budget and leave their error for the next check, as HIP does."""
+"""Device memory that a run can do with less of, on the CPU: compiled against
+a stand-in for the HIP runtime whose allocations fail beyond a budget and
+leave their error for the next check, as HIP does."""
 import subprocess
 
 import pytest
 
 from tbplas_amd import build
 
-CODE = r"""
+STAND_IN = r"""
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -40,6 +40,9 @@ hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 namespace tbg {
 void launch_fill_zero(void*, size_t, hipStream_t) { TBG_HIP(hipGetLastError()); }
 }
+"""
+
+KEPT = r"""
 int main(int, char** v) {
     const int free_buffers = std::atoi(v[1]), steps = std::atoi(v[2]), room = std::atoi(v[3]),
               most = std::atoi(v[4]);
@@ -61,16 +64,39 @@ int main(int, char** v) {
 }
 """
 
+UNITS = r"""
+int main() {
+    for (size_t have = 0; have < 40; ++have)
+        for (int most = 1; most <= 24; ++most) {
+            budget = have * 10;
+            int64_t want = most;           // by halves, rounded up
+            while (want > 1 && (size_t)want > have) want = (want + 1) / 2;
+            tbg::DevBuf d;
+            try {
+                const int64_t got = tbg::alloc_units(d, 10, most);
+                if (have == 0 || got != want || d.bytes != 10 * (size_t)got || used != d.bytes)
+                    return 1;
+            } catch (const tbg::Error& e) {
+                if (have > 0 || e.code != TBG_EOOM || used != 0) return 2;
+            }
+            if (hipGetLastError() != hipSuccess) return 3;
+        }
+}
+"""
 
-@pytest.fixture(scope="module")
-def exe(tmp_path_factory):
-    d = tmp_path_factory.mktemp("kept")
+
+def _compile(main, d):
     src, out = d / "t.cpp", d / "t"
-    src.write_text(CODE)
+    src.write_text(STAND_IN + main)
     subprocess.run(["g++", "-std=c++17", "-O0", "-w", "-D__HIP_PLATFORM_AMD__",
                     "-I/opt/rocm/include", "-I", build.CSRC, str(src), "-o", str(out)],
                    check=True)
     return str(out)
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    return _compile(KEPT, tmp_path_factory.mktemp("kept"))
 
 
 @pytest.mark.parametrize("free,steps,room,most,kept", [
@@ -81,8 +107,14 @@ def exe(tmp_path_factory):
     (15, 500, 99, 16, 16), (14, 500, 99, 16, 8), (6, 500, 99, 16, 4), (2, 500, 99, 16, 2),
     (1, 500, 99, 16, 2), (0, 500, 99, 16, 1)])
 def test_as_many_states_as_memory_gives(exe, free, steps, room, most, kept):
-    """kept - 2 buffers beside the two of the engine, and a spare one."""
+    """The states a DC run keeps (Engine::keep_history): kept - 2 buffers
+    beside the two of the engine, and a spare one."""
     r = subprocess.run([exe, str(free), str(steps), str(room), str(most)], capture_output=True,
                        text=True)
     assert r.returncode == 0, r.stdout
     assert r.stdout.split() == [str(kept), str(kept + 1 if kept > 1 else 2)]
+
+
+def test_scratch_by_halves(tmp_path):
+    r = subprocess.run([_compile(UNITS, tmp_path)])
+    assert r.returncode == 0
