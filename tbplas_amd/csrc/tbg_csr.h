@@ -5,6 +5,32 @@
 
 namespace tbg {
 
+// One allocation for a builder call's scratch arrays: nine pairs of hipMalloc
+// and hipFree, each a wait for the device, took 3 of the 19 ms of assembling
+// 2M orbitals twice.  What does not fit is allocated by itself, and all of
+// them are where there is no memory for them at once (one by one they are
+// freed as soon as they are done with: 12 bytes an orbital less at the most).
+struct Scratch {
+    DevBuf all;
+    size_t used = 0;
+    explicit Scratch(size_t bytes) {
+        try {
+            all.alloc(bytes);
+        } catch (const Error& e) {
+            if (e.code != TBG_EOOM) throw;
+        }
+    }
+    void give(DevBuf& d, size_t bytes) {
+        const size_t at = (used + 255) / 256 * 256;
+        if (!all.p || at + bytes > all.bytes) {
+            d.alloc(bytes);
+            return;
+        }
+        d.borrow(all.as<unsigned char>() + at, bytes);
+        used = at + bytes;
+    }
+};
+
 void scan_i64(tbg_handle* h, const int64_t* in, int64_t n, int64_t* out, bool exclusive,
               DevBuf& tmp);
 

@@ -311,24 +311,6 @@ __global__ void k_check_hops(int64_t m, const int64_t* hop_i, const int64_t* hop
         atomicOr(bad, 1);
 }
 
-// One allocation for a builder call's scratch arrays: nine pairs of hipMalloc
-// and hipFree, each a wait for the device, took 3 of the 19 ms of assembling
-// 2M orbitals twice.  What does not fit is allocated by itself.
-struct Scratch {
-    DevBuf all;
-    size_t used = 0;
-    explicit Scratch(size_t bytes) : all(bytes) {}
-    void give(DevBuf& d, size_t bytes) {
-        const size_t at = (used + 255) / 256 * 256;
-        if (at + bytes > all.bytes) {
-            d.alloc(bytes);
-            return;
-        }
-        d.borrow(all.as<unsigned char>() + at, bytes);
-        used = at + bytes;
-    }
-};
-
 // n + 1 counts or offsets, `rows` times, the scan's sums, flags and cursors
 static size_t scratch_bytes(int64_t n, int rows) {
     return (size_t)(n + 1) * (8 * rows + 4) + (size_t)(n / kScanTile + 2) * 8 +

@@ -64,6 +64,42 @@ int main(int, char** v) {
 }
 """
 
+SCRATCH = r"""
+#include "tbg_csr.h"
+int main() {
+    budget = 1000;
+    {
+        tbg::Scratch w(900);               // at once, and what is beyond it
+        tbg::DevBuf a, b, c;
+        w.give(a, 100);
+        w.give(b, 300);
+        if (used != 900 || a.owned || b.owned || (char*)b.p != (char*)a.p + 256) return 1;
+        w.give(c, 90);
+        if (!a.p || used != 900) return 2;
+        tbg::DevBuf d;
+        try {
+            w.give(d, 400);
+            return 3;
+        } catch (const tbg::Error& e) {
+            if (e.code != TBG_EOOM) return 4;
+        }
+    }
+    if (used != 0) return 5;
+    {
+        tbg::Scratch w(1200);              // 700 of it are needed at a time
+        tbg::DevBuf a;
+        w.give(a, 200);
+        for (int i = 0; i < 2; ++i) {
+            tbg::DevBuf b;
+            w.give(b, 500);
+            if (used != 700) return 6;
+        }
+        if (hipGetLastError() != hipSuccess) return 7;
+    }
+    return used == 0 ? 0 : 8;
+}
+"""
+
 UNITS = r"""
 int main() {
     for (size_t have = 0; have < 40; ++have)
@@ -113,6 +149,11 @@ def test_as_many_states_as_memory_gives(exe, free, steps, room, most, kept):
                        text=True)
     assert r.returncode == 0, r.stdout
     assert r.stdout.split() == [str(kept), str(kept + 1 if kept > 1 else 2)]
+
+
+def test_scratch_at_once_or_one_by_one(tmp_path):
+    r = subprocess.run([_compile(SCRATCH, tmp_path)])
+    assert r.returncode == 0
 
 
 def test_scratch_by_halves(tmp_path):
