@@ -133,7 +133,11 @@ static std::shared_ptr<Ring> batch_ring(tbg_handle* h, int ni, const tbg_ham* co
         if (!t->gone()) return t->ring();
     std::vector<std::vector<int64_t>> segs;
     const BlockSrc src = batch_src<R>(ni, hams, cat, inst_slices, segs);
-    auto B = build_ring(h, src, segs, (int)sizeof(R), V, Kp / V, terms, cat.real_vals != 0);
+    std::shared_ptr<Ring> B;
+    if (!with_memory([&] {
+            B = build_ring(h, src, segs, (int)sizeof(R), V, Kp / V, terms, cat.real_vals != 0);
+        }))
+        return nullptr;
     // (a thirty-second of the memory: 9 GB, the tables of about 100M orbitals)
     auto t = h->batch_ring.add(key, B, B ? B->bytes() : 0, h->memory / 32);
     for (int i = 0; i < ni; ++i) hams[i]->batches.join(t);

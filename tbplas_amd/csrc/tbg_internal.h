@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <memory>
+#include <new>
 #include <utility>
 #include <string>
 #include <vector>
@@ -107,6 +108,20 @@ inline int64_t alloc_units(DevBuf& d, size_t b, int64_t most) {
             if (e.code != TBG_EOOM || most <= 1) throw;
         }
     }
+}
+
+// Runs f; false where there is no memory, on the device or the host, for what
+// it makes.
+template <typename F>
+bool with_memory(F&& f) {
+    try {
+        f();
+        return true;
+    } catch (const Error& e) {
+        if (e.code != TBG_EOOM) throw;
+    } catch (const std::bad_alloc&) {
+    }
+    return false;
 }
 
 // Complex storage type of a working precision.

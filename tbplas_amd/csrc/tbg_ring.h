@@ -86,7 +86,8 @@ std::string ring_key(int real_bytes, int V, int groups);
 
 // The tables of H for groups of V states of real_bytes-byte reals (built on
 // first use, the last few kept on H), or null when the handle does not ask
-// for resident passes, H has no tiles, or no block fits.
+// for resident passes, H has no tiles, no block fits, or there is no memory
+// for the tables.
 std::shared_ptr<Ring> get_ring(tbg_handle* h, const tbg_ham* H, int real_bytes, int V, int groups,
                                int terms);
 

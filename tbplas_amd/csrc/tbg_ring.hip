@@ -560,15 +560,20 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     R->sched[1] = nrow;
     R->sched[2] = computed;
     R->sched[3] = covered;
-    auto up = [&](DevBuf& d, const void* p, size_t bytes) {
-        d.alloc(std::max<size_t>(bytes, 16));
-        if (bytes) TBG_HIP(hipMemcpyAsync(d.p, p, bytes, hipMemcpyHostToDevice, h->stream));
+    // (all the memory first: no copy is under way where there is none)
+    R->meta.alloc(meta.size() * sizeof(RingMeta));
+    R->ends.alloc(ends.size() * sizeof(int));
+    R->rows.alloc(rows.size() * sizeof(int));
+    R->idx.alloc(idx.size() * sizeof(uint16_t));
+    R->vals.alloc(vals.size());
+    auto up = [&](DevBuf& d, const void* p) {
+        TBG_HIP(hipMemcpyAsync(d.p, p, d.bytes, hipMemcpyHostToDevice, h->stream));
     };
-    up(R->meta, meta.data(), meta.size() * sizeof(RingMeta));
-    up(R->ends, ends.data(), ends.size() * sizeof(int));
-    up(R->rows, rows.data(), rows.size() * sizeof(int));
-    up(R->idx, idx.data(), idx.size() * sizeof(uint16_t));
-    up(R->vals, vals.data(), vals.size());
+    up(R->meta, meta.data());
+    up(R->ends, ends.data());
+    up(R->rows, rows.data());
+    up(R->idx, idx.data());
+    up(R->vals, vals.data());
     TBG_HIP(hipStreamSynchronize(h->stream));
     return R;
 }
@@ -594,7 +599,11 @@ std::shared_ptr<Ring> get_ring(tbg_handle* h, const tbg_ham* H, int real_bytes, 
     src.padded = H->padded;
     src.nrows = H->n;
     src.vsz = H->vals.bytes / (size_t)std::max<int64_t>(H->padded, 1);
-    auto R = build_ring(h, src, {H->tiles}, real_bytes, V, groups, terms, H->real_vals);
+    std::shared_ptr<Ring> R;
+    if (!with_memory([&] {
+            R = build_ring(h, src, {H->tiles}, real_bytes, V, groups, terms, H->real_vals);
+        }))
+        return nullptr;   // (tried again by the next run)
     H->rings.emplace_back(key, R);
     if (H->rings.size() > 2) H->rings.erase(H->rings.begin());
     return R;
