@@ -537,7 +537,8 @@ void corr_ac_impl(tbg_handle* h, const tbg_ham* H, const double* bes, int nb, co
                   nbuf.as<double>(), 0, counter.as<int>(), 0, st);
     const StepPoly sp = time_poly(bes, nb);
     const int64_t astride = (int64_t)e.plan.nchunks * 8 * K;
-    DevBuf apart((size_t)e.part_steps * astride * sizeof(double));
+    DevBuf apart;
+    e.part_steps = (int)alloc_units(apart, (size_t)astride * sizeof(double), e.part_steps);
     auto reduce_corr = [&](int steps) {
         if (steps > 0)
             launch_reduce(apart.as<double>(), 8 * K, e.plan.inst_chunk_dev.template as<int>(), 1,

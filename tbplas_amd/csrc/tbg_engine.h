@@ -181,15 +181,15 @@ struct Engine {
     }
 
     // The epilogue's partial sums of up to part_steps steps, kept apart until
-    // one launch adds them (keep_sums; 16 as a captured graph has steps).
+    // one launch adds them (keep_sums; 16 as a captured graph has steps, fewer
+    // where there is no memory for them).
     int part_steps = 1, part_at = 0;
     int64_t part_stride = 0;
     double* part_now() const { return part.template as<double>() + part_at * part_stride; }
     void keep_sums() {
         if (part.bytes > ((size_t)4 << 20)) return;   // (a step is long enough)
         part_stride = (int64_t)(part.bytes / sizeof(double));
-        part_steps = 16;
-        part.alloc((size_t)part_steps * part_stride * sizeof(double));
+        part_steps = (int)alloc_units(part, (size_t)part_stride * sizeof(double), 16);
     }
     // After a step that formed sums of nv values: adds them to row *counter
     // of out, at once or (add_rest) at the end of a run.

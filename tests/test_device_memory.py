@@ -152,6 +152,22 @@ int main() {
 }
 """
 
+SUMS = r"""
+int main() {
+    for (int have : {1, 2, 3, 7, 8, 15, 16, 40}) {
+        tbg_handle h;
+        tbg::Engine<double> e;
+        e.h = &h;
+        budget = 800 * (size_t)have;
+        e.part.alloc(800);
+        e.keep_sums();
+        const int want = have >= 16 ? 16 : have >= 8 ? 8 : have >= 4 ? 4 : have >= 2 ? 2 : 1;
+        if (e.part_steps != want || used != 800 * (size_t)want || e.part_stride != 100) return 1;
+        if (hipGetLastError() != hipSuccess) return 2;
+    }
+}
+"""
+
 UNITS = r"""
 int main() {
     for (size_t have = 0; have < 40; ++have)
@@ -212,6 +228,11 @@ def test_no_memory_for_resident_tables(tmp_path):
 
 def test_scratch_at_once_or_one_by_one(tmp_path):
     r = subprocess.run([_compile(SCRATCH, tmp_path)])
+    assert r.returncode == 0
+
+
+def test_sums_of_as_many_steps_as_memory_gives(tmp_path):
+    r = subprocess.run([_compile(SUMS, tmp_path)])
     assert r.returncode == 0
 
 
