@@ -18,7 +18,9 @@ resident in HBM, replayed from a hipGraph.  The one JSON line also holds
   * ``roofline``: the dominant kernel (largest share of the step's device
     time) from a segment of --profile-steps steps run right after the
     timed ones with HIP events around every launch on the library's stream:
-    its average launch duration and the bytes one launch must move (for the
+    its average launch duration and the bytes one launch must move (for a
+    resident pass: the block tables once, and of every row what the pass
+    reads and writes, without the halo, which L2 can serve; for the
     tile pass: the workgroup tables, the distinct rows of v_{m-1} its tiles
     gather, v_{m-2} on the tiles and their halo rings, and the output read
     plus written and the last two terms written on the owned rows, counted
@@ -26,9 +28,9 @@ resident in HBM, replayed from a hipGraph.  The one JSON line also holds
     8 TB/s.  ``traffic`` is the counter-measured L2-to-HBM bytes per launch
     (FETCH_SIZE and WRITE_SIZE, copy-calibrated) from profiles/traffic.json
     when that file was measured on the sources the workload's kernels are
-    built from and on the same tiles, else null.  ``one_term_equivalent`` restates the speed as one-term-per-pass
-    algorithmic bytes (five vector streams per state and H once per term)
-    per measured time per term;
+    built from and on the same tiles, else null.  ``one_term_equivalent``
+    restates the speed as one-term-per-pass algorithmic bytes (five vector
+    streams per state and H once per term) per measured time per term;
   * ``fp64_k8`` (the same 8 states in complex128, 3.4 nm tiles) and
     ``fp64_k1`` (one complex128 state, 7.5 nm tiles: the speedup
     denominator);
@@ -468,9 +470,11 @@ def timed_run(run, h, args, total):
     return ms, kt
 
 
-def pass_bytes_fn(sched, n, nnz, K, s, real):
+def pass_bytes_fn(sched, n, nnz, K, s, real, psi0=1.0):
     """bytes_of for propagation launches: a full tile pass from the
-    library's table counts, the one-term kernel from its streams."""
+    library's table counts, a resident pass from the rows and the tables,
+    the one-term kernel from its streams; psi0: the share of the launches
+    ending a step that read the initial states for a dot product."""
     full = None if sched is None else sched["pass_bytes"]
 
     def f(kind):
@@ -479,15 +483,17 @@ def pass_bytes_fn(sched, n, nnz, K, s, real):
         if kind.startswith("pass0x"):
             return full
         if kind.startswith("ring") and sched is not None:
-            # rows of v_{m-1} of the blocks and their rings, of v_{m-2} on the
-            # rows computed (not in a first pass), and of the owned rows:
-            # output read (not in a first pass) and written, psi0 (last), two
-            # terms written (not in a last)
+            # of every row: v_{m-1}, v_{m-2} and the output read (the first
+            # pass of a step only v_{m-1}), the output written, psi0 (last)
+            # or two terms written (not in a last); the tables once: L2 can
+            # serve the groups of states that share them, and the neighbours
+            # that read a block's rows as their halo
             first, last = int(kind[4]) % 2, int(kind[4]) // 2
-            own = (0 if first else 1) + 1 + (1 if last else 0) + (0 if last else 2)
-            return sched["tables"] + sched["row_bytes"] * (
-                sched["gathered_rows"] + (0 if first else sched["streamed_rows"]) +
-                own * sched["owned_rows"])
+            rows = (1 if first else 3) + 1 + (psi0 if last else 2)
+            slots = sched["row_bytes"] // s
+            groups = slots // 2 if s == 8 and slots % 2 == 0 else slots
+            return int(sched["tables"] // groups +
+                       rows * sched["row_bytes"] * sched["owned_rows"])
         return None
     return f
 
@@ -708,7 +714,7 @@ def ac_workload(args, exact=None):
             if kind == "ac_corr":
                 # cols, J_x, J_y values (complex), psi1x, psi1y gathered, psi2 own row
                 return nnz * (4 + 2 * sz) + 3 * per * n * sz
-            return pass_bytes_fn(sched, n, nnz, 3 * per, sz, real)(kind)
+            return pass_bytes_fn(sched, n, nnz, 3 * per, sz, real, psi0=0.0)(kind)
         label = (lambda k, prec=prec, real=real, threads=threads:
                  kernel_label(k, prec, 3 * per, real, threads))
         res[prec] = {"value": K * (T - 1) / t_prop, "ms_per_step": t_prop / (T - 1) * 1e3,
@@ -813,7 +819,7 @@ def dc_workload(args):
         if kind == "dc_dot":   # J_a psi(t) read, J_a QE read (FP64)
             steps = Tp / (1 + math.ceil((Tp - 1) / 16))
             return steps * 2 * per * n * 8 + 2 * ne * per * n * 16
-        return pass_bytes_fn(sched, n, nnz, 2 * per, 8, real)(kind)
+        return pass_bytes_fn(sched, n, nnz, 2 * per, 8, real, psi0=0.5)(kind)
     value = 2 * K * (2 * T - 1) / dt
     return {"metric": "DC correlation step·vectors/s (disordered field-threaded graphene)",
             "value": round(value, 2), "unit": "step·vectors/s", "higher_is_better": True,

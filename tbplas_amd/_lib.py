@@ -266,8 +266,10 @@ def dev(a, dtype=None, device=0):
 
 def host(t):
     """numpy copy of a device tensor.  NumPy advises huge pages for its large
-    arrays and torch does not: 64 MB arrive in 6.7 ms instead of 16 ms, most
-    of which were the page faults of the destination."""
+    arrays and torch does not, which matters where the host is slow to give
+    fresh pages: 64 MB arrived in 6.7 ms instead of 16 ms on one machine
+    (most of it the page faults of the destination), in the same time on
+    another."""
     torch = torch_cuda()
     out = torch.from_numpy(np.empty(t.shape, dtype=str(t.dtype)[6:]))
     return out.copy_(t).numpy()

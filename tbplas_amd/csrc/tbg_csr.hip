@@ -359,8 +359,8 @@ static bool same_indptr(tbg_handle* h, int64_t n, const int64_t* a, const int64_
 // indptr (n+1) from the emission stream (diag_mode 1: |orb_eng| >= cutoff,
 // 2: orb_eng != 0, 0: no diagonal); returns nnz.
 static int64_t place_count(tbg_handle* h, int64_t n, int64_t m, const double* orb_eng,
-                           int diag_mode, double cutoff, const int64_t* hop_i, const int64_t* hop_j, int64_t* indptr,
-                    Scratch& w) {
+                           int diag_mode, double cutoff, const int64_t* hop_i,
+                           const int64_t* hop_j, int64_t* indptr, Scratch& w) {
     check_hops(n, m);
     check_hop_indices(h, n, m, hop_i, hop_j, w);
     DevBuf cnt, tmp;
