@@ -301,6 +301,31 @@ def test_dc_more_energies_than_grid_rows(handle):
     H.close()
 
 
+def test_dc_sums_round_as_trees(handle):
+    """After one step the window is zero, QE is psi0 and the correlation is
+    |J psi0|^2 / |psi0|^2 of 24,000 positive terms.  Against 80-bit sums: a
+    chain of n equal terms leaves sqrt(n / 3) roundings of 2^-53 / sqrt(3),
+    0.64e-16 of the sum each.  The partial sums of 384 splits, by eights, and
+    of 94 chunks, by 32s, leave chains of 3 to 32: 2.1e-16 together, allowed
+    twice; one after the other they leave 7e-16 and 4e-16, and more where
+    terms of one size round alike."""
+    s, _ = _sample(100, 120, 20.0, 0.0, 0.0)
+    ip, ix, hop, dx, dy = oracle.build_ham_dxy_loop(s.orb_eng, s.hop_i, s.hop_j, s.hop_v, s.dr)
+    H = tbpm.Hamiltonian(s.num_orb, ip, ix, hop, dx, dy, cur_scale=9.0, precision="fp64",
+                         handle=handle)
+    bes = tbpm.bessel_series(tau_of(s), 1e-14)
+    err = []
+    for psi in _states(s.num_orb, 24):
+        c = tbpm.corr_dc(H, bes, psi[None], 1, 2 * math.pi / 18.0, np.array([0.1]), np.arange(1))[1]
+        z = psi.astype(np.clongdouble)
+        for a, d in enumerate((dx, dy)):
+            j = np.add.reduceat(hop.astype(np.clongdouble) * d * 9.0 * z[ix], ip[:-1])
+            want = np.sum(np.abs(j) ** 2) / np.sum(np.abs(z) ** 2)
+            err.append(float((np.clongdouble(c[0, a, 0, 0]) - want).real / want))
+    assert np.sqrt(np.mean(np.square(err))) < 4.2e-16
+    H.close()
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("resident", [True, False])
 @pytest.mark.parametrize("T", [7, 16, 37])
