@@ -60,10 +60,8 @@ struct Ring {
     // what one pass of depth terms must move: table bytes, rows loaded,
     // rows computed in the first term, rows owned
     int64_t sched[4] = {0, 0, 0, 0};
-    DevBuf meta, ends, rows, idx, vals;
-    size_t bytes() const {
-        return meta.bytes + ends.bytes + rows.bytes + idx.bytes + vals.bytes;
-    }
+    DevBuf all, meta, ends, rows, idx, vals;   // (the others are parts of all)
+    size_t bytes() const { return all.bytes; }
 };
 
 // Vectors per lane (states of one workgroup) for Kp slots: 16-byte units

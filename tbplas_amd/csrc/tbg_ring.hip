@@ -20,9 +20,11 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <functional>
 #include <mutex>
 #include <thread>
 
@@ -32,39 +34,96 @@ namespace tbg {
 
 namespace {
 
-// f(i, thread) for i < n on up to 16 host threads; the first exception is
-// rethrown here.
-template <typename F>
-void parallel_for(int64_t n, int64_t grain, F&& f) {
-    const int nt = (int)std::max<int64_t>(
-        1, std::min<int64_t>(std::min(16u, std::max(1u, std::thread::hardware_concurrency())),
-                             n / std::max<int64_t>(grain, 1)));
-    std::atomic<int64_t> next{0};
-    std::exception_ptr err;
-    std::mutex mu;
-    const int64_t step = std::max<int64_t>(1, std::min<int64_t>(grain, n / (4 * nt) + 1));
-    auto work = [&](int th) {
+// Up to 16 host threads for the whole of a build: started for each of its five
+// phases they took 0.2 to 0.7 of the 1.8 to 3.4 ms that the tables of 8,000 to
+// 33,000 rows took.  Between two phases they look for the next one for a
+// while, then sleep.
+class Team {
+public:
+    explicit Team(int want) {
         try {
-            for (;;) {
-                const int64_t a = next.fetch_add(step);
-                if (a >= n) break;
-                for (int64_t i = a; i < std::min(n, a + step); ++i) f(i, th);
+            for (int t = 1; t < want; ++t) {
+                threads_.emplace_back([this, t] { serve(t); });
+                ++size_;
             }
-        } catch (...) {
-            std::lock_guard<std::mutex> g(mu);
-            if (!err) err = std::current_exception();
-            next.store(n);
+        } catch (...) {   // no more threads: the ones that started do the work
         }
-    };
-    std::vector<std::thread> ts;
-    try {
-        for (int t = 1; t < nt; ++t) ts.emplace_back(work, t);
-    } catch (...) {   // no more threads: the ones that started do the work
     }
-    work(0);
-    for (auto& t : ts) t.join();
-    if (err) std::rethrow_exception(err);
-}
+    ~Team() {
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            stop_ = true;
+            phase_.fetch_add(1, std::memory_order_release);
+        }
+        cv_.notify_all();
+        for (auto& t : threads_) t.join();
+    }
+    Team(const Team&) = delete;
+    Team& operator=(const Team&) = delete;
+
+    // f(i, thread) for i < n, at least `grain` of them a thread; the first
+    // exception is rethrown here.
+    template <typename F>
+    void run(int64_t n, int64_t grain, F&& f) {
+        grain = std::max<int64_t>(grain, 1);
+        const int nt = (int)std::max<int64_t>(1, std::min<int64_t>(size_, n / grain));
+        const int64_t step = std::max<int64_t>(1, std::min<int64_t>(grain, n / (4 * nt) + 1));
+        std::atomic<int64_t> next{0};
+        std::exception_ptr err;
+        std::mutex err_mu;
+        const std::function<void(int)> work = [&](int th) {
+            if (th >= nt) return;
+            try {
+                for (;;) {
+                    const int64_t a = next.fetch_add(step);
+                    if (a >= n) break;
+                    for (int64_t i = a; i < std::min(n, a + step); ++i) f(i, th);
+                }
+            } catch (...) {
+                std::lock_guard<std::mutex> g(err_mu);
+                if (!err) err = std::current_exception();
+                next.store(n);
+            }
+        };
+        if (nt > 1) {
+            {
+                std::lock_guard<std::mutex> g(mu_);
+                work_ = &work;
+                busy_.store(size_ - 1, std::memory_order_relaxed);
+                phase_.fetch_add(1, std::memory_order_release);
+            }
+            cv_.notify_all();
+        }
+        work(0);
+        if (nt > 1)
+            while (busy_.load(std::memory_order_acquire) > 0) std::this_thread::yield();
+        if (err) std::rethrow_exception(err);
+    }
+
+private:
+    void serve(int th) {
+        for (unsigned seen = 0;;) {
+            for (int spin = 0; spin < 4000 && phase_.load(std::memory_order_acquire) == seen; ++spin)
+                std::this_thread::yield();
+            {
+                std::unique_lock<std::mutex> g(mu_);
+                cv_.wait(g, [&] { return phase_.load(std::memory_order_relaxed) != seen; });
+                seen = phase_.load(std::memory_order_relaxed);
+                if (stop_) return;
+            }
+            (*work_)(th);
+            busy_.fetch_sub(1, std::memory_order_release);
+        }
+    }
+    std::vector<std::thread> threads_;
+    int size_ = 1;
+    std::mutex mu_;
+    std::condition_variable cv_;
+    std::atomic<unsigned> phase_{0};
+    std::atomic<int> busy_{0};
+    const std::function<void(int)>* work_ = nullptr;
+    bool stop_ = false;
+};
 
 constexpr int kHostThreads = 16;
 
@@ -124,6 +183,39 @@ bool grow(const Csr& A, Marks& mk, std::vector<int>& rows, int depth, int64_t ca
     return true;
 }
 
+struct Block {
+    std::vector<int> rows, ends;
+    std::vector<uint16_t> pos;   // of each computed row's entries, in the block
+    int seg = 0, w = 0;
+};
+
+// The positions in block b (as grown, its rows marked) of the entries of the
+// rows that a pass computes: those of a row of ring q lie in the rings up to
+// q + 1, which the pass holds one term earlier (false: they do not).  W a row,
+// or b.w columns of them for wide rows; places beyond a row's entries hold
+// the row itself (with a value of zero).
+bool positions(const Csr& A, const Marks& mk, Block& b, int depth, int W) {
+    const int nC = b.ends[depth - 1];
+    const size_t ww = W ? W : b.w;
+    b.pos.resize(nC * ww);
+    int ring = 0;
+    for (int l = 0; l < nC; ++l) {
+        while (l >= b.ends[ring]) ++ring;
+        const int r = b.rows[l], w = A.width(r);
+        const int end = b.ends[ring + 1];
+        for (int j = 0; j < (int)ww; ++j) {
+            int pos = l;
+            if (j < w) {
+                const int c = A.cols[A.elem(r, j)];
+                pos = mk.loc[c];
+                if (mk.mark[c] != mk.stamp || pos >= end) return false;
+            }
+            b.pos[W ? l * ww + j : (size_t)j * nC + l] = (uint16_t)pos;
+        }
+    }
+    return true;
+}
+
 // A compact piece of a caller's tile, from which blocks are made.
 struct Atom {
     std::vector<int> rows;
@@ -172,11 +264,6 @@ void split_tile(const Csr& A, Marks& mk, int64_t r0, int64_t r1, int k, int seg,
     }
 }
 
-struct Block {
-    std::vector<int> rows, ends;
-    int seg = 0, w = 0;
-};
-
 }  // namespace
 
 std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
@@ -213,6 +300,8 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     const int nr = ring_rows(real_bytes, V, real_vals, W);
     const int nro = ring_owned(real_bytes, V, real_vals, W);
     std::vector<Marks> marks(kHostThreads);
+    const int64_t cores = std::max(1u, std::thread::hardware_concurrency());
+    Team team((int)std::min({(int64_t)kHostThreads, cores, covered / 256 + 1}));
 
     // growth of a block per ring, from a few tiles: side(k) = side(0) + k c
     // with side = sqrt(rows)
@@ -311,7 +400,7 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
             for (size_t i = 0; i + 1 < segs[sg].size(); ++i) tiles.emplace_back((int)sg, (int64_t)i);
         std::vector<std::vector<Atom>> cut(tiles.size());
         const double piece = std::max(24.0, target / 8.0);
-        parallel_for((int64_t)tiles.size(), 16, [&](int64_t i, int th) {
+        team.run((int64_t)tiles.size(), 16, [&](int64_t i, int th) {
             marks[th].need(n);
             const auto& t = segs[tiles[i].first];
             const int64_t a = t[tiles[i].second], b = t[tiles[i].second + 1];
@@ -323,11 +412,11 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     }
     const int na = (int)atoms.size();
     std::vector<int> atom_of((size_t)n, -1);
-    parallel_for(na, 64, [&](int64_t i, int) {
+    team.run(na, 64, [&](int64_t i, int) {
         for (int r : atoms[i].rows) atom_of[r] = (int)i;
     });
     std::vector<std::vector<std::pair<int, int>>> nbr((size_t)na);   // (atom, couplings)
-    parallel_for(na, 64, [&](int64_t i, int) {
+    team.run(na, 64, [&](int64_t i, int) {
         auto& v = nbr[i];
         for (int r : atoms[i].rows)
             for (int j = 0, w = A.width(r); j < w; ++j) {
@@ -441,8 +530,8 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
     // rings and tables, split where a block does not fit
     const int64_t ng = (int64_t)groups_of.size();
     std::vector<std::vector<Block>> made((size_t)ng);
-    std::atomic<bool> fits{true};
-    parallel_for(ng, 4, [&](int64_t i, int th) {
+    std::atomic<bool> fits{true}, sound{true};
+    team.run(ng, 4, [&](int64_t i, int th) {
         Marks& mk = marks[th];
         mk.need(n);
         std::vector<std::vector<int>> todo(1);
@@ -466,9 +555,14 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
                 continue;
             }
             for (int r : b.rows) b.w = std::max(b.w, A.width(r));
+            if (!positions(A, mk, b, depth, W)) {
+                sound = false;
+                return;
+            }
             made[i].push_back(std::move(b));
         }
     });
+    TBG_REQUIRE(sound, "internal: resident-pass table out of range");
     if (!fits) return nullptr;
     auto R = std::make_shared<Ring>();
     std::vector<Block*> blocks;
@@ -498,82 +592,66 @@ std::shared_ptr<Ring> build_ring(tbg_handle* h, const BlockSrc& src,
         R->owned_max = std::max(R->owned_max, k.ends[0]);
     }
     while (R->seg_block.size() < segs.size() + 1) R->seg_block.push_back(nb);
-    std::vector<int> rows((size_t)nrow);
-    std::vector<uint16_t> idx((size_t)(W ? ntab * 4 : nent));
-    std::vector<unsigned char> vals((size_t)(W ? ntab * W : nent) * vsz);
     const int shift = unit_bytes == 16 ? 4 : 3;
     TBG_REQUIRE(unit_bytes == 16 || unit_bytes == 8, "internal: unit of another size");
-    std::atomic<bool> sound{true};
-    parallel_for(nb, 4, [&](int64_t b, int th) {
+    // the tables one behind the other, copied at once (pages that the threads
+    // touch first, no zeros before)
+    struct Part {
+        size_t bytes, at;
+    } part[5] = {{meta.size() * sizeof(RingMeta), 0},
+                 {ends.size() * sizeof(int), 0},
+                 {(size_t)nrow * sizeof(int), 0},
+                 {(size_t)(W ? ntab * 4 : nent) * sizeof(uint16_t), 0},
+                 {(size_t)(W ? ntab * W : nent) * vsz, 0}};
+    size_t total = 0;
+    for (Part& p : part) {
+        p.at = total;
+        total += (p.bytes + 255) / 256 * 256;
+    }
+    const std::unique_ptr<unsigned char[]> buf(new unsigned char[total]);
+    std::memcpy(buf.get() + part[0].at, meta.data(), part[0].bytes);
+    std::memcpy(buf.get() + part[1].at, ends.data(), part[1].bytes);
+    int* const rows = reinterpret_cast<int*>(buf.get() + part[2].at);
+    unsigned char* const idx = buf.get() + part[3].at;
+    unsigned char* const vals = buf.get() + part[4].at;
+    team.run(nb, 4, [&](int64_t b, int) {
         const Block& k = *blocks[b];
         const RingMeta& m = meta[b];
-        Marks& mk = marks[th];
-        mk.need(n);
-        const int st = ++mk.stamp;
-        for (size_t q = 0; q < k.rows.size(); ++q) {
-            mk.mark[k.rows[q]] = st;
-            mk.loc[k.rows[q]] = (int)q;
-            rows[m.offR + q] = k.rows[q];
-        }
-        // every position a row of ring q reads lies in the rings up to q + 1,
-        // which the pass holds one term earlier
-        int ring = 0;
+        std::memcpy(rows + m.offR, k.rows.data(), k.rows.size() * sizeof(int));
+        if (!W) std::memcpy(idx + m.offE * 2, k.pos.data(), k.pos.size() * 2);
+        const int ww = W ? W : m.w;
         for (int l = 0; l < m.pad; ++l) {
-            while (l >= k.ends[ring]) ++ring;
             const int r = k.rows[l], w = A.width(r);
-            const int ww = W ? W : m.w;
             for (int j = 0; j < ww; ++j) {
-                const int64_t at = m.offE + (int64_t)j * m.pad + l;
-                const int64_t av = W ? (m.offT + l) * W + j : at;
-                int pos = l;                    // (zero value on the row itself)
-                if (j < w) {
-                    const int64_t e = A.elem(r, j);
-                    const int c = A.cols[e];
-                    if (mk.mark[c] != st || mk.loc[c] >= k.ends[ring + 1]) {
-                        sound = false;
-                        return;
-                    }
-                    pos = mk.loc[c];
-                    std::memcpy(vals.data() + av * vsz, A.vals.data() + e * vsz, vsz);
-                } else {
-                    std::memset(vals.data() + av * vsz, 0, vsz);
-                }
-                if (W) {
-                    uint32_t& word = reinterpret_cast<uint32_t*>(idx.data())[(m.offT + l) * 2 +
-                                                                              j % 2];
-                    word |= j < 2 ? (uint32_t)pos << shift : (uint32_t)pos << 18;
-                } else {
-                    idx[at] = (uint16_t)pos;
-                }
+                const int64_t av = W ? (m.offT + l) * W + j : m.offE + (int64_t)j * m.pad + l;
+                if (j < w) std::memcpy(vals + av * vsz, A.vals.data() + A.elem(r, j) * vsz, vsz);
+                else std::memset(vals + av * vsz, 0, vsz);
+            }
+            if (W) {
+                const uint16_t* p = k.pos.data() + (size_t)l * W;
+                const uint32_t word[2] = {(uint32_t)p[0] << shift | (uint32_t)p[2] << 18,
+                                          (uint32_t)p[1] << shift |
+                                              (W > 3 ? (uint32_t)p[3] << 18 : 0u)};
+                std::memcpy(idx + (m.offT + l) * 8, word, 8);
             }
         }
     });
-    TBG_REQUIRE(sound, "internal: resident-pass table out of range");
     R->depth = depth;
     R->width = W;
     R->nblocks = nb;
     R->rows_lane = nr;
     R->owned_lane = nro;
     R->halo = (double)computed / (double)covered;
-    R->sched[0] = (int64_t)(rows.size() * 4 + idx.size() * 2 + vals.size()) +
-                  (int64_t)nb * (int64_t)(sizeof(RingMeta) + 4 * (depth + 1));
+    R->sched[0] = 0;
+    for (const Part& p : part) R->sched[0] += (int64_t)p.bytes;
     R->sched[1] = nrow;
     R->sched[2] = computed;
     R->sched[3] = covered;
-    // (all the memory first: no copy is under way where there is none)
-    R->meta.alloc(meta.size() * sizeof(RingMeta));
-    R->ends.alloc(ends.size() * sizeof(int));
-    R->rows.alloc(rows.size() * sizeof(int));
-    R->idx.alloc(idx.size() * sizeof(uint16_t));
-    R->vals.alloc(vals.size());
-    auto up = [&](DevBuf& d, const void* p) {
-        TBG_HIP(hipMemcpyAsync(d.p, p, d.bytes, hipMemcpyHostToDevice, h->stream));
-    };
-    up(R->meta, meta.data());
-    up(R->ends, ends.data());
-    up(R->rows, rows.data());
-    up(R->idx, idx.data());
-    up(R->vals, vals.data());
+    R->all.alloc(total);
+    DevBuf* const to[5] = {&R->meta, &R->ends, &R->rows, &R->idx, &R->vals};
+    for (int i = 0; i < 5; ++i)
+        to[i]->borrow(R->all.as<unsigned char>() + part[i].at, part[i].bytes);
+    TBG_HIP(hipMemcpyAsync(R->all.p, buf.get(), total, hipMemcpyHostToDevice, h->stream));
     TBG_HIP(hipStreamSynchronize(h->stream));
     return R;
 }

@@ -144,13 +144,13 @@ def _few_steps(n, K, prec, steps):
     """Whether so few steps on a new Hamiltonian of n rows do not pay for the
     tables of resident passes.  Below some 70,000 rows these take longer to
     make than the tiles' (ms, one complex128 state: 0.8 / 0.3 at 2,100 rows,
-    1.7 / 0.5 at 8,300, 3.3 / 1.4 at 33,000; 5.5 / 5.4 at 131,600, and less
+    1.6 / 0.5 at 8,300, 2.7 / 1.5 at 33,000; 5.3 / 5.6 at 131,600, and less
     from there on), and a step gains 8 to 20 us.  Steps after which they are
-    even: 71, 116, 201 there, 60 to 245 for one complex64 state, 41 to 171
-    for four; 20 to 60 with more than 32 bytes a row (114 once), AC and DC
-    runs 10 to 90."""
+    even: 65, 107, 140 there, 54 to 162 for one complex64 state, 36 to 162
+    for four; 10 to 50 with more than 32 bytes a row (115 once), AC and DC
+    runs 10 to 70."""
     from .sample import _row_bytes
-    return n < 70_000 and steps < (150 if _row_bytes(K, prec) <= 32 else 50)
+    return n < 70_000 and steps < (100 if _row_bytes(K, prec) <= 32 else 40)
 
 
 def apply(H, K, bes, enabled=True, steps=None):

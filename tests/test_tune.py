@@ -51,8 +51,8 @@ def test_shapes(terms, state):
 
 
 @pytest.mark.parametrize("n,K,steps,resident", [
-    (8000, 1, 64, False), (8000, 1, 149, False), (8000, 1, 150, True), (8000, 2, 64, False),
-    (8000, 4, 64, True), (8000, 4, 49, False), (69999, 1, 1, False), (70000, 1, 1, True),
+    (8000, 1, 64, False), (8000, 1, 99, False), (8000, 1, 100, True), (8000, 2, 64, False),
+    (8000, 4, 40, True), (8000, 4, 39, False), (69999, 1, 1, False), (70000, 1, 1, True),
     (8000, 1, None, True), (2_000_000, 8, 1, True)])
 @pytest.mark.parametrize("tuned", [False, True])
 def test_few_steps_on_a_small_sample_take_tile_passes(n, K, steps, resident, tuned, monkeypatch):
